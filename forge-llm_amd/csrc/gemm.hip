@@ -1371,9 +1371,8 @@ __global__ void __launch_bounds__(256) tail_reduce_grouped(GTable t) {
 // The slab loads of four z at a time are issued together (the sum keeps the
 // z order); each slab is read once, so it is streamed (nontemporal).
 typedef float v4f __attribute__((ext_vector_type(4)));
-__global__ void __launch_bounds__(256) splitk_reduce_kernel(float* __restrict__ C, const float* __restrict__ partial,
-                                                            int64_t n, int splits, int beta,
-                                                            const float* __restrict__ resid) {
+__device__ __forceinline__ void splitk_sum(float* __restrict__ C, const float* __restrict__ partial, int64_t n,
+                                           int splits, int beta, const float* __restrict__ resid) {
   int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x * 4;
   // float4 path: C and resid 16-byte aligned, every partial slab too (pool-aligned base, n % 4 == 0)
@@ -1409,6 +1408,21 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(float* __restrict__ 
       }
     }
   }
+}
+
+__global__ void __launch_bounds__(256) splitk_reduce_kernel(float* __restrict__ C, const float* __restrict__ partial,
+                                                            int64_t n, int splits, int beta,
+                                                            const float* __restrict__ resid) {
+  splitk_sum(C, partial, n, splits, beta, resid);
+}
+
+#include "gemm_pieces.h"
+
+// The grouped launch's K pieces, summed per job in order z = 0 .. splits - 1
+// (onto C when the job accumulates).
+__global__ void __launch_bounds__(256) splitk_reduce_grouped(PTable t) {
+  const PJob& jb = t.job[blockIdx.y];
+  splitk_sum(jb.C, t.slab + jb.slab0, (int64_t)jb.M * jb.N, t.splits, jb.beta, nullptr);
 }
 
 // Tile shape and K split for one GEMM (rules from measurements of the three
@@ -1613,6 +1627,143 @@ TailPlan plan_tail(int64_t tiles, int K, int cus) {
   return t;
 }
 
+// ───────── when to split the operands ahead (gemm_pieces.h) ─────────
+// Times in us, fitted to sweeps of M, N = 768 .. 32000, K = 768 .. 28672:
+//   * a round of two workgroups per CU on 128 x 256 tiles or of one on 256 x
+//     256 takes 1.18 or 1.13 per chunk of 16 k and 8 or 14 for its prologue
+//     and epilogue; a round of one 128-row workgroup per CU 0.58 of that;
+//   * K pieces cost their partial sums' traffic at 5 TB/s and a launch;
+//   * the split 8 B per (padded) operand element at 5.2 TB/s and 10 for its
+//     launch and what the GEMM's own first tiles wait for it;
+//   * the kernels that split while staging 2 M N K at 360 TFLOP/s and 10.
+// E.g. 4096 x 28672 over K = 4096 (2560) goes to pieces at 2160 + 210, 2048 x
+// 4096 over K = 1024 (57) stays: its pieces would take 49 + 10.
+struct PiecePlan {
+  int wm = 0;  // tiles of 64 wm x 256; 0: not worth it
+  int splits = 1;
+  double us = 0.0;
+};
+inline double piece_waves_us(int64_t wgs, int nk, int wm, int cus) {
+  if (wm == 4) return (double)((wgs + cus - 1) / cus) * (1.13 * nk + 14.0) * 256.0 / cus;
+  const double t2 = (1.18 * nk + 8.0) * 256.0 / cus;
+  const int64_t full = wgs / (2 * cus), rem = wgs % (2 * cus);
+  return (double)full * t2 + (rem == 0 ? 0.0 : rem <= cus ? 0.58 * t2 : t2);
+}
+constexpr int64_t kPiecesMaxBytes = (int64_t)8 << 30;  // both operands' pieces of one GEMM
+
+// force_splits: 0 = free choice of the K split.  The same plan serves a GEMM
+// whose pieces' sums stay unreduced (parts_out), so that their sum is what the
+// reduced form stores.
+inline PiecePlan plan_pieces(int M, int N, int K, int cus, int force_splits) {
+  PiecePlan best;
+  if (K < 64 || (int64_t)M * N * K < ((int64_t)1 << 31)) return best;
+  const int nkc = (K + 15) / 16;
+  const double old_us = 2.0 * M * N * (double)K / 360e6 + 10.0;
+  best.us = old_us;
+  for (const int wm : {2, 4}) {
+    const int64_t tm = (M + 64 * wm - 1) / (64 * wm), tn = (N + 255) / 256;
+    const double pieces = 64.0 * ((double)nkc * 16) * ((double)tm * wm + (double)tn * 4);  // elements
+    if (4.0 * pieces > (double)kPiecesMaxBytes) continue;
+    for (int s = 1; s <= 8; ++s) {
+      if (force_splits && s != force_splits) continue;
+      if (s > 1 && nkc / s < 8) continue;
+      const int per = (nkc + s - 1) / s;
+      if ((nkc + per - 1) / per != s) continue;
+      double us = piece_waves_us(tm * tn * s, per, wm, cus) + pieces * 8.0 / 5.2e6 + 10.0;
+      if (s > 1) us += (double)(s + 1) * M * N * 4.0 / 5e6 + 3.0;
+      if (us < best.us) best = PiecePlan{wm, s, us};
+    }
+  }
+  return best;
+}
+
+// Queues the split of the table's operands (8 B per element written and read).
+inline int queue_split(SplitTable& t, bool scoped) {
+  double bytes = 0.0;
+  t.units = 0;
+  for (int i = 0; i < t.count; ++i) {
+    t.job[i].unit0 = t.units;
+    t.units += split_units(t.job[i]);
+    bytes += 8.0 * (double)t.job[i].rows * t.job[i].k;
+  }
+  fg::KProfScope prof(scoped ? "gemm_split" : nullptr, 0.0, bytes);
+  const int blocks = (t.units + 3) / 4;
+  FG_LAUNCH(split_pieces_kernel, dim3(blocks < 4096 ? blocks : 4096), dim3(256), 0, t);
+  return FG_OK;
+}
+inline int64_t piece_bytes(int rows, int K, int tile) {
+  return (int64_t)((rows + tile - 1) / tile) * tile * ((K + 15) / 16) * 64;
+}
+
+// The GEMM of launch_gemm on split operands; `got` is false when the pieces'
+// workspace cannot be had (the caller then takes the kernels that need none).
+struct SwigluOut {
+  float* O = nullptr;
+  int H = 0;
+};
+inline int launch_pieces(const PiecePlan& pl, bool ak, bool bk, float* C, const float* A, const float* B, int M, int N,
+                         int K, int lda, int ldb, int beta, const float* resid, float* parts_out, bool scoped,
+                         const XpArgs& xp, const SwigluOut& sw, bool& got) {
+  const int TM = 64 * pl.wm, TN = 256, nkc = (K + 15) / 16, per = (nkc + pl.splits - 1) / pl.splits;
+  const int64_t abytes = piece_bytes(M, K, TM), bbytes = piece_bytes(N, K, TN);
+  fg::Workspace wsp, wsx, wss;
+  got = wsp.get((size_t)(abytes + bbytes)) == FG_OK;
+  float* partial = parts_out;
+  if (got && pl.splits > 1 && !partial) {
+    got = wss.get(sizeof(float) * (size_t)pl.splits * M * N) == FG_OK;
+    partial = (float*)wss.ptr;
+  }
+  if (!got) return FG_OK;
+  char* pa = (char*)wsp.ptr;
+  char* pb = pa + abytes;
+  const float *xpa, *xpb;
+  int rc = resolve_xp(xp, xp_job(A, ak, M, K, lda, nullptr), xp_job(B, bk, N, K, ldb, nullptr), wsx, scoped, xpa, xpb);
+  if (rc) return rc;
+  SplitTable st;
+  st.count = 2;
+  st.job[0] = SplitJob{A, pa, xpa, M, K, lda, nkc, (M + TM - 1) / TM * 2 * pl.wm, ak ? 1 : 0, 0, 0};
+  st.job[1] = SplitJob{B, pb, xpb, N, K, ldb, nkc, (N + TN - 1) / TN * 8, bk ? 1 : 0, sw.O ? sw.H : 0, 0};
+  rc = queue_split(st, scoped);
+  if (rc) return rc;
+  {
+    fg::KProfScope prof(!scoped ? nullptr : ak ? (bk ? "gemm_nt" : "gemm_nn") : "gemm_tn", 2.0 * M * N * (double)K,
+                        4.0 * ((double)M * K + (double)N * K +
+                               (1.0 + (beta ? 1.0 : 0.0) + (resid ? 1.0 : 0.0) + (sw.O ? 0.5 : 0.0)) * M * N));
+    const dim3 grid((unsigned)(((M + TM - 1) / TM) * ((N + TN - 1) / TN)), (unsigned)pl.splits), block(128 * pl.wm);
+    if (sw.O) {
+      if (pl.wm == 4)
+        FG_LAUNCH((gemm_pieces_swiglu_kernel<4, 4>), grid, block, 0, sw.O, C, pa, pb, M, sw.H, nkc, xpa, xpb);
+      else
+        FG_LAUNCH((gemm_pieces_swiglu_kernel<2, 3>), grid, block, 0, sw.O, C, pa, pb, M, sw.H, nkc, xpa, xpb);
+    } else {
+      const bool full = M % TM == 0 && N % TN == 0;
+#define FG_PIECES(WM, NB, S)                                                                                      \
+  if (full)                                                                                                       \
+    FG_LAUNCH((gemm_pieces_kernel<WM, NB, S, false>), grid, block, 0, C, pa, pb, M, N, nkc, per, beta, partial, resid, \
+              xpa, xpb);                                                                                          \
+  else                                                                                                            \
+    FG_LAUNCH((gemm_pieces_kernel<WM, NB, S, true>), grid, block, 0, C, pa, pb, M, N, nkc, per, beta, partial, resid,  \
+              xpa, xpb);
+      if (pl.wm == 4) {
+        FG_PIECES(4, 4, 4)
+      } else {
+        FG_PIECES(2, 4, 3)
+      }
+#undef FG_PIECES
+    }
+  }
+  if (pl.splits > 1 && !parts_out) {
+    fg::KProfScope prof2(scoped ? "gemm_splitk_reduce" : nullptr, 0.0,
+                         4.0 * (double)M * N * (pl.splits + 1 + (beta ? 1 : 0) + (resid ? 1 : 0)));
+    const int64_t n = (int64_t)M * N;
+    const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
+    int64_t blocks = (n / 4 + 255) / 256 + 1;
+    if (blocks > 8LL * cus) blocks = 8LL * cus;
+    FG_LAUNCH(splitk_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, C, partial, n, pl.splits, beta, resid);
+  }
+  return FG_OK;
+}
+
 // Queues C (+)= A·B on fg::stream(); split-K partials live in `ws`, which
 // the caller keeps until the kernels are ordered before any later reuse.
 // parts_out: the plan must split K in two; the two pieces' M x N partial sums
@@ -1636,6 +1787,13 @@ int launch_gemm(const char* name, fg::Workspace& ws, float* C, const float* A, c
   const GemmPlan pl = plan_gemm(AK, BKc, M, N, K, cus);
   FG_ARG_CHECK(!parts_out || (pl.splits == 2 && !beta && !resid),
                "%s: the plan for M=%d N=%d K=%d takes %d K pieces, not two", name, M, N, K, pl.splits);
+  // input gradients keep the number of K pieces fg_matmulT_bwd_x_pieces names
+  const PiecePlan pp = plan_pieces(M, N, K, cus, AK && !BKc ? pl.splits : 0);
+  if (pp.wm) {
+    bool got = false;
+    int rc = launch_pieces(pp, AK, BKc, C, A, B, M, N, K, lda, ldb, beta, resid, parts_out, scoped, xp, SwigluOut(), got);
+    if (rc || got) return rc;
+  }
   const int tiles = ((M + pl.tm - 1) / pl.tm) * ((N + pl.tn - 1) / pl.tn);
   // Fast path: every tile full and every vector access aligned.
   const bool even = (M % pl.tm == 0) && (N % pl.tn == 0) && (K % BK == 0) && (lda % 4 == 0) && (ldb % 4 == 0) &&
@@ -1809,8 +1967,17 @@ extern "C" int fg_matmulT_fwd_swiglu_p(float* O, float* GU, const float* X, cons
   FG_ARG_CHECK(M > 0 && K > 0 && H > 0, "fg_matmulT_fwd_swiglu: bad shape M=%d K=%d H=%d", M, K, H);
   FG_ARG_CHECK(O && GU && X && Wgu, "fg_matmulT_fwd_swiglu: null pointer");
   const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
+  // on pieces, where plan_pieces' choice for the plain forward is one that
+  // the epilogue fits (the same products in the same order as that forward)
+  const PiecePlan pp = plan_pieces(M, 2 * H, K, cus, 0);
+  if (pp.wm && pp.splits == 1 && M % (64 * pp.wm) == 0 && H % 128 == 0) {
+    bool got = false;
+    int rc = launch_pieces(pp, true, true, GU, X, Wgu, M, 2 * H, K, K, K, 0, nullptr, nullptr, true,
+                           XpArgs{xp_x, xp_w, have}, SwigluOut{O, H}, got);
+    if (rc || got) return rc;
+  }
   const GemmPlan pl = plan_gemm(true, true, M, 2 * H, K, cus);
-  const bool fused = pl.w && pl.tn == 256 && pl.splits == 1 && M % 256 == 0 && H % 128 == 0 && K % BK == 0 &&
+  const bool fused = !pp.wm && pl.w && pl.tn == 256 && pl.splits == 1 && M % 256 == 0 && H % 128 == 0 && K % BK == 0 &&
                      (int64_t)(M / 256) * (2 * H / 256) % cus == 0 && (uintptr_t)X % 16 == 0 &&
                      (uintptr_t)Wgu % 16 == 0 && (uintptr_t)GU % 16 == 0;
   if (!fused) {  // the GEMM, then the SwiGLU pass
@@ -1877,12 +2044,166 @@ extern "C" int fg_matmulT_bwd_w(float* gW, const float* gY, const float* X, int 
   return fg_matmulT_bwd_w_p(gW, gY, X, M, K, N, beta, nullptr, nullptr, 0);
 }
 
+namespace {
+// The grouped weight gradients on split operands, where the whole list gains
+// by it (the same times as plan_pieces, tiles and operands summed over the
+// jobs); `done` false: the caller takes the kernels that split while staging.
+// The list is cut into launches of at most kPieceJobs jobs, kGroupedBytes of
+// pieces and distinct outputs.
+constexpr int64_t kGroupedBytes = (int64_t)4 << 30;
+int grouped_pieces(const fg_wgrad_job* jobs, int count, int cus, bool& done) {
+  done = false;
+  double flop = 0.0;
+  for (int i = 0; i < count; ++i) {
+    const fg_wgrad_job& jb = jobs[i];
+    if (!(jb.gW && jb.gY && jb.X && jb.M > 0 && jb.K > 0 && jb.N > 0)) return FG_OK;  // reported by the caller
+    if (4 * (piece_bytes(jb.N, jb.M, 256) + piece_bytes(jb.K, jb.M, 256)) > 2 * kPiecesMaxBytes) return FG_OK;
+    flop += 2.0 * jb.M * jb.K * (double)jb.N;
+  }
+  if (flop < 8e9) return FG_OK;
+  int b = 0;
+  while (b < count) {
+    // the next launch: jobs [b, e)
+    int e = b;
+    int64_t bytes = 0;
+    for (; e < count && e - b < kPieceJobs; ++e) {
+      const int64_t add = piece_bytes(jobs[e].N, jobs[e].M, 256) + piece_bytes(jobs[e].K, jobs[e].M, 256);
+      bool again = false;
+      for (int j = b; j < e; ++j) again |= jobs[j].gW == jobs[e].gW;
+      if (again || (e > b && bytes + add > kGroupedBytes)) break;
+      bytes += add;
+    }
+    int wm = 0, splits = 1;
+    double best = 0.0, old_us = 10.0;
+    for (int j = b; j < e; ++j) old_us += 2.0 * jobs[j].M * jobs[j].K * (double)jobs[j].N / 360e6;
+    best = old_us;
+    for (const int cwm : {2, 4}) {
+      double tiles = 0.0, chunks = 0.0, pieces = 0.0, outs = 0.0;
+      int kmin = INT32_MAX;
+      for (int j = b; j < e; ++j) {
+        const double t = (double)((jobs[j].N + 64 * cwm - 1) / (64 * cwm)) * ((jobs[j].K + 255) / 256);
+        const int nkc = (jobs[j].M + 15) / 16;
+        tiles += t;
+        chunks += t * nkc;
+        kmin = min(kmin, nkc);
+        pieces += (double)(piece_bytes(jobs[j].N, jobs[j].M, 64 * cwm) + piece_bytes(jobs[j].K, jobs[j].M, 256)) / 4.0;
+        outs += (double)jobs[j].N * jobs[j].K;
+      }
+      for (int s = 1; s <= 8; ++s) {
+        if (s > 1 && kmin / s < 8) break;
+        double us = piece_waves_us((int64_t)tiles * s, (int)(chunks / tiles / s + 1.0), cwm, cus) +
+                    pieces * 8.0 / 5.2e6 + 10.0;
+        if (s > 1) us += (s + 1) * outs * 4.0 / 5e6 + 3.0;
+        if (us < best) {
+          best = us;
+          wm = cwm;
+          splits = s;
+        }
+      }
+    }
+    if (!wm && b == 0) return FG_OK;
+    if (!wm) wm = 2;  // a remainder of a list that started on pieces
+    const int TM = 64 * wm, TN = 256;
+    PTable t;
+    t.count = e - b;
+    t.tiles = 0;
+    t.splits = splits;
+    t.slab = nullptr;
+    bytes = 0;
+    int64_t slab = 0;
+    int missing = 0;
+    double lflop = 0.0, lbytes = 0.0;
+    for (int j = b; j < e; ++j) {
+      bytes += piece_bytes(jobs[j].N, jobs[j].M, TM) + piece_bytes(jobs[j].K, jobs[j].M, TN);
+      slab += (int64_t)splits * jobs[j].N * jobs[j].K;
+      missing += !jobs[j].xp_gy + !jobs[j].xp_x;
+    }
+    fg::Workspace wsp, wss, wsx;
+    if (wsp.get((size_t)bytes) != FG_OK || (splits > 1 && wss.get(sizeof(float) * (size_t)slab) != FG_OK)) {
+      if (b == 0) return FG_OK;
+      return FG_ERR_OOM;
+    }
+    if (missing) {
+      int rc = wsx.get((size_t)missing * kXpParts * sizeof(float));
+      if (rc) return rc;
+    }
+    float* next = static_cast<float*>(wsx.ptr);
+    XpTable xt;
+    xt.count = 0;
+    char* pieces = (char*)wsp.ptr;
+    t.slab = (float*)wss.ptr;
+    slab = 0;
+    for (int j = b; j < e; ++j) {
+      const fg_wgrad_job& jb = jobs[j];
+      PJob& q = t.job[j - b];
+      q.C = jb.gW;
+      q.M = jb.N;  // gW[N,K] (+)= gY^T · X: M_gemm = N, N_gemm = K, K_gemm = M
+      q.N = jb.K;
+      q.nkc = (jb.M + 15) / 16;
+      q.beta = jb.beta ? 1 : 0;
+      q.tile0 = t.tiles;
+      q.slab0 = slab;
+      q.A = pieces;
+      pieces += piece_bytes(jb.N, jb.M, TM);
+      q.B = pieces;
+      pieces += piece_bytes(jb.K, jb.M, TN);
+      q.xpa = jb.xp_gy;
+      q.xpb = jb.xp_x;
+      if (!q.xpa) {
+        xt.job[xt.count++] = xp_job(jb.gY, false, jb.N, jb.M, jb.N, next);
+        q.xpa = next;
+        next += kXpParts;
+      }
+      if (!q.xpb) {
+        xt.job[xt.count++] = xp_job(jb.X, false, jb.K, jb.M, jb.K, next);
+        q.xpb = next;
+        next += kXpParts;
+      }
+      t.tiles += ((q.M + TM - 1) / TM) * ((q.N + TN - 1) / TN);
+      slab += (int64_t)splits * q.M * q.N;
+      lflop += 2.0 * jb.M * jb.K * (double)jb.N;
+      lbytes += 4.0 * ((double)q.M * jb.M + (double)q.N * jb.M + (1.0 + q.beta) * q.M * q.N);
+    }
+    int rc = queue_absmax(xt, true);
+    if (rc) return rc;
+    SplitTable st;
+    st.count = 0;
+    for (int j = b; j < e; ++j) {
+      const fg_wgrad_job& jb = jobs[j];
+      const PJob& q = t.job[j - b];
+      st.job[st.count++] = SplitJob{jb.gY, (char*)q.A, q.xpa, q.M, jb.M, jb.N, q.nkc, (q.M + TM - 1) / TM * 2 * wm, 0, 0, 0};
+      st.job[st.count++] = SplitJob{jb.X, (char*)q.B, q.xpb, q.N, jb.M, jb.K, q.nkc, (q.N + TN - 1) / TN * 8, 0, 0, 0};
+      if (st.count == kSplitJobs || j + 1 == e) {
+        rc = queue_split(st, true);
+        if (rc) return rc;
+        st.count = 0;
+      }
+    }
+    fg::KProfScope prof("gemm_tn", lflop, lbytes);
+    const dim3 grid(t.tiles, splits), block(128 * wm);
+    if (wm == 4)
+      FG_LAUNCH((gemm_pieces_grouped<4, 4, 4>), grid, block, 0, t);
+    else
+      FG_LAUNCH((gemm_pieces_grouped<2, 4, 3>), grid, block, 0, t);
+    if (splits > 1) FG_LAUNCH(splitk_reduce_grouped, dim3(4 * cus, t.count), dim3(256), 0, t);
+    done = true;
+    b = e;
+  }
+  return FG_OK;
+}
+}  // namespace
+
 extern "C" int fg_matmulT_bwd_w_grouped(const fg_wgrad_job* jobs, int count) {
   FG_REQUIRE_INIT();
   FG_ARG_CHECK(count >= 0 && (count == 0 || jobs), "fg_matmulT_bwd_w_grouped: bad job list");
+  const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
+  {
+    bool done = false;
+    int rc = grouped_pieces(jobs, count, cus, done);
+    if (rc || done) return rc;
+  }
   // 256x256 tiles (gemm_w_grouped) when they make at least two rounds of
   // CUs, else 128x256 ping-pong tiles (twice as many to spread)
-  const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
   int64_t w_tiles = 0;
   for (int i = 0; i < count; ++i)
     w_tiles += (int64_t)((jobs[i].N + 255) / 256) * ((jobs[i].K + 255) / 256);

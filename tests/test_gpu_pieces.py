@@ -1,0 +1,93 @@
+"""The GEMMs on operands split ahead of time (csrc/gemm_pieces.h), which large
+shapes take: ragged rows, columns and k against fp64 on sampled rows and
+columns, in the three layouts, with the residual and accumulating; the K
+split; the grouped weight gradients over jobs of different lengths; and the
+fused SwiGLU epilogue bit for bit against the separate pass.
+
+Bound: the two-piece split leaves 3 * 2^-22 (7e-7) of a product and the fp32
+sums of random-sign terms about 2^-24 sqrt(K / 2) <= 5e-6 of the result's norm
+only at K ~ 10^4, less for the chunked order: 2e-6 up to K = 8000, 4e-6 above.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from util import rel_l2
+
+
+def up(fh, a):
+    return fh.DeviceArray.from_numpy(np.ascontiguousarray(a, np.float32))
+
+
+def _sample(rs, n, k=48):
+    """k indexes of [0, n), the edges among them."""
+    return np.unique(np.concatenate([[0, 1, n - 2, n - 1], rs.integers(0, n, k)]))
+
+
+def _check(got, ref, K):
+    assert rel_l2(got, ref) < (2e-6 if K <= 8000 else 4e-6)
+
+
+# forward tiles of 256 rows ragged in M, N and K; of 128 rows; split over K
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(8187, 2003, 4090), (4045, 1228, 8091), (3031, 11946, 7906)])
+def test_matmulT_on_pieces_vs_fp64(fh, M, K, N):
+    rs = np.random.default_rng(M)
+    X = rs.standard_normal((M, K), dtype=np.float32)
+    W = rs.standard_normal((N, K), dtype=np.float32) * np.float32(0.05)
+    R = rs.standard_normal((M, N), dtype=np.float32)
+    dX, dW, dR, dY = up(fh, X), up(fh, W), up(fh, R), fh.DeviceArray((M, N))
+    i, j = _sample(rs, M), _sample(rs, N)
+    fh.call("matmulT_fwd", dY, dX, dW, M, K, N)
+    Y = dY.numpy()
+    Xd, Wd = X.astype(np.float64), W.astype(np.float64)
+    _check(Y[i], Xd[i] @ Wd.T, K)
+    _check(Y[:, j], Xd @ Wd[j].T, K)
+    fh.call("matmulT_fwd_resid", dY, dR, dX, dW, M, K, N)
+    np.testing.assert_array_equal(dY.numpy(), R + Y)
+    # gradients, written and accumulated (R is the incoming gradient)
+    gX, gW = fh.DeviceArray((M, K)), fh.DeviceArray((N, K))
+    fh.call("matmulT_bwd", gX, 0, gW, 0, dR, dX, dW, M, K, N)
+    x0, w0 = gX.numpy(), gW.numpy()
+    Rd = R.astype(np.float64)
+    _check(x0[i], Rd[i] @ Wd, N)
+    _check(w0[j], Rd[:, j].T @ Xd, M)
+    fh.call("matmulT_bwd", gX, 1, gW, 1, dR, dX, dW, M, K, N)
+    _check(gX.numpy()[i], 2 * x0[i].astype(np.float64), 1)
+    _check(gW.numpy()[j], 2 * w0[j].astype(np.float64), 1)
+
+
+@pytest.mark.gpu
+def test_grouped_weight_gradients_on_pieces(fh):
+    """Jobs of different token counts (one shorter than a K piece of the
+    others) and ragged outputs in one launch, fresh and accumulating."""
+    rs = np.random.default_rng(5)
+    shapes = [(8190, 4093, 4100), (8190, 1021, 4100), (70, 300, 500), (4096, 4096, 4096)]  # M (tokens), K, N
+    host, rows = [], []
+    for M, K, N in shapes:
+        g, x = rs.standard_normal((M, N), dtype=np.float32), rs.standard_normal((M, K), dtype=np.float32)
+        w0 = rs.standard_normal((N, K), dtype=np.float32)
+        host.append((g, x, w0, up(fh, g), up(fh, x), up(fh, w0)))
+    for beta in (1, 0):
+        jobs = (fh.WgradJob * len(shapes))(*[
+            fh.WgradJob(h[5].ptr, h[3].ptr, h[4].ptr, M, K, N, beta, None, None)
+            for h, (M, K, N) in zip(host, shapes)])
+        fh.check(fh.lib.fg_matmulT_bwd_w_grouped(ctypes.cast(jobs, ctypes.c_void_p), len(shapes)), "grouped")
+        for (g, x, w0, _, _, dw), (M, K, N) in zip(host, shapes):
+            j = _sample(rs, N)
+            ref = g[:, j].astype(np.float64).T @ x.astype(np.float64) + beta * w0[j].astype(np.float64)
+            _check(dw.numpy()[j], ref, M)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,H", [(4096, 2048, 4096), (8064, 1030, 4096)])
+def test_swiglu_epilogue_on_pieces_is_the_separate_pass(fh, M, K, H):
+    rs = np.random.default_rng(H)
+    dX, dW = up(fh, rs.standard_normal((M, K))), up(fh, rs.standard_normal((2 * H, K)) * 0.02)
+    gu, o, gu2, o2 = (fh.DeviceArray(s) for s in ((M, 2 * H), (M, H), (M, 2 * H), (M, H)))
+    fh.call("matmulT_fwd_swiglu", o, gu, dX, dW, M, K, H)
+    fh.call("matmulT_fwd", gu2, dX, dW, M, K, 2 * H)
+    fh.call("swiglu_gu_fwd", o2, gu2, M, H)
+    np.testing.assert_array_equal(gu.numpy(), gu2.numpy())
+    np.testing.assert_array_equal(o.numpy(), o2.numpy())
