@@ -1,8 +1,9 @@
 // Token-side kernels of the device-resident training loop (train.js:246-276):
 //  - batch_gather: the B windows of seqLen+1 ids of one step, cut from a token
 //    buffer resident in device memory at host-drawn starts (train.js:255-260);
-//  - sort_*: a bitonic sort of 64-bit keys (id << 32 | position), which orders
-//    the positions of equal ids by increasing position;
+//  - sort_*: a sort of 64-bit keys (id << 32 | position), which orders the
+//    positions of equal ids by increasing position: by counting up to
+//    kRankMax keys, a bitonic network above;
 //  - embed_bwd_sorted: the embedding backward (tensor.js:92-98) over the
 //    sorted keys, each id's row summed in increasing position onto the
 //    existing gradient row — the reference's sequence of fp32 +=, with no
@@ -118,59 +119,107 @@ __global__ void __launch_bounds__(kThreads) embed_bwd_sorted_kernel(float* __res
 }
 
 // The same sums for D % 4 == 0 and 16-byte aligned rows: one wave per sorted
-// position, lane l holding float4 columns l, l+64, ... of the gradient row
-// (every element still takes row + g[t1] + g[t2] + ... in increasing t, one
-// fp32 add at a time, as above).  J float4 per lane per pass (J·64 >= the row
-// width up to 1024 float4, so a row takes one pass): the row's loads and those
-// of its first gradient row are issued together.  beta 0 starts each sum
-// from +0 instead of reading the row (the same bits as reading a zero row).
-template <int J>
+// position and run of 64 float4 columns, one float4 per lane (every element
+// still takes row + g[t1] + g[t2] + ... in increasing t, one fp32 add at a
+// time, as above).  A run's keys are read 64 at a time, one per lane, and its
+// gradient rows kRunLoads at a time before the first is added: text repeats
+// its commonest id hundreds of times in a step, and that run, walked one
+// dependent load after another by a wave that held the whole row, was the
+// launch's length (ids of frequency 1/rank, 8192 x 768: 323 us with one row
+// in flight, 50 us with 32).  beta 0 starts
+// each sum from +0 instead of reading the row (the same bits as reading a
+// zero row).
+constexpr int kRunLoads = 32;
 __global__ void __launch_bounds__(kThreads) embed_bwd_sorted4_kernel(float* __restrict__ gW,
                                                                      const float* __restrict__ g,
                                                                      const uint64_t* __restrict__ keys, int T,
                                                                      int V, int D4, int beta) {
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6));
-  const int nw = gridDim.x * (kThreads / 64);
+  const int segs = (D4 + 63) / 64;
+  const int64_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6));
+  const int64_t nw = (int64_t)gridDim.x * (kThreads / 64);
   const float4* g4 = reinterpret_cast<const float4*>(g);
-  for (int s = wave; s < T; s += nw) {
+  for (int64_t w = wave; w < (int64_t)T * segs; w += nw) {
+    const int s = (int)(w / segs), seg = (int)(w - (int64_t)s * segs);
     const uint64_t key = keys[s];
     const uint64_t prev = s > 0 ? keys[s - 1] : kNoKey;
     if (key == kNoKey) break;
     const uint32_t id = (uint32_t)(key >> 32);
     if (id >= (uint32_t)V) break;
     if (s > 0 && (uint32_t)(prev >> 32) == id) continue;
+    const int col = seg * 64 + lane;
+    const bool in = col < D4;
+    const int c = in ? col : D4 - 1;  // a valid column (not stored past D4)
     float4* row = reinterpret_cast<float4*>(gW) + (int64_t)id * D4;
-    const float4* g0 = g4 + (int64_t)(uint32_t)key * D4;
-    for (int c0 = lane; c0 < D4; c0 += 64 * J) {
-      float4 acc[J], v[J];
+    float4 acc = beta ? row[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+    int k = s;
+    for (bool more = true; more;) {
+      // the next keys of the run: lane l holds position k + l
+      const uint64_t kk = k + lane < T ? keys[k + lane] : kNoKey;
+      const uint64_t same = __ballot((uint32_t)(kk >> 32) == id);  // kNoKey's id field is never a valid id
+      const int n = ~same ? __builtin_ctzll(~same) : 64;
+      more = n == 64;
+      k += 64;
+      const int t = (int)(uint32_t)kk;
+      for (int i = 0; i < n; i += kRunLoads) {
+        float4 v[kRunLoads];
 #pragma unroll
-      for (int j = 0; j < J; ++j) {
-        const int c = c0 + 64 * j < D4 ? c0 + 64 * j : c0;  // a valid column (unused past D4)
-        acc[j] = beta ? row[c] : make_float4(0.f, 0.f, 0.f, 0.f);
-        v[j] = g0[c];
-      }
+        for (int q = 0; q < kRunLoads; ++q)
+          if (i + q < n) v[q] = g4[(int64_t)__builtin_amdgcn_readlane(t, i + q) * D4 + c];
 #pragma unroll
-      for (int j = 0; j < J; ++j) {
-        acc[j].x += v[j].x; acc[j].y += v[j].y; acc[j].z += v[j].z; acc[j].w += v[j].w;
-      }
-      for (int k = s + 1; k < T; ++k) {
-        const uint64_t kk = keys[k];
-        if ((uint32_t)(kk >> 32) != id) break;  // kNoKey's id field is never a valid id
-        const float4* gr = g4 + (int64_t)(uint32_t)kk * D4;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-          const int c = c0 + 64 * j < D4 ? c0 + 64 * j : c0;
-          const float4 u = gr[c];
-          acc[j].x += u.x; acc[j].y += u.y; acc[j].z += u.z; acc[j].w += u.w;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < J; ++j) {
-        const int c = c0 + 64 * j;
-        if (c < D4) row[c] = acc[j];
+        for (int q = 0; q < kRunLoads; ++q)
+          if (i + q < n) {
+            acc.x += v[q].x; acc.y += v[q].y; acc.z += v[q].z; acc.w += v[q].w;
+          }
       }
     }
+    if (in) row[col] = acc;
+  }
+}
+
+// Sorts up to kRankMax keys by counting: the position of a key is the number
+// of keys below it.  One workgroup per 64 positions (lane = position), its
+// waves share the ids to compare with; ids are wave-uniform (scalar loads),
+// one compare and one add per pair.  With less to do per pair than the
+// bitonic network has stages, and 128 workgroups at work instead of one per
+// 8192 keys: 8192 ids 75 -> 17 us.  Quadratic, so longer lists keep the
+// network.
+constexpr int kRankMax = 16384;
+constexpr int kRankThreads = 1024;
+__global__ void __launch_bounds__(kRankThreads) sort_rank_kernel(uint64_t* __restrict__ keys,
+                                                                 const int32_t* __restrict__ ids, int T, int V,
+                                                                 int P) {
+  constexpr int kWaves = kRankThreads / 64;
+  __shared__ int part[kWaves][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t0 = blockIdx.x * 64, t = t0 + lane;
+  if (t0 >= T) {  // positions past the ids
+    if (wave == 0 && t < P) keys[t] = kNoKey;
+    return;
+  }
+  const uint32_t id = t < T ? (uint32_t)ids[t] : ~0u;
+  const bool valid = id < (uint32_t)V;
+  // an earlier position counts when its id is <= le, a later one when < lt:
+  // ids outside [0, V) (as unsigned, at or above V) sort after every valid
+  // one, in order of position
+  const uint32_t le = valid ? id : ~0u, lt = valid ? id : (uint32_t)V;
+  const int per = (T + kWaves - 1) / kWaves, lo = wave * per, hi = min(T, lo + per);
+  const uint32_t* u = reinterpret_cast<const uint32_t*>(ids);
+  int count = 0;
+  const int e0 = min(hi, t0), m1 = min(hi, t0 + 64);
+#pragma unroll 16
+  for (int i = lo; i < e0; ++i) count += u[i] <= le;
+  for (int i = max(lo, t0); i < m1; ++i) count += i < t ? u[i] <= le : u[i] < lt;
+#pragma unroll 16
+  for (int i = max(lo, t0 + 64); i < hi; ++i) count += u[i] < lt;
+  part[wave][lane] = count;
+  __syncthreads();
+  if (wave == 0 && t < P) {
+    int r = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) r += part[w][lane];
+    if (t >= T) r = t;
+    keys[r] = valid ? ((uint64_t)id << 32) | (uint64_t)(uint32_t)t : kNoKey;
   }
 }
 
@@ -206,6 +255,11 @@ extern "C" int fg_embed_sort_keys(uint64_t* keys, int64_t len, const int32_t* id
   const int64_t P = keys_len(T);
   FG_ARG_CHECK(len >= P, "fg_embed_sort_keys: %lld keys given, %lld needed for T=%d", (long long)len,
                (long long)P, T);
+  if (P <= kRankMax) {
+    fg::KProfScope prof("embed_sort", 0.0, 16.0 * (double)P);
+    FG_LAUNCH(sort_rank_kernel, dim3((unsigned)((P + 63) / 64)), dim3(kRankThreads), 0, keys, ids, T, V, (int)P);
+    return FG_OK;
+  }
   const int C = (int)(P < kSortChunk ? P : kSortChunk);
   const unsigned chunks = (unsigned)(P / C);
   fg::KProfScope prof("embed_sort", 0.0, 16.0 * (double)P);
@@ -227,12 +281,10 @@ extern "C" int fg_embed_bwd_sorted(float* gW, const float* g, const uint64_t* ke
   fg::KProfScope prof("embed_bwd", 0.0, (beta ? 12.0 : 8.0) * (double)T * D);
   if (D % 4 == 0 && (uintptr_t)gW % 16 == 0 && (uintptr_t)g % 16 == 0) {
     const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
-    const int blocks = max(1, min((T + 3) / 4, 32 * cus));  // one wave per sorted position
     const int D4 = D / 4;
-    if (D4 <= 64) FG_LAUNCH((embed_bwd_sorted4_kernel<1>), dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D4, beta);
-    else if (D4 <= 256) FG_LAUNCH((embed_bwd_sorted4_kernel<4>), dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D4, beta);
-    else if (D4 <= 512) FG_LAUNCH((embed_bwd_sorted4_kernel<8>), dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D4, beta);
-    else FG_LAUNCH((embed_bwd_sorted4_kernel<16>), dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D4, beta);
+    const int64_t waves = (int64_t)T * ((D4 + 63) / 64);
+    const int blocks = (int)max((int64_t)1, min((waves + 3) / 4, (int64_t)32 * cus));
+    FG_LAUNCH(embed_bwd_sorted4_kernel, dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D4, beta);
     return FG_OK;
   }
   const int grid = T < 2048 ? T : 2048;

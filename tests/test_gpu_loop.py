@@ -267,3 +267,40 @@ def test_train_loop_js(fh):
     ref = _first_loss_125m_oracle()
     print("125m first loss: gpu %.7f oracle %.7f" % (l0[0], ref))
     assert abs(l0[0] - ref) <= 1e-5 * abs(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,V", [(63, 9), (64, 9), (65, 9), (129, 2), (16384, 300), (16385, 300)])
+def test_embed_sort_keys_by_counting(fh, T, V):
+    """The counting sort at its edges (blocks of 64 positions, 16384 keys and
+    the first length that takes the network): invalid ids last, equal ids in
+    order of position."""
+    rng = np.random.default_rng(T)
+    ids = rng.integers(-1, V + 1, T).astype(np.int32)
+    P = keys_len(fh, T)
+    keys = fh.DeviceArray((P,), np.uint64)
+    fh.call("embed_sort_keys", keys, P, up(fh, ids), T, V)
+    t = np.arange(T, dtype=np.uint64)
+    exp = np.where((ids >= 0) & (ids < V), (ids.astype(np.uint64) << np.uint64(32)) | t, NO_KEY)
+    np.testing.assert_array_equal(keys.numpy(), np.sort(np.concatenate([exp, np.full(P - T, NO_KEY, np.uint64)])))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("run", [1, 31, 32, 33, 63, 64, 65, 127, 128, 200])
+@pytest.mark.parametrize("D", [4, 256, 260])
+def test_embed_bwd_sorted_run_lengths(fh, run, D):
+    """Runs of one id around the 64 keys read at a time and the rows loaded
+    at a time, at columns of one lane, whole waves and a remainder: the sums
+    in increasing position, bit for bit."""
+    ids = np.concatenate([np.full(run, 2), np.full(run, 0), [1]]).astype(np.int32)
+    T, V = len(ids), 4
+    rng = np.random.default_rng(run + D)
+    ids = rng.permutation(ids)
+    g = rng.standard_normal((T, D)).astype(np.float32)
+    P = keys_len(fh, T)
+    keys = fh.DeviceArray((P,), np.uint64)
+    fh.call("embed_sort_keys", keys, P, up(fh, ids), T, V)
+    gW = up(fh, np.zeros(V * D, np.float32))
+    fh.call("embed_bwd_sorted", gW, up(fh, g.ravel()), keys, T, V, D, 0)
+    ref = oracle.embed_bwd(g.ravel(), ids, V, D, gW=np.zeros(V * D, np.float32))
+    np.testing.assert_array_equal(gW.numpy(), ref)
