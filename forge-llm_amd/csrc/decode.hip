@@ -31,7 +31,7 @@
 // norm of x, or the attention combine) so the two overlap, and the attention
 // loads K and V rows together.
 #include "common.h"
-#include "qformat.h"
+#include "qdot.h"
 
 #include <math.h>
 
@@ -288,7 +288,10 @@ __global__ void __launch_bounds__(kThreads) dec_attn_part_kernel(double* __restr
   __shared__ double vsc[kChunk];
   __shared__ double pj[kChunk];
   __shared__ double red[PP][W4];
-  const int h = blockIdx.x, c = blockIdx.y;
+  // kv heads fastest: workgroups go round the XCDs in turn, so with eight kv
+  // heads (or a multiple) a group's query heads read their shared K and V rows
+  // through one L2
+  const int c = blockIdx.y, h = (blockIdx.x % nKV) * (nH / nKV) + blockIdx.x / nKV;
   const int pos = state[1];
   const int n = (pos >= 0 && pos < maxSeq) ? pos + 1 : 0;
   const int j0 = c * kChunk;
@@ -409,34 +412,31 @@ __global__ void __launch_bounds__(kThreads) dec_attn_part_kernel(double* __restr
   }
 }
 
-// x[n] = fp32(x[n] + fp32(Wo[n]·att)), where att is first combined from the
-// attention partials: per head M = max m, w_s = e^(m_s − M), l = Σ l_s·w_s,
-// att = fp32(fp32(Σ acc_s·w_s) · (1 / (l || 1))) (attention.js:55-57).
-// Dynamic LDS: att[D] floats (rounded up to 4), then w[nH·S], M[nH], inv[nH]
-// doubles.
-template <int QT>
-__global__ void __launch_bounds__(kThreads) dec_wo_kernel(float* __restrict__ x, const double* __restrict__ part,
-                                                          const int32_t* __restrict__ state,
-                                                          const uint8_t* __restrict__ W, int64_t rb, int D, int nH,
-                                                          int dH, int maxSeq, int S) {
-  extern __shared__ __attribute__((aligned(16))) float att[];
-  double* wsh = reinterpret_cast<double*>(att + ((D + 3) & ~3));
+// att (LDS, element i of the D at place(i)) combined from the attention
+// partials: per head M = max m, w_s = e^(m_s − M), l = Σ l_s·w_s,
+// att = fp32(fp32(Σ acc_s·w_s) · (1 / (l || 1))) (attention.js:55-57).  wsh:
+// w[nH·S], M[nH], inv[nH] doubles.  The partials' maxima are fetched by all
+// threads at once and the sums over chunks keep eight loads in flight: a
+// thread per head walking its chunks one load at a time took half the launch
+// (12 heads, 8 chunks: 9.7 us of launch, 6.6 now).
+template <typename Place>
+__device__ __forceinline__ void combine_to_lds(float* att, double* wsh, const double* __restrict__ part,
+                                               const int32_t* __restrict__ state, int D, int nH, int dH, int maxSeq,
+                                               int S, Place place) {
   double* Mh = wsh + nH * S;
   double* invh = Mh + nH;
-  const int stride = gridDim.x * kWaves;
-  int r = blockIdx.x * kWaves + (threadIdx.x >> 6);
-  WRows<QT, 1> rw;
-  if (r < D) {
-    rw.set(0, W, r, rb);
-    rw.prefetch(D);
-  }
   const int pos = state[1];
   const int n = (pos >= 0 && pos < maxSeq) ? pos + 1 : 0;
   const int Sa = (n + kChunk - 1) / kChunk;
+  for (int i = threadIdx.x; i < nH * Sa; i += kThreads) {
+    const int hh = i / Sa, s = i - hh * Sa;
+    wsh[hh * S + s] = part[((int64_t)hh * S + s) * (dH + 2)];
+  }
+  __syncthreads();
   for (int hh = threadIdx.x; hh < nH; hh += kThreads) {
     double M = -INFINITY;
     for (int s = 0; s < Sa; ++s) {
-      const double m = part[((int64_t)hh * S + s) * (dH + 2)];
+      const double m = wsh[hh * S + s];
       M = m > M ? m : M;
     }
     Mh[hh] = M;
@@ -444,11 +444,12 @@ __global__ void __launch_bounds__(kThreads) dec_wo_kernel(float* __restrict__ x,
   __syncthreads();
   for (int i = threadIdx.x; i < nH * Sa; i += kThreads) {
     const int hh = i / Sa, s = i - hh * Sa;
-    wsh[hh * S + s] = exp(part[((int64_t)hh * S + s) * (dH + 2)] - Mh[hh]);
+    wsh[hh * S + s] = exp(wsh[hh * S + s] - Mh[hh]);
   }
   __syncthreads();
   for (int hh = threadIdx.x; hh < nH; hh += kThreads) {
     double l = 0.0;
+#pragma unroll 8
     for (int s = 0; s < Sa; ++s) l += part[((int64_t)hh * S + s) * (dH + 2) + 1] * wsh[hh * S + s];
     invh[hh] = (l != 0.0 && l == l) ? 1.0 / l : 1.0;  // `1 / (l || 1)`
   }
@@ -456,10 +457,30 @@ __global__ void __launch_bounds__(kThreads) dec_wo_kernel(float* __restrict__ x,
   for (int i = threadIdx.x; i < D; i += kThreads) {
     const int hh = i / dH, d = i - hh * dH;
     double o = 0.0;
+#pragma unroll 8
     for (int s = 0; s < Sa; ++s) o += part[((int64_t)hh * S + s) * (dH + 2) + 2 + d] * wsh[hh * S + s];
-    att[i] = (float)((double)(float)o * invh[hh]);
+    att[place(i)] = (float)((double)(float)o * invh[hh]);
   }
   __syncthreads();
+}
+
+// x[n] = fp32(x[n] + fp32(Wo[n]·att)), att combined by every workgroup.
+// Dynamic LDS: att[D] floats (rounded up to 4), then combine_to_lds' doubles.
+template <int QT>
+__global__ void __launch_bounds__(kThreads) dec_wo_kernel(float* __restrict__ x, const double* __restrict__ part,
+                                                          const int32_t* __restrict__ state,
+                                                          const uint8_t* __restrict__ W, int64_t rb, int D, int nH,
+                                                          int dH, int maxSeq, int S) {
+  extern __shared__ __attribute__((aligned(16))) float att[];
+  const int stride = gridDim.x * kWaves;
+  int r = blockIdx.x * kWaves + (threadIdx.x >> 6);
+  WRows<QT, 1> rw;
+  if (r < D) {
+    rw.set(0, W, r, rb);
+    rw.prefetch(D);
+  }
+  combine_to_lds(att, reinterpret_cast<double*>(att + ((D + 3) & ~3)), part, state, D, nH, dH, maxSeq, S,
+                 [](int i) { return i; });
   for (bool first = true; r < D; r += stride, first = false) {
     if (!first) {
       rw.set(0, W, r, rb);
@@ -566,6 +587,294 @@ __global__ void __launch_bounds__(kThreads) dec_head_kernel(float* __restrict__ 
   }
 }
 
+// ───────── the five matvecs over half and quantized matrices ─────────
+// Rows in the unit form of qdot.h: one kernel, parametrised by what precedes
+// the product (Op::prologue fills x in unit order), which rows a group of R
+// holds and what becomes of their sums.  A group's first loads are issued
+// before the prologue.
+constexpr int kUnitRows = 4;
+static_assert(fgq::kUnitThreads == kThreads, "combine_to_lds strides by kThreads");
+
+// fp32(x·ss·w) of rmsnorm_to_lds, in unit order; x in registers between the
+// two passes (K <= 8192: eight float4 per thread).
+template <int QT>
+__device__ __forceinline__ void rmsnorm_to_units(float* xs, const float* __restrict__ x, bool ok, float* copy,
+                                                 const float* __restrict__ w, int K, double eps, double* sh) {
+#pragma clang fp contract(off)
+  const int U = K / fgq::unit_elems(QT);
+  float4 v[8];
+  double s = 0.0;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    const int i = 4 * (threadIdx.x + t * fgq::kUnitThreads);
+    if (i < K) {
+      v[t] = ok ? *reinterpret_cast<const float4*>(x + i) : make_float4(NAN, NAN, NAN, NAN);
+      if (copy) *reinterpret_cast<float4*>(copy + i) = v[t];
+      s += (double)v[t].x * v[t].x;
+      s += (double)v[t].y * v[t].y;
+      s += (double)v[t].z * v[t].z;
+      s += (double)v[t].w * v[t].w;
+    }
+  }
+  s = fg_wave_sum_d(s);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  double t8 = 0.0;
+  for (int i = 0; i < fgq::kUnitWaves; ++i) t8 += sh[i];
+  const double rms = sqrt(t8 / K);
+  const double ss = 1.0 / sqrt(rms * rms + eps);
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    const int i = 4 * (threadIdx.x + t * fgq::kUnitThreads);
+    if (i < K) {
+      const float4 g = *reinterpret_cast<const float4*>(w + i);
+      *reinterpret_cast<float4*>(xs + fgq::x_place<QT>(i, U)) =
+          make_float4((float)(((double)v[t].x * ss) * (double)g.x), (float)(((double)v[t].y * ss) * (double)g.y),
+                      (float)(((double)v[t].z * ss) * (double)g.z), (float)(((double)v[t].w * ss) * (double)g.w));
+    }
+  }
+}
+
+template <int QT>
+__device__ __forceinline__ void copy_to_units(float* xs, const float* __restrict__ x, int K) {
+  const int U = K / fgq::unit_elems(QT);
+  for (int i = 4 * threadIdx.x; i < K; i += 4 * fgq::kUnitThreads)
+    *reinterpret_cast<float4*>(xs + fgq::x_place<QT>(i, U)) = *reinterpret_cast<const float4*>(x + i);
+}
+
+struct QkvOp {
+  float *q, *kc, *vc, *x;
+  const float* emb;
+  int V;
+  const float* ln1;
+  double eps;
+  const uint8_t* W;
+  int64_t rb;
+  const float *rcos, *rsin;
+  const int32_t* state;
+  int D, qD, kvD, dH, maxSeq;
+  int64_t layer_off;
+  __device__ int rows() const { return qD + 2 * kvD; }
+  __device__ const uint8_t* row(int n) const { return W + min(n, rows() - 1) * rb; }
+  template <int QT>
+  __device__ void prologue(float* xs, double* sh) const {
+    const int tok = emb ? state[0] : 0;
+    const bool ok = !emb || (tok >= 0 && tok < V);
+    rmsnorm_to_units<QT>(xs, emb && ok ? emb + (int64_t)tok * D : x, ok, emb && blockIdx.x == 0 ? x : nullptr, ln1, D,
+                         eps, sh);
+  }
+  __device__ void store(int n0, const double (&s)[kUnitRows]) const {
+#pragma clang fp contract(off)
+    const int pos = state[1];
+    if (pos < 0 || pos >= maxSeq) return;  // the host rejects such positions
+    const int half = dH >> 1;
+    const int64_t cache_off = layer_off + (int64_t)pos * kvD;
+#pragma unroll
+    for (int r = 0; r < kUnitRows; r += 2) {  // rows() is even: whole pairs
+      const int n = n0 + r;
+      if (n >= rows()) break;
+      const float a = (float)s[r], b = (float)s[r + 1];
+      if (n < qD + kvD) {
+        const int i2 = (n % dH) >> 1;
+        const double c = rcos[pos * half + i2], sn = rsin[pos * half + i2];
+        const float o0 = (float)((double)a * c - (double)b * sn);
+        const float o1 = (float)((double)a * sn + (double)b * c);
+        float* o = n < qD ? q + n : kc + cache_off + n - qD;
+        o[0] = o0;
+        o[1] = o1;
+      } else {
+        vc[cache_off + n - qD - kvD] = a;
+        vc[cache_off + n - qD - kvD + 1] = b;
+      }
+    }
+  }
+};
+
+// x += W·in (the output and down projections)
+struct ResidOp {
+  float* x;
+  const float* in;
+  const uint8_t* W;
+  int64_t rb;
+  int N, K;
+  __device__ int rows() const { return N; }
+  __device__ const uint8_t* row(int n) const { return W + min(n, N - 1) * rb; }
+  template <int QT>
+  __device__ void prologue(float* xs, double*) const { copy_to_units<QT>(xs, in, K); }
+  __device__ void store(int n0, const double (&s)[kUnitRows]) const {
+#pragma unroll
+    for (int r = 0; r < kUnitRows; ++r)
+      if (n0 + r < N) x[n0 + r] = (float)((double)x[n0 + r] + (double)(float)s[r]);
+  }
+};
+
+// x += Wo·att with the partials combined by every workgroup (short caches)
+struct WoOp {
+  float* x;
+  const double* part;
+  const int32_t* state;
+  const uint8_t* W;
+  int64_t rb;
+  int D, nH, dH, maxSeq, S;
+  __device__ int rows() const { return D; }
+  __device__ const uint8_t* row(int n) const { return W + min(n, D - 1) * rb; }
+  template <int QT>
+  __device__ void prologue(float* xs, double*) const {
+    const int U = D / fgq::unit_elems(QT);
+    combine_to_lds(xs, reinterpret_cast<double*>(xs + D), part, state, D, nH, dH, maxSeq, S,
+                   [=](int i) { return fgq::x_place<QT>(i & ~3, U) + (i & 3); });
+  }
+  __device__ void store(int n0, const double (&s)[kUnitRows]) const {
+#pragma unroll
+    for (int r = 0; r < kUnitRows; ++r)
+      if (n0 + r < D) x[n0 + r] = (float)((double)x[n0 + r] + (double)(float)s[r]);
+  }
+};
+
+// rows 4i .. 4i + 3 of a group: gate 2i, up 2i, gate 2i + 1, up 2i + 1
+struct GateUpOp {
+  float* h;
+  const float *x, *ln2;
+  double eps;
+  const uint8_t *Wg, *Wu;
+  int64_t rb;
+  int H, D;
+  __device__ int rows() const { return 2 * H; }
+  __device__ const uint8_t* row(int n) const { return ((n & 1) ? Wu : Wg) + min(n >> 1, H - 1) * rb; }
+  template <int QT>
+  __device__ void prologue(float* xs, double* sh) const {
+    rmsnorm_to_units<QT>(xs, x, true, nullptr, ln2, D, eps, sh);
+  }
+  __device__ void store(int n0, const double (&s)[kUnitRows]) const {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int r = 0; r < kUnitRows; r += 2) {
+      const int j = (n0 + r) >> 1;
+      if (j >= H) break;
+      const double g = (double)(float)s[r], u = (double)(float)s[r + 1];
+      h[j] = (float)((g / (1.0 + exp(-g))) * u);
+    }
+  }
+};
+
+struct HeadOp {
+  float* logits;
+  const float *x, *lnf;
+  double eps;
+  const uint8_t* W;
+  int64_t rb;
+  int V, D;
+  __device__ int rows() const { return V; }
+  __device__ const uint8_t* row(int n) const { return W + (int64_t)min(n, V - 1) * rb; }
+  template <int QT>
+  __device__ void prologue(float* xs, double* sh) const {
+    rmsnorm_to_units<QT>(xs, x, true, nullptr, lnf, D, eps, sh);
+  }
+  __device__ void store(int n0, const double (&s)[kUnitRows]) const {
+#pragma unroll
+    for (int r = 0; r < kUnitRows; ++r)
+      if (n0 + r < V) logits[n0 + r] = (float)s[r];
+  }
+};
+
+template <int QT, typename Op>
+__global__ void __launch_bounds__(fgq::kUnitThreads, 3) dec_unit_kernel(Op op, int U, int P) {
+  extern __shared__ __attribute__((aligned(16))) float xs[];
+  __shared__ double red[fgq::kUnitWaves][kUnitRows];
+  __shared__ double sh[fgq::kUnitWaves];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int part = wave & (P - 1), slots = fgq::kUnitWaves / P, groups = (op.rows() + kUnitRows - 1) / kUnitRows;
+  int g = blockIdx.x * slots + wave / P;
+  fgq::UnitRows<QT, kUnitRows> rw;
+  auto start = [&]() {
+    if (g >= groups) return;
+#pragma unroll
+    for (int r = 0; r < kUnitRows; ++r) rw.row[r] = op.row(g * kUnitRows + r);
+    rw.start(U, part);
+  };
+  start();
+  op.template prologue<QT>(xs, sh);
+  __syncthreads();
+  for (int base = blockIdx.x * slots; base < groups; base += gridDim.x * slots) {
+    const int n0 = g * kUnitRows;
+    double acc[kUnitRows];
+    if (g < groups) {
+      rw.finish(acc, xs, U, part, P);
+    } else {
+#pragma unroll
+      for (int r = 0; r < kUnitRows; ++r) acc[r] = 0.0;
+    }
+    const bool on = g < groups;
+    g += gridDim.x * slots;
+    start();
+    fgq::unit_reduce<kUnitRows>(acc, red, P);
+    if ((threadIdx.x & 63) == 0 && part == 0 && on) op.store(n0, acc);
+  }
+}
+
+inline bool aligned16(const void* p) { return (uintptr_t)p % 16 == 0; }
+// Whether matrix rows of K run in the unit form: a type that has it, whole
+// units, aligned blocks, and x with the kernel's own arrays in 64 KB of LDS.
+inline bool use_units(int type, const void* W, int K) {
+  const int e = type == fgq::kF16    ? fgq::unit_elems(fgq::kF16)
+                : type == fgq::kQ8_0 ? fgq::unit_elems(fgq::kQ8_0)
+                : type == fgq::kQ4_K || type == fgq::kQ5_K || type == fgq::kQ6_K ? fgq::unit_elems(fgq::kQ4_K) : 0;
+  return e > 0 && K % e == 0 && K <= 16000 && aligned16(W);
+}
+template <int QT, typename Op>
+int launch_unit(const Op& op, int rows, int K, size_t more_lds = 0) {
+  if constexpr (fgq::has_units(QT)) {
+    const int U = K / fgq::unit_elems(QT), P = fgq::unit_parts(U), slots = fgq::kUnitWaves / P;
+    const int groups = (rows + kUnitRows - 1) / kUnitRows;
+    const int cap = 8 * (fg::device_cu_count() > 0 ? fg::device_cu_count() : 256);
+    FG_LAUNCH((dec_unit_kernel<QT, Op>), dim3((unsigned)min((groups + slots - 1) / slots, cap)),
+              dim3(fgq::kUnitThreads), (size_t)K * sizeof(float) + more_lds, op, U, P);
+  }
+  return FG_OK;
+}
+
+// att = the combined attention of dec_wo_kernel's prologue, once for all of
+// its consumers: for long caches each workgroup of the output projection
+// reading every partial (nH·S·dH doubles, 1 MB at 32 heads x 32 chunks x 128)
+// cost more than the projection.  One workgroup per 64 columns of a head, its
+// four waves over the chunks.
+__global__ void __launch_bounds__(kThreads) dec_combine_kernel(float* __restrict__ att, const double* __restrict__ part,
+                                                               const int32_t* __restrict__ state, int dH, int maxSeq,
+                                                               int S) {
+  __shared__ double red[kWaves][64], rl[kWaves];
+  const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, d = blockIdx.y * 64 + lane;
+  const int pos = state[1];
+  const int n = (pos >= 0 && pos < maxSeq) ? pos + 1 : 0;
+  const int Sa = (n + kChunk - 1) / kChunk;
+  const double* p = part + (int64_t)h * S * (dH + 2);
+  double M = -INFINITY;
+  for (int s = lane; s < Sa; s += 64) {
+    const double m = p[(int64_t)s * (dH + 2)];
+    M = m > M ? m : M;
+  }
+  M = wave_max_d(M);
+  double o = 0.0, l = 0.0;
+  const int per = (Sa + kWaves - 1) / kWaves, s1 = min(Sa, (wave + 1) * per);
+#pragma unroll 4
+  for (int s = wave * per; s < s1; ++s) {
+    const double* ps = p + (int64_t)s * (dH + 2);
+    const double w = exp(ps[0] - M);
+    l += ps[1] * w;
+    if (d < dH) o += ps[2 + d] * w;
+  }
+  red[wave][lane] = o;
+  if (lane == 0) rl[wave] = l;
+  __syncthreads();
+  if (wave == 0 && d < dH) {
+    for (int w = 1; w < kWaves; ++w) {
+      o += red[w][lane];
+      l += rl[w];
+    }
+    const double inv = (l != 0.0 && l == l) ? 1.0 / l : 1.0;  // `1 / (l || 1)`
+    att[h * dH + d] = (float)((double)(float)o * inv);
+  }
+}
+
 unsigned grid_for_waves(int64_t waves) {
   int64_t g = (waves + kWaves - 1) / kWaves;
   const int64_t cap = (int64_t)(fg::device_cu_count() > 0 ? fg::device_cu_count() : 256) * 16;
@@ -627,6 +936,8 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
   while (4 * LP < dH && LP < 64) LP <<= 1;
   fg::KProfScope prof("decode_step", 0.0, (double)wbytes);
   const bool emb_f32 = m->emb_type == fgq::kF32;
+  // the unit kernels read the vectors as float4
+  const bool vec = aligned16(m->x) && aligned16(m->q) && aligned16(m->h) && aligned16(m->tok_emb) && aligned16(m->ln_f);
   if (!emb_f32) {
     const uint8_t* emb = static_cast<const uint8_t*>(m->tok_emb);
     const int64_t erb = fgq::row_bytes(m->emb_type, D);
@@ -642,7 +953,14 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
     {
       const uint8_t* W = static_cast<const uint8_t*>(ly.wqkv);
       const int64_t rb = fgq::row_bytes(ly.wqkv_type, D);
-      FGQ_DISPATCH(ly.wqkv_type, {
+      if (vec && aligned16(ly.ln1) && use_units(ly.wqkv_type, W, D)) {
+        const QkvOp op{m->q, kcache, vcache, m->x, emb0, V, ly.ln1, eps, W, rb, m->rope_cos, m->rope_sin, state,
+                       D, qD, kvD, dH, m->maxSeq, layer_off};
+        FGQ_DISPATCH(ly.wqkv_type, {
+          const int rc = launch_unit<QT>(op, qD + 2 * kvD, D);
+          if (rc) return rc;
+        });
+      } else FGQ_DISPATCH(ly.wqkv_type, {
         FG_LAUNCH(dec_qkv_kernel<QT>, dim3(grid_for_waves((qD + 2 * kvD) / 2)), dim3(kThreads), lds_qkv, m->q,
                   kcache, vcache, m->x, emb0, V, ly.ln1, eps, W, rb, m->rope_cos, m->rope_sin, state, D, qD, kvD,
                   dH, m->maxSeq, layer_off);
@@ -666,7 +984,25 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
     {
       const uint8_t* W = static_cast<const uint8_t*>(ly.wo);
       const int64_t rb = fgq::row_bytes(ly.wo_type, D);
-      FGQ_DISPATCH(ly.wo_type, {
+      // a workgroup reads all nH·S·dH partials when it combines them itself
+      // (98 KB at 768 x 16 chunks); beyond that one more launch combines them
+      // once, into q's place
+      const size_t comb = ((size_t)nH * S + 2 * nH) * sizeof(double);
+      if (vec && use_units(ly.wo_type, W, D) && (int64_t)D * S <= 16384 && lds_wo <= 60 * 1024) {
+        const WoOp op{m->x, (const double*)m->attn_part, state, W, rb, D, nH, dH, m->maxSeq, S};
+        FGQ_DISPATCH(ly.wo_type, {
+          const int rc = launch_unit<QT>(op, D, D, comb);
+          if (rc) return rc;
+        });
+      } else if (vec && use_units(ly.wo_type, W, D)) {
+        FG_LAUNCH(dec_combine_kernel, dim3(nH, (dH + 63) / 64), dim3(kThreads), 0, m->q, (const double*)m->attn_part,
+                  state, dH, m->maxSeq, S);
+        const ResidOp op{m->x, m->q, W, rb, D, D};
+        FGQ_DISPATCH(ly.wo_type, {
+          const int rc = launch_unit<QT>(op, D, D);
+          if (rc) return rc;
+        });
+      } else FGQ_DISPATCH(ly.wo_type, {
         FG_LAUNCH(dec_wo_kernel<QT>, dim3(grid_for_waves(D)), dim3(kThreads), lds_wo, m->x,
                   (const double*)m->attn_part, state, W, rb, D, nH, dH, m->maxSeq, S);
       });
@@ -675,7 +1011,13 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
       const uint8_t* Wg = static_cast<const uint8_t*>(ly.gate);
       const uint8_t* Wu = static_cast<const uint8_t*>(ly.up);
       const int64_t rb = fgq::row_bytes(ly.gate_type, D);
-      FGQ_DISPATCH(ly.gate_type, {
+      if (vec && aligned16(ly.ln2) && use_units(ly.gate_type, Wg, D) && use_units(ly.gate_type, Wu, D)) {
+        const GateUpOp op{m->h, m->x, ly.ln2, eps, Wg, Wu, rb, H, D};
+        FGQ_DISPATCH(ly.gate_type, {
+          const int rc = launch_unit<QT>(op, 2 * H, D);
+          if (rc) return rc;
+        });
+      } else FGQ_DISPATCH(ly.gate_type, {
         FG_LAUNCH(dec_gateup_kernel<QT>, dim3(grid_for_waves(H)), dim3(kThreads), D * sizeof(float), m->h, m->x,
                   ly.ln2, eps, Wg, Wu, rb, H, D);
       });
@@ -683,7 +1025,13 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
     {
       const uint8_t* W = static_cast<const uint8_t*>(ly.down);
       const int64_t rb = fgq::row_bytes(ly.down_type, H);
-      FGQ_DISPATCH(ly.down_type, {
+      if (vec && use_units(ly.down_type, W, H)) {
+        const ResidOp op{m->x, m->h, W, rb, D, H};
+        FGQ_DISPATCH(ly.down_type, {
+          const int rc = launch_unit<QT>(op, D, H);
+          if (rc) return rc;
+        });
+      } else FGQ_DISPATCH(ly.down_type, {
         FG_LAUNCH(dec_down_kernel<QT>, dim3(grid_for_waves(D)), dim3(kThreads), H * sizeof(float), m->x,
                   m->h, W, rb, D, H);
       });
@@ -692,7 +1040,13 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
   {
     const uint8_t* W = static_cast<const uint8_t*>(m->wcls);
     const int64_t rb = fgq::row_bytes(m->cls_type, D);
-    FGQ_DISPATCH(m->cls_type, {
+    if (vec && use_units(m->cls_type, W, D)) {
+      const HeadOp op{logits, m->x, m->ln_f, eps, W, rb, V, D};
+      FGQ_DISPATCH(m->cls_type, {
+        const int rc = launch_unit<QT>(op, V, D);
+        if (rc) return rc;
+      });
+    } else FGQ_DISPATCH(m->cls_type, {
       FG_LAUNCH(dec_head_kernel<QT>, dim3(grid_for_waves((V + 1) / 2)), dim3(kThreads), D * sizeof(float), logits,
                 m->x, m->ln_f, eps, W, rb, V, D);
     });

@@ -4,9 +4,9 @@
 //   fg_dequantize  out = dequantize(q)             quant.js:102-199, bit-exact
 //   fg_quantize    q = quantizeRow(x)              quant.js:322-590, bit-exact
 //
-// The matvec is HBM-bound (a weight is read once per call): one wave per two
-// rows, x staged once per workgroup in LDS, per-format lane mappings from
-// qformat.h.  Decoding is exact integer/fp16 work; sums are fp64.
+// The matvec is HBM-bound (a weight is read once per call): units of qdot.h
+// for F16, Q8_0 and the K-quants; otherwise one wave per two rows, x staged
+// once per workgroup in LDS, per-format lane mappings from qformat.h.  Decoding is exact integer/fp16 work; sums are fp64.
 //
 // The quantizers restate the reference's scalar algorithms (closed-form
 // Q8_0 and Q4_K, the make_qx_quants / make_qkx2_quants searches of Q6_K and
@@ -17,7 +17,7 @@
 // the bytes are identical to it.  Quantization is a one-time load step, not a
 // per-token cost.
 #include "common.h"
-#include "qformat.h"
+#include "qdot.h"
 
 #include <math.h>
 
@@ -56,6 +56,53 @@ __global__ void __launch_bounds__(kThreads) qmatvec_kernel(OutT* __restrict__ y,
     for (int r = 0; r < R; ++r) {
       const double s = fg_wave_sum_d(acc[r]);
       if ((threadIdx.x & 63) == 0 && r0 + r < N) y[r0 + r] = (OutT)s;
+    }
+  }
+}
+
+// The types with a unit form (qdot.h): R rows per wave group, P waves sharing
+// a row's units, x staged in unit order by each workgroup after the loads of
+// its first rows are on their way.
+template <int QT, int R, typename OutT>
+__global__ void __launch_bounds__(kUnitThreads, 3) qmatvec_unit_kernel(OutT* __restrict__ y,
+                                                                       const uint8_t* __restrict__ W,
+                                                                       const float* __restrict__ x, int N, int K,
+                                                                       int64_t rb, int P) {
+  extern __shared__ __attribute__((aligned(16))) float xs[];
+  __shared__ double red[kUnitWaves][R];
+  const int U = K / unit_elems(QT);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int part = wave & (P - 1), slots = kUnitWaves / P, groups = (N + R - 1) / R;
+  int g = blockIdx.x * slots + wave / P;
+  UnitRows<QT, R> rw;
+  auto start = [&]() {
+    if (g >= groups) return;
+#pragma unroll
+    for (int r = 0; r < R; ++r) rw.row[r] = W + (int64_t)min(g * R + r, N - 1) * rb;
+    rw.start(U, part);
+  };
+  start();
+  for (int i = 4 * threadIdx.x; i < K; i += 4 * kUnitThreads) {
+    const float4 v = make_float4(x[i], x[i + 1], x[i + 2], x[i + 3]);
+    *reinterpret_cast<float4*>(xs + x_place<QT>(i, U)) = v;
+  }
+  __syncthreads();
+  for (int base = blockIdx.x * slots; base < groups; base += gridDim.x * slots) {
+    const int r0 = g * R;
+    double acc[R];
+    if (g < groups) {
+      rw.finish(acc, xs, U, part, P);
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) acc[r] = 0.0;
+    }
+    g += gridDim.x * slots;
+    start();  // the next rows' loads cross the reduction
+    unit_reduce<R>(acc, red, P);
+    if ((threadIdx.x & 63) == 0 && part == 0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (r0 + r < N) y[r0 + r] = (OutT)acc[r];
     }
   }
 }
@@ -446,16 +493,30 @@ unsigned grid_for(int64_t items, int per_block) {
 
 template <int QT, typename OutT>
 int launch_qmatvec(OutT* y, const uint8_t* W, const float* x, int N, int K) {
-  constexpr int R = 2;
   const int64_t rb = row_bytes(QT, K);
-  const bool lds = (size_t)K * sizeof(float) <= 64 * 1024;
-  // up to 8 workgroups per CU (a launch-shape sweep over rows per wave, split
-  // K and workgroups per CU at the Llama-3-8B shapes found this the fastest
-  // for every type; x is staged once per workgroup)
-  int64_t g = ((N + R - 1) / R + kWaves - 1) / kWaves;
-  const int64_t cap = (int64_t)(fg::device_cu_count() > 0 ? fg::device_cu_count() : 256) * 8;
-  if (g > cap) g = cap;
   fg::KProfScope prof("qmatvec", 2.0 * N * K, (double)rb * N + 4.0 * K + 4.0 * N);
+  const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
+  if constexpr (has_units(QT)) {
+    // x in LDS beside the kernel's own arrays (64 KB), whole units, aligned blocks
+    if (K <= 16000 && K % unit_elems(QT) == 0 && (uintptr_t)W % 16 == 0) {
+      const int P = unit_parts(K / unit_elems(QT)), slots = kUnitWaves / P;
+      // four rows per wave group, or one where that would leave CUs idle
+      const bool wide = (int64_t)((N + 3) / 4) * P >= 8LL * cus;
+      const int groups = wide ? (N + 3) / 4 : N;
+      const dim3 grid((unsigned)min((groups + slots - 1) / slots, 8 * cus)), block(kUnitThreads);
+      if (wide)
+        FG_LAUNCH((qmatvec_unit_kernel<QT, 4, OutT>), grid, block, (size_t)K * sizeof(float), y, W, x, N, K, rb, P);
+      else
+        FG_LAUNCH((qmatvec_unit_kernel<QT, 1, OutT>), grid, block, (size_t)K * sizeof(float), y, W, x, N, K, rb, P);
+      return FG_OK;
+    }
+  }
+  constexpr int R = 2;
+  const bool lds = (size_t)K * sizeof(float) <= 64 * 1024;
+  // up to 8 workgroups per CU (x is staged once per workgroup)
+  int64_t g = ((N + R - 1) / R + kWaves - 1) / kWaves;
+  const int64_t cap = (int64_t)cus * 8;
+  if (g > cap) g = cap;
   if (lds)
     FG_LAUNCH((qmatvec_kernel<QT, R, true, OutT>), dim3((unsigned)g), dim3(kThreads), (size_t)K * sizeof(float), y,
               W, x, N, K, rb);

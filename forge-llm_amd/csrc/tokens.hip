@@ -207,10 +207,10 @@ __global__ void __launch_bounds__(kRankThreads) sort_rank_kernel(uint64_t* __res
   const uint32_t* u = reinterpret_cast<const uint32_t*>(ids);
   int count = 0;
   const int e0 = min(hi, t0), m1 = min(hi, t0 + 64);
-#pragma unroll 16
+#pragma unroll 32
   for (int i = lo; i < e0; ++i) count += u[i] <= le;
   for (int i = max(lo, t0); i < m1; ++i) count += i < t ? u[i] <= le : u[i] < lt;
-#pragma unroll 16
+#pragma unroll 32
   for (int i = max(lo, t0 + 64); i < hi; ++i) count += u[i] < lt;
   part[wave][lane] = count;
   __syncthreads();
