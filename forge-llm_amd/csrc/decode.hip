@@ -412,6 +412,111 @@ __global__ void __launch_bounds__(kThreads) dec_attn_part_kernel(double* __restr
   }
 }
 
+// The same chunk of attention for head dims that are multiples of 4 up to 256
+// (LP = 8 .. 64 lanes of four dims each), built for latency: at batch 1 a
+// launch is one workgroup's chain.  Four lanes hold a position (LP / 4 float4
+// of its K row each, the 64 positions of a chunk in one pass, all loads with
+// those of q and V at the start), so a score takes two shuffles instead of
+// log2(LP) per pass; every wave then takes the maximum and the exponentials of
+// all 64 scores itself (lane = position), which saves a barrier and leaves p
+// where its V rows need it.  32 heads of 128 over 2048 positions 28.8 -> 11 us,
+// 12 heads of 64 over 500 9.0 -> 6.5 us.
+template <int LP>
+__global__ void __launch_bounds__(kThreads) dec_attn_chunk_kernel(double* __restrict__ part,
+                                                                  const float* __restrict__ q,
+                                                                  const float* __restrict__ kc,
+                                                                  const float* __restrict__ vc,
+                                                                  const int32_t* __restrict__ state, int nH, int nKV,
+                                                                  int dH, int maxSeq, int64_t layer_off, double scale,
+                                                                  int S) {
+#pragma clang fp contract(off)
+  constexpr int NJ = LP / 4;          // float4 of K per lane
+  constexpr int PP = kThreads / LP;   // position groups of p·V
+  constexpr int NT = kChunk / PP;     // positions per group
+  __shared__ double vsc[kChunk];
+  __shared__ double pj[kWaves][kChunk];
+  __shared__ double red[PP][4 * LP];
+  // kv heads fastest (see dec_attn_part_kernel)
+  const int c = blockIdx.y, h = (blockIdx.x % nKV) * (nH / nKV) + blockIdx.x / nKV;
+  const int pos = state[1];
+  const int n = (pos >= 0 && pos < maxSeq) ? pos + 1 : 0;
+  const int j0 = c * kChunk;
+  if (j0 >= n) return;
+  const int cnt = n - j0 < kChunk ? n - j0 : kChunk;
+  const int kvh = h / (nH / nKV), kvD = nKV * dH;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // scores: position sj, dims 4 (sl + 4 j)
+  const int sj = tid >> 2, sl = tid & 3;
+  const int pg = tid / LP, lc = tid % LP;  // p·V: positions pg + PP t, dims 4 lc
+  const float* kr = kc + layer_off + (int64_t)(j0 + (sj < cnt ? sj : 0)) * kvD + (int64_t)kvh * dH + 4 * sl;
+  const float* vr = vc + layer_off + (int64_t)j0 * kvD + (int64_t)kvh * dH + 4 * lc;
+  const float* qr = q + (int64_t)h * dH + 4 * sl;
+  const bool von = 4 * lc < dH;
+  float4 k4[NJ], q4[NJ], v4[NT];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+    if (4 * (sl + 4 * j) < dH) {
+      k4[j] = *reinterpret_cast<const float4*>(kr + 16 * j);
+      q4[j] = *reinterpret_cast<const float4*>(qr + 16 * j);
+    }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int jj = pg + PP * t;
+    if (jj < cnt && von) v4[t] = *reinterpret_cast<const float4*>(vr + (int64_t)jj * kvD);
+  }
+  double s = 0.0;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+    if (4 * (sl + 4 * j) < dH)
+      s += (double)q4[j].x * k4[j].x + (double)q4[j].y * k4[j].y + (double)q4[j].z * k4[j].z +
+           (double)q4[j].w * k4[j].w;
+  s += __shfl_xor(s, 1, 64);
+  s += __shfl_xor(s, 2, 64);
+  if (sl == 0) vsc[sj] = s * scale;
+  __syncthreads();
+  // chunk max (fp64 scores) and p = exp(fp32 score - m), lane = position
+  {
+    const double sc = lane < cnt ? vsc[lane] : -INFINITY;
+    double m = sc > -INFINITY ? sc : -INFINITY;  // NaN scores never raise the max
+    m = wave_max_d(m);
+    const float sf = (float)sc;
+    const double p = lane < cnt && sf != -INFINITY ? exp((double)sf - m) : 0.0;
+    pj[wave][lane] = p;
+    if (wave == 0) {
+      const double l = fg_wave_sum_d(p);
+      if (lane == 0) {
+        double* out = part + ((int64_t)h * S + c) * (dH + 2);
+        out[0] = m;
+        out[1] = l;
+      }
+    }
+  }
+  // each wave reads back its own copy of p
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int jj = pg + PP * t;
+    if (jj >= cnt || !von) break;
+    const double p = pj[wave][jj];
+    if (p == 0.0) continue;  // the reference skips p = 0 (attention.js:48)
+    acc[0] += p * (double)v4[t].x;
+    acc[1] += p * (double)v4[t].y;
+    acc[2] += p * (double)v4[t].z;
+    acc[3] += p * (double)v4[t].w;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) red[pg][4 * lc + e] = acc[e];
+  __syncthreads();
+  double* out = part + ((int64_t)h * S + c) * (dH + 2) + 2;
+  for (int i = tid; i < dH; i += kThreads) {
+    double o = 0.0;
+#pragma unroll
+    for (int g = 0; g < PP; ++g) o += red[g][i];
+    out[i] = o;
+  }
+}
+
 // att (LDS, element i of the D at place(i)) combined from the attention
 // partials: per head M = max m, w_s = e^(m_s − M), l = Σ l_s·w_s,
 // att = fp32(fp32(Σ acc_s·w_s) · (1 / (l || 1))) (attention.js:55-57).  wsh:
@@ -826,7 +931,10 @@ int launch_unit(const Op& op, int rows, int K, size_t more_lds = 0) {
   if constexpr (fgq::has_units(QT)) {
     const int U = K / fgq::unit_elems(QT), P = fgq::unit_parts(U), slots = fgq::kUnitWaves / P;
     const int groups = (rows + kUnitRows - 1) / kUnitRows;
-    const int cap = 8 * (fg::device_cu_count() > 0 ? fg::device_cu_count() : 256);
+    // one round of resident workgroups (three by registers, fewer by LDS): a
+    // second round would repeat the prologue
+    const int per_cu = min(3, (int)((160 * 1024) / ((size_t)K * sizeof(float) + more_lds + 512)));
+    const int cap = per_cu * (fg::device_cu_count() > 0 ? fg::device_cu_count() : 256);
     FG_LAUNCH((dec_unit_kernel<QT, Op>), dim3((unsigned)min((groups + slots - 1) / slots, cap)),
               dim3(fgq::kUnitThreads), (size_t)K * sizeof(float) + more_lds, op, U, P);
   }
@@ -967,7 +1075,19 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
       });
     }
     int rc;
-    switch (LP) {
+    const bool chunk = dH % 4 == 0 && dH > 16 && dH <= 256 && aligned16(m->q) && aligned16(kcache) && aligned16(vcache);
+    const dim3 agrid(nH, S), ablock(kThreads);
+#define FG_CHUNK(LPS)                                                                                              \
+  FG_LAUNCH((dec_attn_chunk_kernel<LPS>), agrid, ablock, 0, m->attn_part, m->q, kcache, vcache, state, nH, nKV, dH, \
+            m->maxSeq, layer_off, scale, S)
+    if (chunk) {
+      rc = FG_OK;
+      if (LP == 8) FG_CHUNK(8);
+      else if (LP == 16) FG_CHUNK(16);
+      else if (LP == 32) FG_CHUNK(32);
+      else FG_CHUNK(64);
+    } else switch (LP) {
+#undef FG_CHUNK
       case 1: rc = launch_attn<1>(m, kcache, vcache, state, dH, layer_off, scale, S); break;
       case 2: rc = launch_attn<2>(m, kcache, vcache, state, dH, layer_off, scale, S); break;
       case 4: rc = launch_attn<4>(m, kcache, vcache, state, dH, layer_off, scale, S); break;
