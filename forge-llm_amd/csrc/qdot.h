@@ -6,10 +6,9 @@
 // block (Q4_K, Q5_K, Q6_K: a run of 16 low and 16 high nibbles, so two
 // sub-blocks with a scale each), 16 of a Q8_0 block, 8 halves.  A unit's
 // quants are one 16-byte load per plane, at whatever alignment the block size
-// leaves (34 and 210 byte blocks are 2-byte aligned; the loads are unaligned
-// dwordx4, not shorts).  A wave takes R rows at a time: their loads of a step
-// are issued together and a step ahead of their use, the unit's x values and
-// their sums are formed once for all of them.
+// leaves.  A wave takes R rows at a time: their loads of a step are issued
+// together and a step ahead of their use, the unit's x values and their sums
+// are formed once for all of them.
 //
 // x sits in LDS in the order the lanes read it: granules of four values,
 // [64 units][granule of the unit][unit], so that every read is one
@@ -56,6 +55,9 @@ __device__ __forceinline__ int x_place(int i, int U) {
   return 4 * (u0 * G + v * n + (u - u0));
 }
 
+// Loads at any alignment (blocks of 34 and 210 bytes are 2-byte aligned): one
+// instruction.  Reading the words around the block and shifting them into
+// place measured slower (Q6_K, 128256 x 4096: 122 against 160 us).
 template <typename T>
 __device__ __forceinline__ T ld_any(const uint8_t* p) {
   T v;
@@ -152,9 +154,18 @@ __device__ __forceinline__ void unit_x(UnitX<QT>& X, const float* xs, int u, int
   }
 }
 
+// The four bytes of w as they are: without this the compiler sees through the
+// masks that made them and extracts each nibble before converting it, an
+// instruction more per element (v_cvt_f32_ubyte1..3 take bytes in place).
+__device__ __forceinline__ uint32_t as_bytes(uint32_t w) {
+  asm("" : "+v"(w));
+  return w;
+}
+
 // Four bytes of w times x, one fp32 run.
 __device__ __forceinline__ float dot4(uint32_t w, const float* x) {
   float f[4];
+  w = as_bytes(w);
   bytes_f32(w, f);
   float t = f[0] * x[0];
   t = fmaf(f[1], x[1], t);
@@ -183,8 +194,8 @@ __device__ __forceinline__ void unit_dot(double& acc, const Unit<QT>& f, const U
         hi |= ((hs >> 1) & 0x01010101u) << 4;
       }
       float fl[4], fh[4];
-      bytes_f32(lo, fl);
-      bytes_f32(hi, fh);
+      bytes_f32(as_bytes(lo), fl);
+      bytes_f32(as_bytes(hi), fh);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         al = fmaf(fl[i], X.x[4 * v + i], al);
@@ -211,11 +222,10 @@ __device__ __forceinline__ void unit_dot(double& acc, const Unit<QT>& f, const U
     acc = fma((double)(d * (float)(int8_t)(f.sc.y >> by)), ah, acc);
   } else if constexpr (QT == kQ8_0) {
     // int8 q = (q ^ 0x80) - 128: unsigned bytes convert at full rate
+    const uint32_t qw[4] = {f.q.x, f.q.y, f.q.z, f.q.w};
     double a = -128.0 * (X.s0 + X.s1);
-    a += (double)dot4(f.q.x ^ 0x80808080u, X.x);
-    a += (double)dot4(f.q.y ^ 0x80808080u, X.x + 4);
-    a += (double)dot4(f.q.z ^ 0x80808080u, X.x + 8);
-    a += (double)dot4(f.q.w ^ 0x80808080u, X.x + 12);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) a += (double)dot4(qw[v] ^ 0x80808080u, X.x + 4 * v);
     acc = fma((double)h2f(f.d), a, acc);
   } else {
     const uint32_t hw[4] = {f.q.x, f.q.y, f.q.z, f.q.w};
@@ -269,13 +279,55 @@ inline int unit_parts(int U) {
   while (P < kUnitWaves && 64 * P < U) P <<= 1;
   return P;
 }
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov_d(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
+}
+// Sum over each row of 16 lanes (rotations within the row), in every lane.
+__device__ __forceinline__ double row16_sum(double v) {
+  v += dpp_mov_d<0x128>(v);  // row_ror:8
+  v += dpp_mov_d<0x124>(v);
+  v += dpp_mov_d<0x122>(v);
+  v += dpp_mov_d<0x121>(v);
+  return v;
+}
+__device__ __forceinline__ double lane_d(double v, int l) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
+  return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
+}
+// acc[r] = its sum over the wave, in every lane.  Four rows: two exchanges
+// leave each quarter of the wave one row to sum over its 16 lanes.
+template <int R>
+__device__ __forceinline__ void wave_rows_sum(double (&acc)[R]) {
+  if constexpr (R == 4) {
+    const int lane = threadIdx.x & 63;
+    const bool up = lane & 32, odd = lane & 16;
+    const double s0 = __shfl_xor(up ? acc[0] : acc[2], 32, 64), s1 = __shfl_xor(up ? acc[1] : acc[3], 32, 64);
+    const double a = (up ? acc[2] : acc[0]) + s0, b = (up ? acc[3] : acc[1]) + s1;
+    double c = (odd ? b : a) + __shfl_xor(odd ? a : b, 16, 64);
+    c = row16_sum(c);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = lane_d(c, 16 * r);
+  } else {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const double c = row16_sum(acc[r]);
+      acc[r] = (lane_d(c, 0) + lane_d(c, 16)) + (lane_d(c, 32) + lane_d(c, 48));
+    }
+  }
+}
+
 // Sums acc over the wave and the P waves of the group; the result is valid in
 // lane 0 of part 0.  Every wave of the workgroup calls it (barriers for P > 1).
 template <int R>
 __device__ __forceinline__ void unit_reduce(double (&acc)[R], double (*red)[R], int P) {
   const int wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int r = 0; r < R; ++r) acc[r] = fg_wave_sum_d(acc[r]);
+  wave_rows_sum<R>(acc);
   if (P == 1) return;
   __syncthreads();  // the previous group's sums have been read
   if ((threadIdx.x & 63) == 0) {
