@@ -32,6 +32,8 @@
 // contiguous range, then grouped 8 tile-rows at a time for L2 reuse.  When the
 // tile count cannot fill the chip, K is split across gridDim.y and partial
 // tiles are summed by a second kernel in a fixed order (deterministic).
+#include <type_traits>
+
 #include "common.h"
 #include "f16split.h"
 #include "swiglu_math.h"
@@ -1416,6 +1418,9 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(float* __restrict__ 
   splitk_sum(C, partial, n, splits, beta, resid);
 }
 
+}  // namespace
+#include "gemm_small.h"
+namespace {
 #include "gemm_pieces.h"
 
 // The grouped launch's K pieces, summed per job in order z = 0 .. splits - 1
@@ -1787,6 +1792,34 @@ int launch_gemm(const char* name, fg::Workspace& ws, float* C, const float* A, c
   const GemmPlan pl = plan_gemm(AK, BKc, M, N, K, cus);
   FG_ARG_CHECK(!parts_out || (pl.splits == 2 && !beta && !resid),
                "%s: the plan for M=%d N=%d K=%d takes %d K pieces, not two", name, M, N, K, pl.splits);
+  // small products (an input gradient that can be left in two pieces keeps them)
+  const SmallPlan sp = plan_small(M, N, K, AK && !BKc && pl.splits == 2 ? 2 : 0);
+  if (sp.waves) {
+    STable t = small_table(C, A, B, M, N, K, lda, ldb, beta, resid, xp);
+    if (sp.splits > 1) {
+      t.partial = parts_out;
+      if (!t.partial) {
+        int rc = ws.get(sizeof(float) * (size_t)sp.splits * M * N);
+        if (rc) return rc;
+        t.partial = (float*)ws.ptr;
+      }
+    }
+    {
+      fg::KProfScope prof(!scoped ? nullptr : AK ? (BKc ? "gemm_nt" : "gemm_nn") : "gemm_tn", 2.0 * M * N * (double)K,
+                          4.0 * ((double)M * K + (double)N * K + (1.0 + (beta ? 1.0 : 0.0) + (resid ? 1.0 : 0.0)) * M * N));
+      int rc = launch_small<AK, BKc>(t, sp, small_vec(AK, BKc, A, B, K, lda, ldb));
+      if (rc) return rc;
+    }
+    if (sp.splits > 1 && !parts_out) {
+      fg::KProfScope prof2(scoped ? "gemm_splitk_reduce" : nullptr, 0.0,
+                           4.0 * (double)M * N * (sp.splits + 1 + (beta ? 1 : 0) + (resid ? 1 : 0)));
+      const int64_t n = (int64_t)M * N;
+      int64_t blocks = (n / 4 + 255) / 256 + 1;
+      if (blocks > 8LL * cus) blocks = 8LL * cus;
+      FG_LAUNCH(splitk_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, C, t.partial, n, sp.splits, beta, resid);
+    }
+    return FG_OK;
+  }
   // input gradients keep the number of K pieces fg_matmulT_bwd_x_pieces names
   const PiecePlan pp = plan_pieces(M, N, K, cus, AK && !BKc ? pl.splits : 0);
   if (pp.wm) {
@@ -1967,6 +2000,15 @@ extern "C" int fg_matmulT_fwd_swiglu_p(float* O, float* GU, const float* X, cons
   FG_ARG_CHECK(M > 0 && K > 0 && H > 0, "fg_matmulT_fwd_swiglu: bad shape M=%d K=%d H=%d", M, K, H);
   FG_ARG_CHECK(O && GU && X && Wgu, "fg_matmulT_fwd_swiglu: null pointer");
   const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
+  // small: a workgroup takes a gate tile and its up tile (the plain
+  // forward's sums: the same plan)
+  const SmallPlan sp = plan_small(M, 2 * H, K, 0);
+  if (sp.waves && sp.splits == 1) {
+    STable t = small_table(GU, X, Wgu, M, H, K, K, K, 0, nullptr, XpArgs{xp_x, xp_w, have});
+    t.job[0].O = O;
+    fg::KProfScope prof("gemm_nt", 2.0 * M * 2.0 * H * K, 4.0 * ((double)M * K + 2.0 * H * K + 3.0 * (double)M * H));
+    return launch_small<true, true, true>(t, sp, small_vec(true, true, X, Wgu, K, K, K));
+  }
   // on pieces, where plan_pieces' choice for the plain forward is one that
   // the epilogue fits (the same products in the same order as that forward)
   const PiecePlan pp = plan_pieces(M, 2 * H, K, cus, 0);
@@ -2193,13 +2235,58 @@ int grouped_pieces(const fg_wgrad_job* jobs, int count, int cus, bool& done) {
 }
 }  // namespace
 
+namespace {
+// A list that is small as a whole: launches of up to kSmallJobs jobs on the
+// small kernel, each on distinct outputs.
+int grouped_small(const fg_wgrad_job* jobs, int count, bool& done) {
+  done = false;
+  int64_t work = 0;
+  for (int i = 0; i < count; ++i) {
+    const fg_wgrad_job& jb = jobs[i];
+    if (!(jb.gW && jb.gY && jb.X && jb.M > 0 && jb.K > 0 && jb.N > 0)) return FG_OK;  // reported by the caller
+    if ((int64_t)jb.M * jb.K > kSmallMax || (int64_t)jb.M * jb.K * jb.N > kSmallMax - work) return FG_OK;
+    work += (int64_t)jb.M * jb.K * jb.N;
+  }
+  for (int b = 0; b < count;) {
+    STable t;
+    t.partial = nullptr;
+    t.rope = RopeEpi{nullptr, nullptr, 0, 0, 0, 0};
+    t.count = t.tiles = 0;
+    int kmax = 0;
+    double flop = 0.0, bytes = 0.0;
+    for (; b < count && t.count < kSmallJobs; ++b) {
+      const fg_wgrad_job& jb = jobs[b];
+      bool again = false;
+      for (int j = 0; j < t.count; ++j) again |= t.job[j].C == jb.gW;
+      if (again) break;
+      // gW[N,K] (+)= gY^T · X: M_gemm = N, N_gemm = K, K_gemm = M
+      t.job[t.count++] = SJob{jb.gY, jb.X, jb.gW, nullptr, nullptr, nullptr, nullptr, jb.N, jb.K, jb.M, jb.N, jb.K,
+                              jb.beta ? 1 : 0, t.tiles};
+      t.tiles += (int)small_tiles(jb.N, jb.K);
+      kmax = jb.M > kmax ? jb.M : kmax;
+      flop += 2.0 * jb.M * jb.K * (double)jb.N;
+      bytes += 4.0 * ((double)jb.N * jb.M + (double)jb.K * jb.M + (jb.beta ? 2.0 : 1.0) * jb.N * jb.K);
+    }
+    SmallPlan p;
+    p.waves = small_waves(t.tiles, kmax);
+    fg::KProfScope prof("gemm_tn", flop, bytes);
+    int rc = launch_small<false, false>(t, p, true);
+    if (rc) return rc;
+  }
+  done = true;
+  return FG_OK;
+}
+}  // namespace
+
 extern "C" int fg_matmulT_bwd_w_grouped(const fg_wgrad_job* jobs, int count) {
   FG_REQUIRE_INIT();
   FG_ARG_CHECK(count >= 0 && (count == 0 || jobs), "fg_matmulT_bwd_w_grouped: bad job list");
   const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
   {
     bool done = false;
-    int rc = grouped_pieces(jobs, count, cus, done);
+    int rc = grouped_small(jobs, count, done);
+    if (rc || done) return rc;
+    rc = grouped_pieces(jobs, count, cus, done);
     if (rc || done) return rc;
   }
   // 256x256 tiles (gemm_w_grouped) when they make at least two rounds of
@@ -2363,13 +2450,22 @@ extern "C" int fg_matmulT_fwd_rope_p(float* Y, const float* X, const float* W, i
   FG_ARG_CHECK(M > 0 && pos0 >= 0 && posStride >= 0, "fg_matmulT_fwd_rope: bad rows/positions");
   const int maxpos = pos0 + (posStride > 0 ? (M < posStride ? M : posStride) : M) - 1;
   FG_ARG_CHECK(maxpos < npos, "fg_matmulT_fwd_rope: positions up to %d exceed the %d-entry table", maxpos, npos);
+  const RopeEpi re{cos_tab, sin_tab, (nH + nKV) * dH, dH, pos0, posStride};
+  const SmallPlan sp = K > 0 ? plan_small(M, N, K, 0) : SmallPlan();
+  if (sp.waves && sp.splits == 1) {  // small: turned in the epilogue
+    FG_REQUIRE_INIT();
+    FG_ARG_CHECK(Y && X && W, "matmulT_fwd_rope: null pointer");
+    STable t = small_table(Y, X, W, M, N, K, K, K, 0, nullptr, XpArgs{xp_x, xp_w, have});
+    t.rope = re;
+    fg::KProfScope prof("gemm_nt", 2.0 * M * N * (double)K, 4.0 * ((double)M * K + (double)N * K + (double)M * N));
+    return launch_small<true, true>(t, sp, small_vec(true, true, X, W, K, K, K));
+  }
   {
     fg::Workspace ws;
     int rc = launch_gemm<true, true>("matmulT_fwd_rope", ws, Y, X, W, M, N, K, K, K, 0, nullptr, nullptr, true,
                                      XpArgs{xp_x, xp_w, have});
     if (rc) return rc;
   }
-  const RopeEpi re{cos_tab, sin_tab, (nH + nKV) * dH, dH, pos0, posStride};
   const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
   fg::KProfScope prof("qkv_rope_fwd", 0.0, 8.0 * M * (double)re.cols);
   const bool quad = dH % 4 == 0 && N % 4 == 0 && (uintptr_t)Y % 16 == 0 && (uintptr_t)cos_tab % 16 == 0 &&
