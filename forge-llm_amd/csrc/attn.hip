@@ -44,36 +44,73 @@ constexpr float kLn2 = 0.6931471805599453f;
 
 // ═════════════════════════ scalar kernels (dH <= 128) ═════════════════════════
 // kSMax: the largest head size the instance handles (8, 16, 32, 64 or 128:
-// registers per row and LDS tiles [kSRows][kSMax]).  One wave per 64 rows, so
-// a launch is as long as one wave's chain over its keys.  Head columns past dH
-// are zeros in registers and LDS (their products add +0), so the loops over a
-// head have no branches and read a key's row, which every lane shares, as
-// float4 broadcasts.  B8 T32 nH4/nKV2 dH16, forward / dQ / dK and dV: 119 /
-// 119 / 328 us with a test per column in the 64-wide class, 18 / 14 / 28 us.
-constexpr int kSRows = 64;  // rows per workgroup (one wave)
+// registers per row and LDS tiles [kSRows][kSMax]).  A workgroup has 64 rows,
+// one per lane, and each of its kSWaves waves the keys (queries) of its own
+// residue: what bounds these launches is a wave's chain over its keys, and a
+// small batch leaves the other SIMDs idle.  The waves' sums meet in LDS
+// [wave][column][row], a wave adding every kSWaves-th column in wave order.
+// Head columns past dH are zeros in registers and LDS (their products add +0),
+// so the loops over a head have no branches and read a key's row, which every
+// lane shares, as float4 broadcasts.  Classes above 32 (tensors without the
+// MFMA kernels' alignment) keep one wave: their sums would not fit.
+// B8 T32 nH4/nKV2 dH16, forward / dQ / dK and dV, in the step: one wave 17 /
+// 13 / 27 us and D's launch 6, eight 7 / 10 / 10; B4 T1024 nH16 dH16, whole:
+// eight 166 us forward and 333 backward.
+constexpr int kSRows = 64;
+template <int kSMax>
+constexpr int kSWaves = kSMax <= 32 ? 8 : 1;
+template <int kSMax>
+constexpr int kSThreads = kSRows * kSWaves<kSMax>;
 
 // Fills a [kSRows][kSMax] tile with rows row0 .. of a head's columns (row
 // stride ld), zeros past dH and past `rows`.
 template <int kSMax>
 __device__ __forceinline__ void scalar_tile(float (*__restrict__ tile)[kSMax], const float* __restrict__ src, int ld,
                                             int rows, int dH) {
+  constexpr int kPer = kSMax / kSWaves<kSMax>;
 #pragma unroll 16
-  for (int i = 0; i < kSMax; ++i) {
-    const int e = threadIdx.x + i * kSRows, r = e / kSMax, d = e % kSMax;
+  for (int i = 0; i < kPer; ++i) {
+    const int e = threadIdx.x + i * kSThreads<kSMax>, r = e / kSMax, d = e % kSMax;
     tile[r][d] = r < rows && d < dH ? src[(size_t)r * ld + d] : 0.f;
   }
 }
 
+// The waves' x, summed: wave w returns columns w, w + kSWaves, .. (x[c] of
+// column w + c kSWaves) of its lane's row.
 template <int kSMax>
-__global__ void __launch_bounds__(kSRows) attn_fwd_scalar(float* __restrict__ O, float* __restrict__ lse,
+__device__ __forceinline__ void scalar_sum(float* __restrict__ red, float (&x)[kSMax]) {
+  constexpr int NW = kSWaves<kSMax>;
+  if constexpr (NW > 1) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < kSMax; ++d) red[(wave * kSMax + d) * kSRows + lane] = x[d];
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < kSMax / NW; ++c) {
+      float s = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) s += red[(w * kSMax + wave + c * NW) * kSRows + lane];
+      x[c] = s;
+    }
+  }
+}
+
+template <int kSMax>
+__global__ void __launch_bounds__(kSThreads<kSMax>) attn_fwd_scalar(float* __restrict__ O, float* __restrict__ lse,
                                                           const float* __restrict__ Q, const float* __restrict__ K,
                                                           const float* __restrict__ V, int T, int nH, int nKV,
                                                           int dH, float scale) {
-  __shared__ __attribute__((aligned(16))) float Ks[kSRows][kSMax], Vs[kSRows][kSMax];
+  constexpr int NW = kSWaves<kSMax>;
+  constexpr int kTile = kSRows * kSMax, kRed = NW > 1 ? NW * (kSMax + 2) * kSRows : 0;
+  __shared__ __attribute__((aligned(16))) float lds[kRed > 2 * kTile ? kRed : 2 * kTile];
+  float (*Ks)[kSMax] = reinterpret_cast<float (*)[kSMax]>(lds);
+  float (*Vs)[kSMax] = reinterpret_cast<float (*)[kSMax]>(lds + kTile);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int bh = blockIdx.y, b = bh / nH, h = bh % nH;
   const int group = nH / nKV > 1 ? nH / nKV : 1, kvh = h / group;
   const int qD = nH * dH, kvD = nKV * dH;
-  const int t = blockIdx.x * kSRows + threadIdx.x;
+  const int t = blockIdx.x * kSRows + lane;
   const bool valid = t < T;
   float q[kSMax], o[kSMax];
   const size_t qrow = ((size_t)b * T + (valid ? t : 0)) * qD + (size_t)h * dH;
@@ -92,14 +129,15 @@ __global__ void __launch_bounds__(kSRows) attn_fwd_scalar(float* __restrict__ O,
     __syncthreads();
     if (valid) {
       const int jend = min(t, j0 + kSRows - 1);
-      for (int j = j0; j <= jend; ++j) {
+      for (int j = j0 + wave; j <= jend; j += NW) {
         const int r = j - j0;
         float s = 0.f;
 #pragma unroll
         for (int d = 0; d < kSMax; ++d) s += q[d] * Ks[r][d];
         s *= scale;
         const float mn = fmaxf(m, s);
-        const float alpha = expf(m - mn), p = expf(s - mn);
+        const float mref = mn == -INFINITY ? 0.f : mn;  // no finite score so far
+        const float alpha = expf(m - mref), p = expf(s - mref);
         l = l * alpha + p;
 #pragma unroll
         for (int d = 0; d < kSMax; ++d) o[d] = o[d] * alpha + p * Vs[r][d];
@@ -107,52 +145,76 @@ __global__ void __launch_bounds__(kSRows) attn_fwd_scalar(float* __restrict__ O,
       }
     }
   }
+  if constexpr (NW > 1) {  // each wave's sums at its own maximum, brought to the row's
+    __syncthreads();
+    float* mine = lds + wave * (kSMax + 2) * kSRows + lane;
+#pragma unroll
+    for (int d = 0; d < kSMax; ++d) mine[d * kSRows] = o[d];
+    mine[kSMax * kSRows] = m;
+    mine[(kSMax + 1) * kSRows] = l;
+    __syncthreads();
+    float f[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      f[w] = lds[(w * (kSMax + 2) + kSMax) * kSRows + lane];
+      m = fmaxf(m, f[w]);
+    }
+    l = 0.f;
+    const float mref = m == -INFINITY ? 0.f : m;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      f[w] = expf(f[w] - mref);
+      l += f[w] * lds[(w * (kSMax + 2) + kSMax + 1) * kSRows + lane];
+    }
+#pragma unroll
+    for (int c = 0; c < kSMax / NW; ++c) {
+      float s = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) s += f[w] * lds[(w * (kSMax + 2) + wave + c * NW) * kSRows + lane];
+      o[c] = s;
+    }
+  }
   if (valid) {
     const float il = 1.f / l;
 #pragma unroll
-    for (int d = 0; d < kSMax; ++d)
-      if (d < dH) O[qrow + d] = o[d] * il;
-    lse[(size_t)bh * T + t] = m + logf(l);
+    for (int c = 0; c < kSMax / NW; ++c)
+      if (wave + c * NW < dH) O[qrow + wave + c * NW] = o[c] * il;
+    if (wave == 0) lse[(size_t)bh * T + t] = m + logf(l);
   }
 }
 
-// Dq[(b*nH+h)*T + t] = sum_d dO·O  (shared by both backward families)
-__global__ void __launch_bounds__(256) attn_bwd_pre(float* __restrict__ Dq, const float* __restrict__ dO,
-                                                    const float* __restrict__ O, int B, int T, int nH, int dH) {
-  const int64_t n = (int64_t)B * T * nH;
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-    const int64_t row = e / nH;  // b*T + t
-    const int h = (int)(e - row * nH);
-    const size_t base = (size_t)row * nH * dH + (size_t)h * dH;
-    float acc = 0.f;
-    for (int d = 0; d < dH; ++d) acc += dO[base + d] * O[base + d];
-    const int64_t b = row / T, t = row - b * T;
-    Dq[(b * nH + h) * T + t] = acc;
-  }
-}
-
+// dQ; D = rowsum(dO∘O) of its rows is formed here too and left in Dq for the
+// dK/dV launch.
 template <int kSMax>
-__global__ void __launch_bounds__(kSRows) attn_dq_scalar(float* __restrict__ dQ, int beta,
-                                                         const float* __restrict__ dO, const float* __restrict__ Q,
-                                                         const float* __restrict__ K, const float* __restrict__ V,
-                                                         const float* __restrict__ lse, const float* __restrict__ Dq,
-                                                         int T, int nH, int nKV, int dH, float scale) {
-  __shared__ __attribute__((aligned(16))) float Ks[kSRows][kSMax], Vs[kSRows][kSMax];
+__global__ void __launch_bounds__(kSThreads<kSMax>) attn_dq_scalar(float* __restrict__ dQ, int beta,
+                                                         const float* __restrict__ dO, const float* __restrict__ O,
+                                                         const float* __restrict__ Q, const float* __restrict__ K,
+                                                         const float* __restrict__ V, const float* __restrict__ lse,
+                                                         float* __restrict__ Dq, int T, int nH, int nKV, int dH,
+                                                         float scale) {
+  constexpr int NW = kSWaves<kSMax>;
+  constexpr int kTile = kSRows * kSMax, kRed = NW > 1 ? NW * kTile : 0;
+  __shared__ __attribute__((aligned(16))) float lds[kRed > 2 * kTile ? kRed : 2 * kTile];
+  float (*Ks)[kSMax] = reinterpret_cast<float (*)[kSMax]>(lds);
+  float (*Vs)[kSMax] = reinterpret_cast<float (*)[kSMax]>(lds + kTile);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int bh = blockIdx.y, b = bh / nH, h = bh % nH;
   const int group = nH / nKV > 1 ? nH / nKV : 1, kvh = h / group;
   const int qD = nH * dH, kvD = nKV * dH;
-  const int t = blockIdx.x * kSRows + threadIdx.x;
+  const int t = blockIdx.x * kSRows + lane;
   const bool valid = t < T;
   float q[kSMax], go[kSMax], dq[kSMax];
   const size_t qrow = ((size_t)b * T + (valid ? t : 0)) * qD + (size_t)h * dH;
+  float Dt = 0.f;
 #pragma unroll
   for (int d = 0; d < kSMax; ++d) {
     q[d] = (d < dH) ? Q[qrow + d] : 0.f;
     go[d] = (d < dH) ? dO[qrow + d] : 0.f;
     dq[d] = 0.f;
+    Dt += go[d] * ((d < dH) ? O[qrow + d] : 0.f);
   }
   const float L = valid ? lse[(size_t)bh * T + t] : 0.f;
-  const float Dt = valid ? Dq[(size_t)bh * T + t] : 0.f;
+  if (valid && wave == 0) Dq[(size_t)bh * T + t] = Dt;
   const int last = min(T - 1, blockIdx.x * kSRows + kSRows - 1);
   for (int j0 = 0; j0 <= last; j0 += kSRows) {
     __syncthreads();
@@ -162,7 +224,7 @@ __global__ void __launch_bounds__(kSRows) attn_dq_scalar(float* __restrict__ dQ,
     __syncthreads();
     if (valid) {
       const int jend = min(t, j0 + kSRows - 1);
-      for (int j = j0; j <= jend; ++j) {
+      for (int j = j0 + wave; j <= jend; j += NW) {
         const int r = j - j0;
         float s = 0.f, dp = 0.f;
 #pragma unroll
@@ -177,29 +239,38 @@ __global__ void __launch_bounds__(kSRows) attn_dq_scalar(float* __restrict__ dQ,
       }
     }
   }
+  scalar_sum<kSMax>(lds, dq);
   if (valid) {
 #pragma unroll
-    for (int d = 0; d < kSMax; ++d)
+    for (int c = 0; c < kSMax / NW; ++c) {
+      const int d = wave + c * NW;
       if (d < dH) {
-        const float v = dq[d] * scale;
+        const float v = dq[c] * scale;
         dQ[qrow + d] = beta ? dQ[qrow + d] + v : v;
       }
+    }
   }
 }
 
 template <int kSMax>
-__global__ void __launch_bounds__(kSRows) attn_dkv_scalar(float* __restrict__ dK, int beta_k, float* __restrict__ dV,
-                                                          int beta_v, const float* __restrict__ dO,
+__global__ void __launch_bounds__(kSThreads<kSMax>) attn_dkv_scalar(float* __restrict__ dK, int beta_k,
+                                                          float* __restrict__ dV, int beta_v,
+                                                          const float* __restrict__ dO,
                                                           const float* __restrict__ Q, const float* __restrict__ K,
                                                           const float* __restrict__ V, const float* __restrict__ lse,
                                                           const float* __restrict__ Dq, int T, int nH, int nKV, int dH,
                                                           float scale) {
-  __shared__ __attribute__((aligned(16))) float Qs[kSRows][kSMax], Gs[kSRows][kSMax];
+  constexpr int NW = kSWaves<kSMax>;
+  constexpr int kTile = kSRows * kSMax, kRed = NW > 1 ? NW * kTile : 0;
+  __shared__ __attribute__((aligned(16))) float lds[kRed > 2 * kTile ? kRed : 2 * kTile];
   __shared__ float Ls[kSRows], Ds[kSRows];
+  float (*Qs)[kSMax] = reinterpret_cast<float (*)[kSMax]>(lds);
+  float (*Gs)[kSMax] = reinterpret_cast<float (*)[kSMax]>(lds + kTile);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int bk = blockIdx.y, b = bk / nKV, kvh = bk % nKV;
   const int group = nH / nKV > 1 ? nH / nKV : 1;
   const int qD = nH * dH, kvD = nKV * dH;
-  const int j = blockIdx.x * kSRows + threadIdx.x;
+  const int j = blockIdx.x * kSRows + lane;
   const bool valid = j < T;
   float k[kSMax], v[kSMax], dk[kSMax], dv[kSMax];
   const size_t krow = ((size_t)b * T + (valid ? j : 0)) * kvD + (size_t)kvh * dH;
@@ -220,15 +291,18 @@ __global__ void __launch_bounds__(kSRows) attn_dkv_scalar(float* __restrict__ dK
       const size_t q0 = ((size_t)b * T + t0) * qD + (size_t)h * dH;
       scalar_tile<kSMax>(Qs, Q + q0, qD, T - t0, dH);
       scalar_tile<kSMax>(Gs, dO + q0, qD, T - t0, dH);
-      {
+      if (threadIdx.x < kSRows) {
         const int t = t0 + threadIdx.x;
         Ls[threadIdx.x] = t < T ? lse[bh * T + t] : 0.f;
         Ds[threadIdx.x] = t < T ? Dq[bh * T + t] : 0.f;
       }
       __syncthreads();
       if (valid) {
-        const int tbeg = max(j, t0), tend = min(T - 1, t0 + kSRows - 1);
-        for (int t = tbeg; t <= tend; ++t) {
+        const int tend = min(T - 1, t0 + kSRows - 1);
+        // the wave's first query at or after key j
+        int t = t0 + wave;
+        if (t < j) t += (j - t + NW - 1) / NW * NW;
+        for (; t <= tend; t += NW) {
           const int r = t - t0;
           float s = 0.f, dp = 0.f;
 #pragma unroll
@@ -247,14 +321,18 @@ __global__ void __launch_bounds__(kSRows) attn_dkv_scalar(float* __restrict__ dK
       }
     }
   }
+  scalar_sum<kSMax>(lds, dk);
+  scalar_sum<kSMax>(lds, dv);
   if (valid) {
 #pragma unroll
-    for (int d = 0; d < kSMax; ++d)
+    for (int i = 0; i < kSMax / NW; ++i) {
+      const int d = wave + i * NW;
       if (d < dH) {
-        const float a = dk[d] * scale, c = dv[d];
+        const float a = dk[i] * scale, c = dv[i];
         dK[krow + d] = beta_k ? dK[krow + d] + a : a;
         dV[krow + d] = beta_v ? dV[krow + d] + c : c;
       }
+    }
   }
 }
 
@@ -1478,41 +1556,46 @@ int check_shape(const char* name, int B, int T, int nH, int nKV, int dH) {
 int launch_fwd_scalar(float* O, float* lse, const float* Q, const float* K, const float* V, int B, int T, int nH,
                       int nKV, int dH, float scale) {
   dim3 grid((T + kSRows - 1) / kSRows, B * nH);
-  if (dH <= 8) FG_LAUNCH(attn_fwd_scalar<8>, grid, dim3(kSRows), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
-  else if (dH <= 16) FG_LAUNCH(attn_fwd_scalar<16>, grid, dim3(kSRows), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
-  else if (dH <= 32) FG_LAUNCH(attn_fwd_scalar<32>, grid, dim3(kSRows), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
-  else if (dH <= 64) FG_LAUNCH(attn_fwd_scalar<64>, grid, dim3(kSRows), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
-  else FG_LAUNCH(attn_fwd_scalar<128>, grid, dim3(kSRows), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
+  if (dH <= 8) FG_LAUNCH(attn_fwd_scalar<8>, grid, dim3(kSThreads<8>), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
+  else if (dH <= 16) FG_LAUNCH(attn_fwd_scalar<16>, grid, dim3(kSThreads<16>), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
+  else if (dH <= 32) FG_LAUNCH(attn_fwd_scalar<32>, grid, dim3(kSThreads<32>), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
+  else if (dH <= 64) FG_LAUNCH(attn_fwd_scalar<64>, grid, dim3(kSThreads<64>), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
+  else FG_LAUNCH(attn_fwd_scalar<128>, grid, dim3(kSThreads<128>), 0, O, lse, Q, K, V, T, nH, nKV, dH, scale);
   return FG_OK;
 }
 
 template <int DM>
 int launch_bwd_scalar_t(float* dQ, int beta_q, float* dK, int beta_k, float* dV, int beta_v, const float* dO,
-                        const float* Q, const float* K, const float* V, const float* lse, const float* Dq, int B,
-                        int T, int nH, int nKV, int dH, float scale) {
+                        const float* O, const float* Q, const float* K, const float* V, const float* lse, float* Dq,
+                        int B, int T, int nH, int nKV, int dH, float scale) {
   dim3 gq((T + kSRows - 1) / kSRows, B * nH);
-  FG_LAUNCH(attn_dq_scalar<DM>, gq, dim3(kSRows), 0, dQ, beta_q, dO, Q, K, V, lse, Dq, T, nH, nKV, dH, scale);
+  FG_LAUNCH(attn_dq_scalar<DM>, gq, dim3(kSThreads<DM>), 0, dQ, beta_q, dO, O, Q, K, V, lse, Dq, T, nH, nKV, dH, scale);
   // one workgroup per (sample, kv head): a kv head that no query head maps
   // to (nH < nKV) gets zero gradients, as the reference's loop over h < nH
   // leaves them
   dim3 gk((T + kSRows - 1) / kSRows, B * nKV);
-  FG_LAUNCH(attn_dkv_scalar<DM>, gk, dim3(kSRows), 0, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, Dq, T, nH, nKV, dH,
+  FG_LAUNCH(attn_dkv_scalar<DM>, gk, dim3(kSThreads<DM>), 0, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, Dq, T, nH, nKV, dH,
             scale);
   return FG_OK;
 }
 
 int launch_bwd_scalar(float* dQ, int beta_q, float* dK, int beta_k, float* dV, int beta_v, const float* dO,
-                      const float* Q, const float* K, const float* V, const float* lse, const float* Dq, int B, int T,
-                      int nH, int nKV, int dH, float scale) {
+                      const float* O, const float* Q, const float* K, const float* V, const float* lse, float* Dq,
+                      int B, int T, int nH, int nKV, int dH, float scale) {
   if (dH <= 8)
-    return launch_bwd_scalar_t<8>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, Dq, B, T, nH, nKV, dH, scale);
+    return launch_bwd_scalar_t<8>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, O, Q, K, V, lse, Dq, B, T, nH, nKV, dH,
+                                  scale);
   if (dH <= 16)
-    return launch_bwd_scalar_t<16>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, Dq, B, T, nH, nKV, dH, scale);
+    return launch_bwd_scalar_t<16>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, O, Q, K, V, lse, Dq, B, T, nH, nKV, dH,
+                                  scale);
   if (dH <= 32)
-    return launch_bwd_scalar_t<32>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, Dq, B, T, nH, nKV, dH, scale);
+    return launch_bwd_scalar_t<32>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, O, Q, K, V, lse, Dq, B, T, nH, nKV, dH,
+                                  scale);
   if (dH <= 64)
-    return launch_bwd_scalar_t<64>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, Dq, B, T, nH, nKV, dH, scale);
-  return launch_bwd_scalar_t<128>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, Dq, B, T, nH, nKV, dH, scale);
+    return launch_bwd_scalar_t<64>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, O, Q, K, V, lse, Dq, B, T, nH, nKV, dH,
+                                  scale);
+  return launch_bwd_scalar_t<128>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, O, Q, K, V, lse, Dq, B, T, nH, nKV, dH,
+                                  scale);
 }
 
 // Columns of ngroups groups of g problems (see attn_head_cols).
@@ -1702,13 +1785,7 @@ extern "C" int fg_attn_bwd(float* dQ, int beta_q, float* dK, int beta_k, float* 
     return unpad_heads(dV, dVp, rows, nKV, dH, DP, beta_v);
   }
   if (dH > 128) return bwd_gemm(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, B, T, nH, nKV, dH, scale);
-  {
-    int64_t n = (int64_t)B * T * nH;
-    int64_t blocks = (n + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
-    FG_LAUNCH(attn_bwd_pre, dim3((unsigned)blocks), dim3(256), 0, Dq, dO, O, B, T, nH, dH);
-  }
-  return launch_bwd_scalar(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, Dq, B, T, nH, nKV, dH, scale);
+  return launch_bwd_scalar(dQ, beta_q, dK, beta_k, dV, beta_v, dO, O, Q, K, V, lse, Dq, B, T, nH, nKV, dH, scale);
 }
 
 // Attention of a fused projection qkv[B*T, (nH + 2 nKV) dH] whose q and k

@@ -1,0 +1,64 @@
+"""Attention at head sizes below 32 (a workgroup's waves share a row's keys) at
+the edges of rows, waves and classes, against fp64.
+
+Bound: a score is a sum of dH products, an output of up to T weights, each
+rounding 2^-24 of terms of one size; exp turns a score's absolute error (|s|
+<= 20 here: 20 * 2^-24 = 1.2e-6) into a relative one of its weight.  4e-6 of
+the result's norm holds both.
+"""
+import numpy as np
+import pytest
+
+from util import rel_l2
+
+
+def attention64(q, k, v, go):
+    """o, lse, dq, dk, dv of one sample's causal attention; q [T, nH, dH], k, v [T, nKV, dH]."""
+    T, nH, dH = q.shape
+    nKV = k.shape[1]
+    group = max(1, nH // nKV)
+    o, lse, dq = np.zeros_like(q), np.zeros((nH, T)), np.zeros_like(q)
+    dk, dv = np.zeros_like(k), np.zeros_like(v)
+    future = np.triu(np.ones((T, T), bool), 1)
+    for h in range(nH):
+        z = h // group
+        s = q[:, h] @ k[:, z].T / np.sqrt(dH)
+        s[future] = -np.inf
+        m = s.max(1, keepdims=True)
+        e = np.exp(s - m)
+        lse[h] = m[:, 0] + np.log(e.sum(1))
+        p = e / e.sum(1, keepdims=True)
+        o[:, h] = p @ v[:, z]
+        dv[:, z] += p.T @ go[:, h]
+        dp = go[:, h] @ v[:, z].T
+        ds = p * (dp - (p * dp).sum(1, keepdims=True)) / np.sqrt(dH)
+        dq[:, h] = ds @ k[:, z]
+        dk[:, z] += ds.T @ q[:, h]
+    return o, lse, dq, dk, dv
+
+
+def check(fh, B, T, nH, nKV, dH, beta, tol=4e-6):
+    rs = np.random.default_rng(T * 31 + dH)
+    q, go = (rs.standard_normal((B, T, nH, dH)).astype(np.float32) for _ in range(2))
+    k, v = (rs.standard_normal((B, T, nKV, dH)).astype(np.float32) for _ in range(2))
+    d = [fh.DeviceArray.from_numpy(a) for a in (q, k, v, go)]
+    o, lse = fh.DeviceArray(q.shape), fh.DeviceArray((B, nH, T))
+    fh.call("attn_fwd", o, lse, d[0], d[1], d[2], B, T, nH, nKV, dH)
+    g = [fh.DeviceArray.from_numpy(np.ones(a.shape, np.float32)) for a in (q, k, v)]
+    fh.call("attn_bwd", g[0], beta, g[1], beta, g[2], beta, d[3], d[0], d[1], d[2], o, lse, B, T, nH, nKV, dH)
+    want = [np.stack(a) for a in zip(*[attention64(*(a[b].astype(np.float64) for a in (q, k, v, go))) for b in range(B)])]
+    got = [o.numpy(), lse.numpy()] + [a.numpy() - np.float32(beta) for a in g]
+    for a, w in zip(got, want):
+        if w.any():
+            assert rel_l2(a, w) < tol
+        else:
+            assert not a.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,nH,nKV,dH", [(1, 1, 1, 1, 1), (2, 7, 4, 2, 8), (1, 8, 2, 2, 13), (3, 63, 4, 1, 16),
+                                           (1, 64, 2, 1, 24), (2, 65, 6, 3, 16), (1, 130, 2, 2, 31), (1, 333, 4, 2, 9),
+                                           (1, 70, 2, 4, 16)])
+@pytest.mark.parametrize("beta", [0, 1])
+def test_attention_below_32_vs_fp64(fh, B, T, nH, nKV, dH, beta):
+    check(fh, B, T, nH, nKV, dH, beta)
