@@ -788,20 +788,52 @@ __device__ __forceinline__ float fold_scale(f32x16& s, int e) {
   return 1.f;
 }
 
+// ───────── long chains cut into pieces ─────────
+// A workgroup's 128 rows run through a chain of up to T / 32 blocks, and few
+// heads over a long sequence leave most of the chip idle beside the longest
+// chain.  Row block r of one head (or of one kv head's group member) is then
+// cut into pieces of at most `len` blocks, each an item of its own with a
+// partial result; items of row block r start at first[r], and inside it a
+// head's pieces are neighbours.
+constexpr int kMaxCut = 64;  // row blocks
+struct Cut {
+  int len;  // 0: not cut
+  int first[kMaxCut + 1];
+  __device__ __forceinline__ int block_of(int item) const {
+    int r = 0;
+    while (item >= first[r + 1]) ++r;
+    return r;
+  }
+};
+
 // ───────── forward ─────────
 // Three workgroups per CU at dH <= 64 (168 VGPRs, 52 KB of LDS each): 6% faster
 // than two at B8 T2048 nH16 nKV4, the same at B8 T1024 nH12.
+// With PIECES the key blocks of a query block are cut (rows of `cut` counted
+// from the last query block): a piece leaves its unnormalised O [128][DH], its
+// maxima and its sums [2][128] in part, and attn_fwd_join adds them up.
 template <int DH>
+constexpr int kFwdPart = 128 * (DH + 2);  // floats per piece
+template <int DH, bool PIECES>
 __global__ void __launch_bounds__(kMThreads, DH <= 32 ? 4 : DH <= 64 ? 3 : DH <= 96 ? 2 : 1)
     attn_fwd(float* __restrict__ O, float* __restrict__ lse, const float* __restrict__ Q,
              const float* __restrict__ K, const float* __restrict__ V, int T, int nH, int nKV, float scale,
-             AttnLd L, AttnXp X) {
+             AttnLd L, AttnXp X, Cut cut, float* __restrict__ part) {
   __shared__ __attribute__((aligned(16))) char Ks[2][Tile<DH>::kRow];
   __shared__ __attribute__((aligned(16))) char Vt[2][Tile<DH>::kCol];
   const Exps E = attn_exps<DH>(X, scale, false);
   const int nqb = (T + 127) / 128;
-  const int qblk = nqb - 1 - blockIdx.y;  // longest causal prefix first, across all heads
-  const int bh = blockIdx.x, b = bh / nH, h = bh % nH;
+  // longest causal prefix first, across all heads
+  const int qblk = nqb - 1 - (PIECES ? cut.block_of(blockIdx.x) : (int)blockIdx.y);
+  const int nkb_all = min((T + kBlk - 1) / kBlk, qblk * 4 + 4);
+  int bh = blockIdx.x, kb0 = 0, nkb = nkb_all;
+  if constexpr (PIECES) {
+    const int local = blockIdx.x - cut.first[nqb - 1 - qblk], pieces = (nkb_all + cut.len - 1) / cut.len;
+    bh = local / pieces;
+    kb0 = (local - bh * pieces) * cut.len;
+    nkb = min(nkb_all, kb0 + cut.len);
+  }
+  const int b = bh / nH, h = bh % nH;
   const int group = nH / nKV > 1 ? nH / nKV : 1, kvh = h / group;
   const size_t qD = L.ldq, kvD = L.ldk, oD = L.ldo;
   const int wave = wave_id(), lane = threadIdx.x & 63, hl = lane >> 5;
@@ -820,13 +852,12 @@ __global__ void __launch_bounds__(kMThreads, DH <= 32 ? 4 : DH <= 64 ? 3 : DH <=
   for (int dt = 0; dt < DH / 32; ++dt) oacc[dt] = zero16();
   float m = -INFINITY, l = 0.f;
 
-  const int nkb = min((T + kBlk - 1) / kBlk, qblk * 4 + 4);
   const int mylast = q0w / kBlk;
   BlockLoader<DH> lk;
   ColLoader<DH> lv;
-  lk.load(Kb, kvD, 0, T);
-  lv.load(Vb, kvD, 0, T);
-  for (int kb = 0; kb < nkb; ++kb) {
+  lk.load(Kb, kvD, kb0 * kBlk, T);
+  lv.load(Vb, kvD, kb0 * kBlk, T);
+  for (int kb = kb0; kb < nkb; ++kb) {
     const int buf = kb & 1;
     store_rows2<DH>(Ks[buf], lk, E.k);
     lv.store(Vt[buf], E.v);
@@ -885,11 +916,54 @@ __global__ void __launch_bounds__(kMThreads, DH <= 32 ? 4 : DH <= 64 ? 3 : DH <=
     // after it (back to this buffer) follows the next iteration's barrier,
     // which every wave reaches only once it is done reading this one.
   }
+  if constexpr (PIECES) {
+    float* po = part + (size_t)blockIdx.x * kFwdPart<DH>;
+    const int row = wave * 32 + (lane & 31);
+    store_T<DH>(oacc, po, DH, row, 128, 1.f, 0, -(kPExp + E.v));
+    if (hl == 0) {
+      po[128 * DH + row] = m;
+      po[128 * (DH + 1) + row] = l;
+    }
+    return;
+  }
   const float il = 1.f / l;
   store_T<DH>(oacc, O + (size_t)b * T * oD + (size_t)h * DH, oD, myq, T, il, 0, -(kPExp + E.v));
   if (hl == 0 && myq < T) lse[(size_t)bh * T + myq] = (m + log2f(l)) * kLn2;
 }
 
+
+// The forward's pieces, brought to their common maximum and added in order of
+// their keys; one thread per (row, four columns).
+template <int DH>
+__global__ void __launch_bounds__(256) attn_fwd_join(float* __restrict__ O, float* __restrict__ lse,
+                                                     const float* __restrict__ part, int B, int T, int nH, int ldo,
+                                                     Cut cut) {
+  const int nqb = (T + 127) / 128;
+  const int64_t n = (int64_t)B * nH * T * (DH / 4);
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+    const int c = (int)(e % (DH / 4));
+    const int64_t rq = e / (DH / 4);
+    const int q = (int)(rq % T), bh = (int)(rq / T), b = bh / nH, h = bh - b * nH;
+    const int qblk = q / 128, r = q % 128;
+    const int pieces = (min((T + kBlk - 1) / kBlk, qblk * 4 + 4) + cut.len - 1) / cut.len;
+    const float* p = part + (size_t)(cut.first[nqb - 1 - qblk] + bh * pieces) * kFwdPart<DH>;
+    float m = -INFINITY;
+    for (int i = 0; i < pieces; ++i) m = fmaxf(m, p[(size_t)i * kFwdPart<DH> + 128 * DH + r]);
+    const float mref = m == -INFINITY ? 0.f : m;
+    float l = 0.f;
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < pieces; ++i, p += kFwdPart<DH>) {
+      const float f = fast_exp2(p[128 * DH + r] - mref);
+      const float4 v = *reinterpret_cast<const float4*>(p + r * DH + 4 * c);
+      l += f * p[128 * (DH + 1) + r];
+      o.x += f * v.x; o.y += f * v.y; o.z += f * v.z; o.w += f * v.w;
+    }
+    const float il = 1.f / l;
+    *reinterpret_cast<float4*>(O + ((size_t)b * T + q) * ldo + (size_t)h * DH + 4 * c) =
+        make_float4(o.x * il, o.y * il, o.z * il, o.w * il);
+    if (c == 0) lse[(size_t)bh * T + q] = (m + log2f(l)) * kLn2;
+  }
+}
 
 // ───────── backward: dQ, and D = rowsum(dO∘O) for the dK/dV kernel ─────────
 // Half of D = rowsum(dO∘O) for one query: the d values 16c + 8·half .. +7 of
@@ -1047,7 +1121,7 @@ __device__ __forceinline__ void dkv_body(char* __restrict__ lds, int item, int n
                                          const float* __restrict__ K, const float* __restrict__ V,
                                          const float* __restrict__ lse, const float* __restrict__ Dq, int T, int nH,
                                          int nKV, float scale, const AttnLd& L, float* __restrict__ part,
-                                         float* __restrict__ dS, int npairs, const Exps& E) {
+                                         float* __restrict__ dS, int npairs, const Exps& E, const Cut& cut) {
   char* Qs = lds;
   char* Qc = lds + Tile<DH>::kRow;
   char* Gs = lds + Tile<DH>::kRow + Tile<DH>::kCol;
@@ -1059,8 +1133,25 @@ __device__ __forceinline__ void dkv_body(char* __restrict__ lds, int item, int n
   // member's partial dK/dV goes to part, summed in order by attn_dkv_reduce);
   // items in decreasing causal length (key block 0 sees the most queries).
   const int group = nH / nKV > 1 ? nH / nKV : 1;
-  const int nz = part ? group : 1;
-  const int z = item % nz, bk = (item / nz) % nbk, kblk = item / (nz * nbk);  // nbk = B * nKV
+  // With a cut, also one piece of the query blocks, in z's place gi * pieces + piece.
+  const int nqblk = (T + kBlk - 1) / kBlk;
+  int kblk, bk, z, qb0, len;
+  if (cut.len) {
+    kblk = cut.block_of(item);
+    const int local = item - cut.first[kblk], pieces = (nqblk - kblk * 4 + cut.len - 1) / cut.len;
+    bk = local / (group * pieces);
+    const int zp = local - bk * group * pieces;
+    z = zp / pieces;
+    qb0 = kblk * 4 + (zp - z * pieces) * cut.len;
+    len = min(cut.len, nqblk - qb0);
+  } else {
+    const int nz = part ? group : 1;
+    z = item % nz;
+    bk = (item / nz) % nbk;
+    kblk = item / (nz * nbk);  // nbk = B * nKV
+    qb0 = kblk * 4;            // first query block that can see these keys
+    len = nqblk - qb0;
+  }
   const int b = bk / nKV, kvh = bk % nKV;
   const size_t qD = L.ldq, kvD = L.ldk, oD = L.ldo;
   const int wave = wave_id(), lane = threadIdx.x & 63, hl = lane >> 5;
@@ -1079,17 +1170,14 @@ __device__ __forceinline__ void dkv_body(char* __restrict__ lds, int item, int n
     dk[dt] = zero16();
     dv[dt] = zero16();
   }
-  const int qb0 = kblk * 4;  // first query block that can see these keys
-  const int nqblk = (T + kBlk - 1) / kBlk;
-  const int per_head = nqblk - qb0;
-  const int total = per_head * (part ? 1 : group);
+  const int total = len * (part ? 1 : group);
   const int gbase = part ? z : 0;  // the group member of iteration 0
   // Tiles are loaded, split and stored at the top of each iteration (no
   // register prefetch: it would hold 32 more VGPRs through the MFMA phase
   // and spill (measured: 10% slower at dH = 64, 60% at dH = 128); the other
   // resident workgroup hides the loads).
   for (int it = 0; it < total; ++it) {
-    const int gi = gbase + it / per_head, qb = qb0 + it % per_head;
+    const int gi = gbase + it / len, qb = qb0 + it % len;
     {
       const int h = kvh * group + gi;
       const size_t bh = (size_t)b * nH + h;
@@ -1239,14 +1327,14 @@ __global__ void __launch_bounds__(kMThreads, DH <= 64 ? 2 : 1)
                     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
                     const float* __restrict__ lse, int T, int nH, int nKV, float scale, AttnLd L,
                     float* __restrict__ part, int nbk, int nkv_items, int nq_items, float* __restrict__ dS,
-                    int npairs, AttnXp X) {
+                    int npairs, AttnXp X, Cut cut) {
   __shared__ __attribute__((aligned(16))) char lds[BwdLds<DH>::kMax];
   const Exps E = attn_exps<DH>(X, scale, true);
   const int per_level = nkv_items + nq_items;
   const int y = blockIdx.x / per_level, r = blockIdx.x - y * per_level;
   if (r < nkv_items) {
     dkv_body<DH>(lds, y * nkv_items + r, nbk, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, Dq, T, nH, nKV, scale, L,
-                 part, dS, npairs, E);
+                 part, dS, npairs, E, cut);
   } else {
     const int nqb = (T + 127) / 128;
     dq_body<DH>(lds, nqb - 1 - y, r - nkv_items, false, dQ, beta_q, Dq, dO, O, Q, K, V, lse, T, nH, nKV, scale, L,
@@ -1262,15 +1350,26 @@ __global__ void __launch_bounds__(kMThreads, DH <= 64 ? 2 : 1)
 // fp16 pieces the dK/dV launch formed (the keys of a row are stored in
 // accumulator order), so no split happens here; K^T is staged in LDS (column
 // layout).
-template <int DH>
+// With PIECES its key blocks are cut as attn_fwd's: each piece leaves its sums
+// [128][DH] in part for attn_dq_join.
+template <int DH, bool PIECES>
 __global__ void __launch_bounds__(kMThreads, 2)
     attn_dq_ds(float* __restrict__ dQ, int beta, const float* __restrict__ dS, const float* __restrict__ K, int T,
-               int nH, int nKV, float scale, AttnLd L, int npairs, AttnXp X) {
+               int nH, int nKV, float scale, AttnLd L, int npairs, AttnXp X, Cut cut, float* __restrict__ part) {
   __shared__ __attribute__((aligned(16))) char Kc[2][Tile<DH>::kCol];
   const Exps E = attn_exps<DH>(X, scale, true);
   const int nqb = (T + 127) / 128;
-  const int qblk = nqb - 1 - blockIdx.y;  // longest causal prefix first
-  const int bh = blockIdx.x, b = bh / nH, h = bh % nH;
+  // longest causal prefix first
+  const int qblk = nqb - 1 - (PIECES ? cut.block_of(blockIdx.x) : (int)blockIdx.y);
+  const int nkb_all = min((T + kBlk - 1) / kBlk, qblk * 4 + 4);
+  int bh = blockIdx.x, kb0 = 0, nkb = nkb_all;
+  if constexpr (PIECES) {
+    const int local = blockIdx.x - cut.first[nqb - 1 - qblk], pieces = (nkb_all + cut.len - 1) / cut.len;
+    bh = local / pieces;
+    kb0 = (local - bh * pieces) * cut.len;
+    nkb = min(nkb_all, kb0 + cut.len);
+  }
+  const int b = bh / nH, h = bh % nH;
   const int group = nH / nKV > 1 ? nH / nKV : 1, kvh = h / group;
   const size_t kvD = L.ldk;
   const int wave = wave_id(), lane = threadIdx.x & 63, hl = lane >> 5;
@@ -1284,8 +1383,7 @@ __global__ void __launch_bounds__(kMThreads, 2)
 #pragma unroll
   for (int dt = 0; dt < DH / 32; ++dt) dq[dt] = zero16();
 
-  const int nkb = min((T + kBlk - 1) / kBlk, qblk * 4 + 4);
-  const int mylast = live ? qb : -1;
+  const int mylast = live ? min(qb, nkb - 1) : -1;
   // a block's pieces: hi and lo of chunk c at positions 16c + 8h .. +7 of
   // the query's row (f[c] = hi, f[2 + c] = lo)
   auto load_ds = [&](f16x8 (&f)[4], int kb) {
@@ -1300,10 +1398,10 @@ __global__ void __launch_bounds__(kMThreads, 2)
   // odd ones.
   ColLoader<DH> la, lb;
   f16x8 fa[4], fb[4];
-  la.load(Kb, kvD, 0, T);
-  if (nkb > 1) lb.load(Kb, kvD, kBlk, T);
-  if (mylast >= 0) load_ds(fa, 0);
-  if (mylast >= 1) load_ds(fb, 1);
+  la.load(Kb, kvD, kb0 * kBlk, T);
+  if (nkb > kb0 + 1) lb.load(Kb, kvD, (kb0 + 1) * kBlk, T);
+  if (mylast >= kb0) load_ds(fa, kb0);
+  if (mylast >= kb0 + 1) load_ds(fb, kb0 + 1);
   auto step = [&](ColLoader<DH>& l, f16x8 (&f)[4], int kb) {
     const int buf = kb & 1;
     l.store(Kc[buf], E.k);
@@ -1320,9 +1418,13 @@ __global__ void __launch_bounds__(kMThreads, 2)
     }
     // double-buffered tiles: no trailing barrier (as in attn_fwd)
   };
-  for (int kb = 0; kb < nkb; kb += 2) {
+  for (int kb = kb0; kb < nkb; kb += 2) {
     step(la, fa, kb);
     if (kb + 1 < nkb) step(lb, fb, kb + 1);
+  }
+  if constexpr (PIECES) {
+    store_T<DH>(dq, part + (size_t)blockIdx.x * 128 * DH, DH, wave * 32 + (lane & 31), 128, 1.f, 0, -(E.k + E.ds));
+    return;
   }
   if (L.rc)
     store_T_rope<DH>(dq, dQ + (size_t)b * T * L.ldgq + (size_t)h * DH, L.ldgq, myq, T, scale, L,
@@ -1331,16 +1433,53 @@ __global__ void __launch_bounds__(kMThreads, 2)
     store_T<DH>(dq, dQ + (size_t)b * T * L.ldgq + (size_t)h * DH, L.ldgq, myq, T, scale, beta, -(E.k + E.ds));
 }
 
+// dQ = scale * the sum of its pieces in order of their keys (+beta), its pairs
+// turned back with RoPE tables; one thread per (head, query, d pair).
+template <int DH>
+__global__ void __launch_bounds__(256) attn_dq_join(float* __restrict__ dQ, int beta, const float* __restrict__ part,
+                                                    int B, int T, int nH, float scale, AttnLd L, Cut cut) {
+#pragma clang fp contract(off)
+  const int nqb = (T + 127) / 128;
+  const int64_t n = (int64_t)B * nH * T * (DH / 2);
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+    const int p = (int)(e % (DH / 2));
+    const int64_t rq = e / (DH / 2);
+    const int q = (int)(rq % T), bh = (int)(rq / T), b = bh / nH, h = bh - b * nH;
+    const int qblk = q / 128;
+    const int pieces = (min((T + kBlk - 1) / kBlk, qblk * 4 + 4) + cut.len - 1) / cut.len;
+    const float* src = part + (size_t)(cut.first[nqb - 1 - qblk] + bh * pieces) * 128 * DH + (size_t)(q % 128) * DH + 2 * p;
+    float q0 = 0.f, q1 = 0.f;
+    for (int i = 0; i < pieces; ++i, src += 128 * DH) {
+      const float2 v = *reinterpret_cast<const float2*>(src);
+      q0 += v.x;
+      q1 += v.y;
+    }
+    q0 *= scale;
+    q1 *= scale;
+    const size_t grow = (size_t)b * T + q;
+    float* o = dQ + grow * L.ldgq + (size_t)h * DH + 2 * p;
+    if (L.rc) {
+      const int64_t pos = L.pos0 + (L.posStride > 0 ? (int64_t)grow % L.posStride : (int64_t)grow);
+      const double cc = L.rc[pos * (DH / 2) + p], ss = L.rs[pos * (DH / 2) + p];
+      const double x = q0, y = q1;
+      o[0] = (float)(x * cc + y * ss);
+      o[1] = (float)(-x * ss + y * cc);
+    } else {
+      o[0] = beta ? o[0] + q0 : q0;
+      o[1] = beta ? o[1] + q1 : q1;
+    }
+  }
+}
+
 // dK = scale * sum_z part_z(dK), dV = sum_z part_z(dV) over the group members
-// in order z = 0..group-1 (deterministic), written (+beta) to the outputs;
+// (and their pieces) in order z = 0..group-1 (deterministic), written (+beta) to the outputs;
 // with RoPE tables, dK's pairs turned back as store_T_rope does.  One thread
 // per (kv head, key, d pair).
 template <int DH>
 __global__ void __launch_bounds__(256)
     attn_dkv_reduce(float* __restrict__ dK, int beta_k, float* __restrict__ dV, int beta_v,
-                    const float* __restrict__ part, int B, int T, int nKV, int group, float scale, AttnLd L) {
+                    const float* __restrict__ part, int B, int T, int nKV, int group, float scale, AttnLd L, Cut cut) {
 #pragma clang fp contract(off)
-  const int nkb = (T + 127) / 128;
   const int64_t pairs = (int64_t)B * nKV * T * (DH / 2);
   for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < pairs; e += (int64_t)gridDim.x * 256) {
     const int p = (int)(e % (DH / 2));
@@ -1348,9 +1487,15 @@ __global__ void __launch_bounds__(256)
     const int key = (int)(rk % T), bk = (int)(rk / T);
     const int kblk = key / 128, r = key % 128;
     const int b = bk / nKV, kvh = bk % nKV;
-    const float* src = part + ((size_t)(kblk * (B * nKV) + bk) * group) * 2 * 128 * DH + (size_t)r * DH + 2 * p;
+    size_t item = (size_t)(kblk * (B * nKV) + bk) * group;
+    int nz = group;
+    if (cut.len) {
+      nz = group * (((T + kBlk - 1) / kBlk - kblk * 4 + cut.len - 1) / cut.len);
+      item = cut.first[kblk] + (size_t)bk * nz;
+    }
+    const float* src = part + item * 2 * 128 * DH + (size_t)r * DH + 2 * p;
     float k0 = 0.f, k1 = 0.f, v0 = 0.f, v1 = 0.f;
-    for (int zz = 0; zz < group; ++zz) {
+    for (int zz = 0; zz < nz; ++zz) {
       const float* q = src + (size_t)zz * 2 * 128 * DH;
       k0 += q[0];
       k1 += q[1];
@@ -1374,7 +1519,6 @@ __global__ void __launch_bounds__(256)
     }
     vo[0] = beta_v ? vo[0] + v0 : v0;
     vo[1] = beta_v ? vo[1] + v1 : v1;
-    (void)nkb;
   }
 }
 
@@ -1385,8 +1529,12 @@ __global__ void __launch_bounds__(256)
 // qkv_io already holds them, and dO (when given) into workspace.
 int attn_maxima(fg::Workspace& ws, x3::AttnXp& X, const float* Q, const float* K, const float* V, const float* dO,
                 int B, int T, int nH, int nKV, int DH, const AttnLd& L, float* qkv_io = nullptr,
-                bool have_qkv = false) {
+                bool have_qkv = false, const float* xp_go = nullptr) {
   have_qkv = have_qkv && qkv_io;
+  if (have_qkv && (!dO || xp_go)) {
+    X = x3::AttnXp{qkv_io, qkv_io + FG_XP_PARTS, qkv_io + 2 * FG_XP_PARTS, xp_go};
+    return FG_OK;
+  }
   int rc = ws.get(sizeof(float) * FG_XP_PARTS * 4);
   if (rc) return rc;
   float* xw = static_cast<float*>(ws.ptr);
@@ -1406,15 +1554,84 @@ int attn_maxima(fg::Workspace& ws, x3::AttnXp& X, const float* Q, const float* K
   return FG_OK;
 }
 
+// When and how finely chains of chain(r) blocks, r = 0 .. nr - 1 row blocks of
+// `heads` chains each, are cut.  `slots` workgroups are resident at a time, a
+// block takes `us`, an item `start` blocks more (its fragments, its stores).
+// With fewer items than slots a launch lasts as long as its longest item, with
+// more as the mean load of a slot and some 0.6 of an item of unevenness.  A cut
+// (or what is joined anyway: GQA's group members) adds the partial results'
+// traffic (`bytes` per item, written and read, mostly in the last level cache:
+// 8 TB/s) and the launch that adds them.  Measured, forward / backward us, uncut -> cut:
+//   B1 T4096 nH4/nKV1 dH64    173 / 495 ->  59 / 152
+//   B1 T3000 nH2/nKV2 dH128   222 / 653 ->  51 / 124
+//   B1 T512  nH8/nKV2 dH64     30 /  78 ->  22 /  50
+//   B3 T777  nH12/nKV6 dH80    82 / 238 ->  60 / 181 (padded to 96, one launch for the copies)
+//   B1 T2048 nH16/nKV8 dH128  166 / 490 -> 155 / 412
+// B8 T1024 nH12 dH64 (768 items, longest first) stays whole.
+struct CutCost {
+  double us, start, bytes;
+  bool joined;
+};
+template <class F>
+x3::Cut plan_cut(int nr, int64_t heads, int64_t slots, const CutCost& cost, F chain) {
+  x3::Cut c;
+  c.len = 0;
+  if (nr > x3::kMaxCut) return c;
+  int longest = 0;
+  int64_t total = 0;
+  for (int r = 0; r < nr; ++r) {
+    longest = chain(r) > longest ? chain(r) : longest;
+    total += heads * chain(r);
+  }
+  auto lasts = [&](int64_t items, int len) {
+    const double item = len + cost.start;
+    const double mean = ((double)total + cost.start * (double)items) / (double)slots;
+    return cost.us * (items <= slots ? item : mean + 0.6 * item);
+  };
+  auto join = [&](int64_t items) { return 6.0 + (double)items * 2.0 * cost.bytes / 8e6; };
+  const double whole = (double)longest + cost.start, even = ((double)total + cost.start * (double)(heads * nr)) / (double)slots;
+  double best = 0.95 * (cost.us * (whole > even ? whole : even) + (cost.joined ? join(heads * nr) : 0.0));
+  for (int len = 4; len <= 32 && 2 * len <= longest + 8; ++len) {
+    int64_t items = 0;
+    for (int r = 0; r < nr; ++r) items += heads * ((chain(r) + len - 1) / len);
+    if (items > (1 << 16)) continue;
+    const double us = lasts(items, len) + join(items);
+    if (us < best) {
+      best = us;
+      c.len = len;
+    }
+  }
+  if (!c.len) return c;
+  c.first[0] = 0;
+  for (int r = 0; r < nr; ++r) c.first[r + 1] = c.first[r] + (int)heads * ((chain(r) + c.len - 1) / c.len);
+  return c;
+}
+
 template <int DH>
 int launch_fwd_mfma(float* O, float* lse, const float* Q, const float* K, const float* V, int B, int T, int nH, int nKV,
-                    float scale, const AttnLd& L, float* xp_qkv = nullptr) {
+                    float scale, const AttnLd& L, float* xp_qkv = nullptr, bool have_qkv = false) {
   fg::Workspace wx;
   x3::AttnXp X;
-  int rc = attn_maxima(wx, X, Q, K, V, nullptr, B, T, nH, nKV, DH, L, xp_qkv, false);
+  int rc = attn_maxima(wx, X, Q, K, V, nullptr, B, T, nH, nKV, DH, L, xp_qkv, have_qkv);
   if (rc) return rc;
-  dim3 grid(B * nH, (T + 127) / 128);
-  FG_LAUNCH((x3::attn_fwd<DH>), grid, dim3(kMThreads), 0, O, lse, Q, K, V, T, nH, nKV, scale, L, X);
+  const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
+  const int nqb = (T + 127) / 128, nk32 = (T + kBlk - 1) / kBlk;
+  const x3::Cut cut = plan_cut(nqb, (int64_t)B * nH, (int64_t)cus * (DH <= 32 ? 4 : DH <= 64 ? 3 : DH <= 96 ? 2 : 1),
+                               CutCost{DH <= 32 ? 0.9 : 2.1, 1.0, 512.0 * (DH + 2), false},
+                               [&](int r) { return nk32 < (nqb - r) * 4 ? nk32 : (nqb - r) * 4; });
+  if (cut.len) {
+    fg::Workspace wp;
+    if ((rc = wp.get(sizeof(float) * (size_t)cut.first[nqb] * x3::kFwdPart<DH>))) return rc;
+    FG_LAUNCH((x3::attn_fwd<DH, true>), dim3(cut.first[nqb]), dim3(kMThreads), 0, O, lse, Q, K, V, T, nH, nKV, scale, L,
+              X, cut, (float*)wp.ptr);
+    const int64_t n = (int64_t)B * nH * T * (DH / 4);
+    const int64_t blocks = (n + 255) / 256 < 16LL * cus ? (n + 255) / 256 : 16LL * cus;
+    FG_LAUNCH((x3::attn_fwd_join<DH>), dim3((unsigned)blocks), dim3(256), 0, O, lse, (const float*)wp.ptr, B, T, nH,
+              L.ldo, cut);
+    return FG_OK;
+  }
+  FG_LAUNCH((x3::attn_fwd<DH, false>), dim3(B * nH, nqb), dim3(kMThreads), 0, O, lse, Q, K, V, T, nH, nKV, scale, L, X,
+            cut, nullptr);
   return FG_OK;
 }
 
@@ -1427,7 +1644,8 @@ std::atomic<size_t> g_ds_limit{8ull << 30};
 template <int DH>
 int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, const float* dO, const float* Q,
                     const float* K, const float* V, const float* O, const float* lse, float* Dq, int B, int T, int nH,
-                    int nKV, float scale, const AttnLd& L, const float* xp_qkv = nullptr) {
+                    int nKV, float scale, const AttnLd& L, const float* xp_qkv = nullptr,
+                    const float* xp_go = nullptr) {
   // D = rowsum(dO∘O) first, then the dQ and dK/dV work items in one merged
   // launch; with GQA the dK/dV items are per group member (partials summed in
   // order by attn_dkv_reduce)
@@ -1435,7 +1653,7 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
   fg::Workspace wx;
   x3::AttnXp X;
   {
-    int rc = attn_maxima(wx, X, Q, K, V, dO, B, T, nH, nKV, DH, L, const_cast<float*>(xp_qkv), xp_qkv != nullptr);
+    int rc = attn_maxima(wx, X, Q, K, V, dO, B, T, nH, nKV, DH, L, const_cast<float*>(xp_qkv), xp_qkv != nullptr, xp_go);
     if (rc) return rc;
   }
   {
@@ -1447,13 +1665,6 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
   const int group = nH / nKV > 1 ? nH / nKV : 1;
   const int nkb = (T + 127) / 128;
   const int nbk = B * nKV;
-  fg::Workspace wp;
-  float* part = nullptr;
-  if (group > 1) {
-    int rc = wp.get(sizeof(float) * (size_t)nkb * nbk * group * 2 * 128 * DH);
-    if (rc) return rc;
-    part = (float*)wp.ptr;
-  }
   // dQ from stored dS blocks: the dK/dV items write dS (4 bytes per causal
   // pair), and a second launch forms dQ = dS·K from them
   const int64_t nq32 = (T + kBlk - 1) / kBlk;
@@ -1467,18 +1678,48 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
     if (rc) return rc;
     dS = (float*)wds.ptr;
   }
-  const int nkv_items = nbk * (group > 1 ? group : 1), nq_items = dS ? 0 : B * nH;
-  FG_LAUNCH((x3::attn_bwd_merged<DH>), dim3(nkb * (nkv_items + nq_items)), dim3(kMThreads), 0, dQ, bq, dK, bk, dV,
-            bv, Dq, dO, O, Q, K, V, lse, T, nH, nKV, scale, L, part, nbk, nkv_items, nq_items, dS, npairs, X);
+  // few items and long chains: the query blocks of a key block in pieces
+  x3::Cut cut;
+  cut.len = 0;
   if (dS)
-    FG_LAUNCH((x3::attn_dq_ds<DH>), dim3(B * nH, (T + 127) / 128), dim3(kMThreads), 0, dQ, bq, (const float*)dS, K, T,
-              nH, nKV, scale, L, npairs, X);
-  if (group > 1) {
+    cut = plan_cut(nkb, (int64_t)nbk * group, (int64_t)cus * (DH <= 32 ? 3 : DH <= 64 ? 2 : 1),
+                   CutCost{DH <= 32 ? 3.5 : 5.2, 1.5, 1024.0 * DH, group > 1},
+                   [&](int r) { return (int)nq32 - 4 * r; });
+  fg::Workspace wp;
+  float* part = nullptr;
+  if (group > 1 || cut.len) {
+    const size_t items = cut.len ? (size_t)cut.first[nkb] : (size_t)nkb * nbk * group;
+    int rc = wp.get(sizeof(float) * items * 2 * 128 * DH);
+    if (rc) return rc;
+    part = (float*)wp.ptr;
+  }
+  const int nkv_items = cut.len ? cut.first[nkb] : nbk * (group > 1 ? group : 1), nq_items = dS ? 0 : B * nH;
+  FG_LAUNCH((x3::attn_bwd_merged<DH>), dim3(cut.len ? nkv_items : nkb * (nkv_items + nq_items)), dim3(kMThreads), 0, dQ, bq, dK, bk, dV,
+            bv, Dq, dO, O, Q, K, V, lse, T, nH, nKV, scale, L, part, nbk, nkv_items, nq_items, dS, npairs, X, cut);
+  if (dS) {
+    const x3::Cut qcut = plan_cut(nkb, (int64_t)B * nH, (int64_t)cus * 2, CutCost{0.95, 1.0, 512.0 * DH, false},
+                                  [&](int r) { return nq32 < (nkb - r) * 4 ? (int)nq32 : (nkb - r) * 4; });
+    if (qcut.len) {
+      fg::Workspace wdq;
+      int rc = wdq.get(sizeof(float) * (size_t)qcut.first[nkb] * 128 * DH);
+      if (rc) return rc;
+      FG_LAUNCH((x3::attn_dq_ds<DH, true>), dim3(qcut.first[nkb]), dim3(kMThreads), 0, dQ, bq, (const float*)dS, K, T, nH,
+                nKV, scale, L, npairs, X, qcut, (float*)wdq.ptr);
+      const int64_t n = (int64_t)B * nH * T * (DH / 2);
+      const int64_t blocks = (n + 255) / 256 < 16LL * cus ? (n + 255) / 256 : 16LL * cus;
+      FG_LAUNCH((x3::attn_dq_join<DH>), dim3((unsigned)blocks), dim3(256), 0, dQ, bq, (const float*)wdq.ptr, B, T, nH,
+                scale, L, qcut);
+    } else {
+      FG_LAUNCH((x3::attn_dq_ds<DH, false>), dim3(B * nH, nkb), dim3(kMThreads), 0, dQ, bq, (const float*)dS, K, T, nH,
+                nKV, scale, L, npairs, X, qcut, nullptr);
+    }
+  }
+  if (part) {
     const int64_t pairs = (int64_t)B * nKV * T * (DH / 2);
     int64_t blocks = (pairs + 255) / 256;
     if (blocks > 16LL * cus) blocks = 16LL * cus;
     FG_LAUNCH((x3::attn_dkv_reduce<DH>), dim3((unsigned)blocks), dim3(256), 0, dK, bk, dV, bv, part, B, T, nKV, group,
-              scale, L);
+              scale, L, cut);
   }
   return FG_OK;
 }
@@ -1492,44 +1733,97 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
 // scale stays 1/sqrt(dH).  The copies cost a pass over Q, K, V (and O, dO,
 // the three gradients in the backward); the products cost DP/dH of the
 // unpadded flops.
-// P[rows][nh * DP] = X[rows][nh * dH] (row stride ld), zeros at d >= dH.
-__global__ void __launch_bounds__(256) attn_pad_kernel(float* __restrict__ P, const float* __restrict__ X,
-                                                       int64_t rows, int nh, int dH, int DP, int64_t ld) {
-  const int64_t w = (int64_t)nh * DP, n = rows * w;
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-    const int64_t r = e / w;
-    const int c = (int)(e - r * w), h = c / DP, d = c - h * DP;
-    P[e] = d < dH ? X[r * ld + (int64_t)h * dH + d] : 0.f;
+struct PadJob {
+  const float* X;  // [rows][nh * dH]
+  float* P;        // [rows][nh * DP]
+  float* parts;    // pad: X's FG_XP_PARTS partial maxima, or null
+  int nh, beta;    // unpad: add onto Y
+};
+struct PadTable {
+  PadJob job[5];
+};
+// One launch for all operands (grid: FG_XP_PARTS x jobs): P = X with zeros at
+// d >= dH, and the maxima the MFMA kernels scale by, as absmax_parts gives
+// them, from the same read.  Workgroup w takes rows w, w + 256, .. as one flat
+// range of float4; VEC: X in float4 too (dH % 4 == 0, 16-byte aligned).
+// B3 T777 nH12/nKV6 dH80: a launch per operand and one for the maxima took 23 us
+// of the forward and 49 of the backward, this 8 and 14 (and the three outputs'
+// unpad passes 18, in one launch 11).
+constexpr int kPadThreads = 512;
+template <int DP, bool VEC>
+__global__ void __launch_bounds__(kPadThreads) attn_pad_kernel(PadTable t, int64_t rows, int dH) {
+  const PadJob j = t.job[blockIdx.y];
+  const int w4 = j.nh * (DP / 4);
+  const int nr = rows > blockIdx.x ? (int)((rows - blockIdx.x + FG_XP_PARTS - 1) / FG_XP_PARTS) : 0;
+  float m = 0.f;
+  for (int64_t e = threadIdx.x; e < (int64_t)nr * w4; e += kPadThreads) {
+    const int i = (int)((uint32_t)e / (uint32_t)w4), c4 = (int)e - i * w4;
+    const int64_t r = blockIdx.x + (int64_t)i * FG_XP_PARTS;
+    const int h = c4 / (DP / 4), d = 4 * (c4 - h * (DP / 4));
+    const float* x = j.X + r * (int64_t)j.nh * dH + (int64_t)h * dH + d;
+    float v[4];
+    if constexpr (VEC) {
+      const float4 f = d < dH ? *reinterpret_cast<const float4*>(x) : make_float4(0.f, 0.f, 0.f, 0.f);
+      v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = d + q < dH ? x[q] : 0.f;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float a = fabsf(v[q]);
+      m = fmaxf(m, a < INFINITY ? a : 0.f);  // finite magnitudes
+    }
+    reinterpret_cast<float4*>(j.P)[r * w4 + c4] = make_float4(v[0], v[1], v[2], v[3]);
+  }
+  if (!j.parts) return;
+  __shared__ float wm[kPadThreads / 64];
+  m = fg_wave_max(m);
+  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kPadThreads / 64; ++w) m = fmaxf(m, wm[w]);
+    j.parts[blockIdx.x] = m;
   }
 }
-// Y[rows][nh * dH] (row stride ld) = (beta ? Y + : ) P[rows][nh * DP], d < dH
-// (the add of a beta store, in the same order).
-__global__ void __launch_bounds__(256) attn_unpad_kernel(float* __restrict__ Y, const float* __restrict__ P,
-                                                         int64_t rows, int nh, int dH, int DP, int64_t ld, int beta) {
-  const int64_t w = (int64_t)nh * dH, n = rows * w;
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-    const int64_t r = e / w;
-    const int c = (int)(e - r * w), h = c / dH, d = c - h * dH;
-    const float v = P[r * (int64_t)nh * DP + (int64_t)h * DP + d];
-    float* y = Y + r * ld + c;
-    *y = beta ? *y + v : v;
+// The outputs: X = (beta ? X + : ) P, d < dH (the add of a beta store, in the
+// same order).
+template <int DP>
+__global__ void __launch_bounds__(kPadThreads) attn_unpad_kernel(PadTable t, int64_t rows, int dH) {
+  const PadJob j = t.job[blockIdx.y];
+  const int w = j.nh * dH;
+  float* Y = const_cast<float*>(j.X);
+  const int nr = rows > blockIdx.x ? (int)((rows - blockIdx.x + gridDim.x - 1) / gridDim.x) : 0;
+  for (int64_t e = threadIdx.x; e < (int64_t)nr * w; e += kPadThreads) {
+    const int i = (int)((uint32_t)e / (uint32_t)w), c = (int)e - i * w;
+    const int64_t r = blockIdx.x + (int64_t)i * gridDim.x;
+    const int h = (int)((uint32_t)c / (uint32_t)dH), d = c - h * dH;
+    const float v = j.P[(r * j.nh + h) * DP + d];
+    float* y = Y + r * w + c;
+    *y = j.beta ? *y + v : v;
   }
 }
 bool pad_mfma(int dH) { return dH > 32 && dH < 128 && dH != 64 && dH != 96; }
 int pad_dim(int dH) { return dH <= 64 ? 64 : dH <= 96 ? 96 : 128; }
-int64_t stream_blocks(int64_t n) {
-  const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
-  const int64_t b = (n + 255) / 256;
-  return b < 16LL * cus ? (b > 0 ? b : 1) : 16LL * cus;
-}
-int pad_heads(float* P, const float* X, int64_t rows, int nh, int dH, int DP) {
-  FG_LAUNCH(attn_pad_kernel, dim3((unsigned)stream_blocks(rows * nh * DP)), dim3(256), 0, P, X, rows, nh, dH, DP,
-            (int64_t)nh * dH);
+template <int DP>
+int pad_launch(const PadTable& t, int jobs, int64_t rows, int dH) {
+  bool vec = dH % 4 == 0;
+  for (int i = 0; i < jobs; ++i) vec = vec && (uintptr_t)t.job[i].X % 16 == 0;
+  if (vec)
+    FG_LAUNCH((attn_pad_kernel<DP, true>), dim3(FG_XP_PARTS, jobs), dim3(kPadThreads), 0, t, rows, dH);
+  else
+    FG_LAUNCH((attn_pad_kernel<DP, false>), dim3(FG_XP_PARTS, jobs), dim3(kPadThreads), 0, t, rows, dH);
   return FG_OK;
 }
-int unpad_heads(float* Y, const float* P, int64_t rows, int nh, int dH, int DP, int beta) {
-  FG_LAUNCH(attn_unpad_kernel, dim3((unsigned)stream_blocks(rows * nh * dH)), dim3(256), 0, Y, P, rows, nh, dH, DP,
-            (int64_t)nh * dH, beta);
+int pad_heads(const PadTable& t, int jobs, int64_t rows, int dH, int DP) {
+  return DP == 64 ? pad_launch<64>(t, jobs, rows, dH) : DP == 96 ? pad_launch<96>(t, jobs, rows, dH)
+                                                               : pad_launch<128>(t, jobs, rows, dH);
+}
+int unpad_heads(const PadTable& t, int jobs, int64_t rows, int dH, int DP) {
+  const dim3 grid((unsigned)(rows < 1024 ? rows : 1024), jobs), block(kPadThreads);
+  if (DP == 64) FG_LAUNCH(attn_unpad_kernel<64>, grid, block, 0, t, rows, dH);
+  else if (DP == 96) FG_LAUNCH(attn_unpad_kernel<96>, grid, block, 0, t, rows, dH);
+  else FG_LAUNCH(attn_unpad_kernel<128>, grid, block, 0, t, rows, dH);
   return FG_OK;
 }
 
@@ -1721,15 +2015,17 @@ extern "C" int fg_attn_fwd(float* O, float* lse, const float* Q, const float* K,
     if ((rc = wkv.get(sizeof(float) * (size_t)rows * nKV * DP * 2))) return rc;
     if ((rc = wo.get(sizeof(float) * (size_t)rows * nH * DP))) return rc;
     float *Qp = (float*)wq.ptr, *Kp = (float*)wkv.ptr, *Vp = Kp + (size_t)rows * nKV * DP, *Op = (float*)wo.ptr;
-    if ((rc = pad_heads(Qp, Q, rows, nH, dH, DP))) return rc;
-    if ((rc = pad_heads(Kp, K, rows, nKV, dH, DP))) return rc;
-    if ((rc = pad_heads(Vp, V, rows, nKV, dH, DP))) return rc;
+    fg::Workspace wx;
+    if ((rc = wx.get(sizeof(float) * FG_XP_PARTS * 3))) return rc;
+    float* xp = (float*)wx.ptr;
+    const PadTable in{{{Q, Qp, xp, nH, 0}, {K, Kp, xp + FG_XP_PARTS, nKV, 0}, {V, Vp, xp + 2 * FG_XP_PARTS, nKV, 0}}};
+    if ((rc = pad_heads(in, 3, rows, dH, DP))) return rc;
     const AttnLd L = dense_ld(nH, nKV, DP);
-    rc = DP == 64   ? launch_fwd_mfma<64>(Op, lse, Qp, Kp, Vp, B, T, nH, nKV, scale, L)
-         : DP == 96 ? launch_fwd_mfma<96>(Op, lse, Qp, Kp, Vp, B, T, nH, nKV, scale, L)
-                    : launch_fwd_mfma<128>(Op, lse, Qp, Kp, Vp, B, T, nH, nKV, scale, L);
+    rc = DP == 64   ? launch_fwd_mfma<64>(Op, lse, Qp, Kp, Vp, B, T, nH, nKV, scale, L, xp, true)
+         : DP == 96 ? launch_fwd_mfma<96>(Op, lse, Qp, Kp, Vp, B, T, nH, nKV, scale, L, xp, true)
+                    : launch_fwd_mfma<128>(Op, lse, Qp, Kp, Vp, B, T, nH, nKV, scale, L, xp, true);
     if (rc) return rc;
-    return unpad_heads(O, Op, rows, nH, dH, DP, 0);
+    return unpad_heads(PadTable{{{O, Op, nullptr, nH, 0}}}, 1, rows, dH, DP);
   }
   if (dH > 128) return fwd_gemm(O, lse, Q, K, V, B, T, nH, nKV, dH, scale);
   return launch_fwd_scalar(O, lse, Q, K, V, B, T, nH, nKV, dH, scale);
@@ -1770,19 +2066,22 @@ extern "C" int fg_attn_bwd(float* dQ, int beta_q, float* dK, int beta_k, float* 
     if ((rc = wkv.get(sizeof(float) * nk * 4))) return rc;  // K, V, dK, dV
     float *Qp = (float*)wq.ptr, *Op = Qp + nq, *dOp = Op + nq, *dQp = dOp + nq;
     float *Kp = (float*)wkv.ptr, *Vp = Kp + nk, *dKp = Vp + nk, *dVp = dKp + nk;
-    if ((rc = pad_heads(Qp, Q, rows, nH, dH, DP))) return rc;
-    if ((rc = pad_heads(Op, O, rows, nH, dH, DP))) return rc;
-    if ((rc = pad_heads(dOp, dO, rows, nH, dH, DP))) return rc;
-    if ((rc = pad_heads(Kp, K, rows, nKV, dH, DP))) return rc;
-    if ((rc = pad_heads(Vp, V, rows, nKV, dH, DP))) return rc;
+    fg::Workspace wx;
+    if ((rc = wx.get(sizeof(float) * FG_XP_PARTS * 4))) return rc;
+    float *xp = (float*)wx.ptr, *xg = xp + 3 * FG_XP_PARTS;
+    const PadTable in{{{Q, Qp, xp, nH, 0},
+                       {K, Kp, xp + FG_XP_PARTS, nKV, 0},
+                       {V, Vp, xp + 2 * FG_XP_PARTS, nKV, 0},
+                       {dO, dOp, xg, nH, 0},
+                       {O, Op, nullptr, nH, 0}}};
+    if ((rc = pad_heads(in, 5, rows, dH, DP))) return rc;
     const AttnLd L = dense_ld(nH, nKV, DP);
-    rc = DP == 64   ? launch_bwd_mfma<64>(dQp, 0, dKp, 0, dVp, 0, dOp, Qp, Kp, Vp, Op, lse, Dq, B, T, nH, nKV, scale, L)
-         : DP == 96 ? launch_bwd_mfma<96>(dQp, 0, dKp, 0, dVp, 0, dOp, Qp, Kp, Vp, Op, lse, Dq, B, T, nH, nKV, scale, L)
-                    : launch_bwd_mfma<128>(dQp, 0, dKp, 0, dVp, 0, dOp, Qp, Kp, Vp, Op, lse, Dq, B, T, nH, nKV, scale, L);
+    rc = DP == 64   ? launch_bwd_mfma<64>(dQp, 0, dKp, 0, dVp, 0, dOp, Qp, Kp, Vp, Op, lse, Dq, B, T, nH, nKV, scale, L, xp, xg)
+         : DP == 96 ? launch_bwd_mfma<96>(dQp, 0, dKp, 0, dVp, 0, dOp, Qp, Kp, Vp, Op, lse, Dq, B, T, nH, nKV, scale, L, xp, xg)
+                    : launch_bwd_mfma<128>(dQp, 0, dKp, 0, dVp, 0, dOp, Qp, Kp, Vp, Op, lse, Dq, B, T, nH, nKV, scale, L, xp, xg);
     if (rc) return rc;
-    if ((rc = unpad_heads(dQ, dQp, rows, nH, dH, DP, beta_q))) return rc;
-    if ((rc = unpad_heads(dK, dKp, rows, nKV, dH, DP, beta_k))) return rc;
-    return unpad_heads(dV, dVp, rows, nKV, dH, DP, beta_v);
+    return unpad_heads(PadTable{{{dQ, dQp, nullptr, nH, beta_q}, {dK, dKp, nullptr, nKV, beta_k}, {dV, dVp, nullptr, nKV, beta_v}}},
+                       3, rows, dH, DP);
   }
   if (dH > 128) return bwd_gemm(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, lse, B, T, nH, nKV, dH, scale);
   return launch_bwd_scalar(dQ, beta_q, dK, beta_k, dV, beta_v, dO, O, Q, K, V, lse, Dq, B, T, nH, nKV, dH, scale);

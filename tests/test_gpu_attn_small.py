@@ -62,3 +62,12 @@ def check(fh, B, T, nH, nKV, dH, beta, tol=4e-6):
 @pytest.mark.parametrize("beta", [0, 1])
 def test_attention_below_32_vs_fp64(fh, B, T, nH, nKV, dH, beta):
     check(fh, B, T, nH, nKV, dH, beta)
+
+
+# few heads over long rows: chains in pieces, a last row block of one row, GQA, more and fewer blocks than a piece
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,nH,nKV,dH", [(1, 513, 1, 1, 32), (1, 897, 4, 2, 64), (2, 777, 3, 1, 96), (1, 1100, 2, 2, 128),
+                                           (1, 640, 6, 2, 80), (1, 400, 2, 1, 64)])
+@pytest.mark.parametrize("beta", [0, 1])
+def test_attention_in_pieces_vs_fp64(fh, B, T, nH, nKV, dH, beta):
+    check(fh, B, T, nH, nKV, dH, beta)
