@@ -1640,7 +1640,16 @@ TailPlan plan_tail(int64_t tiles, int K, int cus) {
 //   * K pieces cost their partial sums' traffic at 5 TB/s and a launch;
 //   * the split 8 B per (padded) operand element at 5.2 TB/s and 10 for its
 //     launch and what the GEMM's own first tiles wait for it;
-//   * the kernels that split while staging 2 M N K at 360 TFLOP/s and 10.
+//   * the kernels that split while staging 2 M N K at 360 TFLOP/s and 10; where
+//     some tile or vector of theirs is not whole, and every element is loaded by
+//     itself, at about 110 (forward), 150 (input gradient) or 190 (weight
+//     gradient) and 25, 20 or 10.  The split reads rows of any alignment at the
+//     same speed, so nearly every such shape from 2^29 products on is better
+//     off: forward / input / weight gradient, us, 8192 x 769 -> 2304 260 / 237
+//     / 267 -> 112 / 137 / 147, 1500^3 119 / 97 / 70 -> 65 / 63 / 70, 4096 x 1024
+//     -> 1026 157 / 102 / 87 -> 66 / 53 / 88.  There the sums are cut at least as finely as
+//     the other kernel cuts them (its 16 x 16 x 32 products count as a cut in
+//     two), so that no sum gets longer.
 // E.g. 4096 x 28672 over K = 4096 (2560) goes to pieces at 2160 + 210, 2048 x
 // 4096 over K = 1024 (57) stays: its pieces would take 49 + 10.
 struct PiecePlan {
@@ -1659,18 +1668,24 @@ constexpr int64_t kPiecesMaxBytes = (int64_t)8 << 30;  // both operands' pieces 
 // force_splits: 0 = free choice of the K split.  The same plan serves a GEMM
 // whose pieces' sums stay unreduced (parts_out), so that their sum is what the
 // reduced form stores.
-inline PiecePlan plan_pieces(int M, int N, int K, int cus, int force_splits) {
+// `even`: the other kernels' tiles and vectors are all whole; min_splits: else,
+// the K pieces they would take.
+inline double staged_us(double flop, bool ak, bool bk, bool even) {
+  if (even) return flop / 360e6 + 10.0;
+  return !ak ? flop / 190e6 + 10.0 : bk ? flop / 110e6 + 25.0 : flop / 150e6 + 20.0;
+}
+inline PiecePlan plan_pieces(int M, int N, int K, int cus, bool ak, bool bk, bool even, int force_splits,
+                             int min_splits) {
   PiecePlan best;
-  if (K < 64 || (int64_t)M * N * K < ((int64_t)1 << 31)) return best;
+  if (K < 64 || (int64_t)M * N * K < ((int64_t)1 << (even ? 31 : 29))) return best;
   const int nkc = (K + 15) / 16;
-  const double old_us = 2.0 * M * N * (double)K / 360e6 + 10.0;
-  best.us = old_us;
+  best.us = staged_us(2.0 * M * N * (double)K, ak, bk, even);
   for (const int wm : {2, 4}) {
     const int64_t tm = (M + 64 * wm - 1) / (64 * wm), tn = (N + 255) / 256;
     const double pieces = 64.0 * ((double)nkc * 16) * ((double)tm * wm + (double)tn * 4);  // elements
     if (4.0 * pieces > (double)kPiecesMaxBytes) continue;
     for (int s = 1; s <= 8; ++s) {
-      if (force_splits && s != force_splits) continue;
+      if (force_splits ? s != force_splits : !even && s < min_splits) continue;
       if (s > 1 && nkc / s < 8) continue;
       const int per = (nkc + s - 1) / s;
       if ((nkc + per - 1) / per != s) continue;
@@ -1769,6 +1784,20 @@ inline int launch_pieces(const PiecePlan& pl, bool ak, bool bk, float* C, const 
   return FG_OK;
 }
 
+// Fast path of the kernels that split while staging: every tile full and every
+// vector access aligned.
+inline bool plan_even(const GemmPlan& pl, int M, int N, int K, int lda, int ldb, const float* A, const float* B,
+                      const float* C, const float* resid) {
+  return (M % pl.tm == 0) && (N % pl.tn == 0) && (K % BK == 0) && (lda % 4 == 0) && (ldb % 4 == 0) &&
+         ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && ((uintptr_t)C % 16 == 0) &&
+         (resid == nullptr || (uintptr_t)resid % 16 == 0);
+}
+// The K pieces that plan_pieces has to keep: an input gradient's in two
+// (fg_matmulT_bwd_x_halves), and all of them on whole tiles.
+inline int piece_force(bool ak, bool bk, const GemmPlan& pl, bool even) {
+  return ak && !bk && (even || pl.splits == 2) ? pl.splits : 0;
+}
+
 // Queues C (+)= A·B on fg::stream(); split-K partials live in `ws`, which
 // the caller keeps until the kernels are ordered before any later reuse.
 // parts_out: the plan must split K in two; the two pieces' M x N partial sums
@@ -1820,18 +1849,15 @@ int launch_gemm(const char* name, fg::Workspace& ws, float* C, const float* A, c
     }
     return FG_OK;
   }
-  // input gradients keep the number of K pieces fg_matmulT_bwd_x_pieces names
-  const PiecePlan pp = plan_pieces(M, N, K, cus, AK && !BKc ? pl.splits : 0);
+  const bool even = plan_even(pl, M, N, K, lda, ldb, A, B, C, resid);
+  // an input gradient that can be left in two pieces keeps them
+  const PiecePlan pp = plan_pieces(M, N, K, cus, AK, BKc, even, piece_force(AK, BKc, pl, even), pl.pq ? 2 : pl.splits);
   if (pp.wm) {
     bool got = false;
     int rc = launch_pieces(pp, AK, BKc, C, A, B, M, N, K, lda, ldb, beta, resid, parts_out, scoped, xp, SwigluOut(), got);
     if (rc || got) return rc;
   }
   const int tiles = ((M + pl.tm - 1) / pl.tm) * ((N + pl.tn - 1) / pl.tn);
-  // Fast path: every tile full and every vector access aligned.
-  const bool even = (M % pl.tm == 0) && (N % pl.tn == 0) && (K % BK == 0) && (lda % 4 == 0) && (ldb % 4 == 0) &&
-                    ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && ((uintptr_t)C % 16 == 0) &&
-                    (resid == nullptr || (uintptr_t)resid % 16 == 0);
   float* partial = parts_out;
   if (pl.splits > 1 && !partial) {
     int rc = ws.get(sizeof(float) * (size_t)pl.splits * M * N);
@@ -2011,14 +2037,15 @@ extern "C" int fg_matmulT_fwd_swiglu_p(float* O, float* GU, const float* X, cons
   }
   // on pieces, where plan_pieces' choice for the plain forward is one that
   // the epilogue fits (the same products in the same order as that forward)
-  const PiecePlan pp = plan_pieces(M, 2 * H, K, cus, 0);
+  const GemmPlan pl = plan_gemm(true, true, M, 2 * H, K, cus);
+  const PiecePlan pp = plan_pieces(M, 2 * H, K, cus, true, true, plan_even(pl, M, 2 * H, K, K, K, X, Wgu, GU, nullptr), 0,
+                                   pl.pq ? 2 : pl.splits);
   if (pp.wm && pp.splits == 1 && M % (64 * pp.wm) == 0 && H % 128 == 0) {
     bool got = false;
     int rc = launch_pieces(pp, true, true, GU, X, Wgu, M, 2 * H, K, K, K, 0, nullptr, nullptr, true,
                            XpArgs{xp_x, xp_w, have}, SwigluOut{O, H}, got);
     if (rc || got) return rc;
   }
-  const GemmPlan pl = plan_gemm(true, true, M, 2 * H, K, cus);
   const bool fused = !pp.wm && pl.w && pl.tn == 256 && pl.splits == 1 && M % 256 == 0 && H % 128 == 0 && K % BK == 0 &&
                      (int64_t)(M / 256) * (2 * H / 256) % cus == 0 && (uintptr_t)X % 16 == 0 &&
                      (uintptr_t)Wgu % 16 == 0 && (uintptr_t)GU % 16 == 0;
@@ -2116,9 +2143,13 @@ int grouped_pieces(const fg_wgrad_job* jobs, int count, int cus, bool& done) {
       bytes += add;
     }
     int wm = 0, splits = 1;
-    double best = 0.0, old_us = 10.0;
-    for (int j = b; j < e; ++j) old_us += 2.0 * jobs[j].M * jobs[j].K * (double)jobs[j].N / 360e6;
-    best = old_us;
+    double best = 10.0;  // the kernels that split while staging (see plan_pieces)
+    for (int j = b; j < e; ++j) {
+      const fg_wgrad_job& jb = jobs[j];
+      const bool even = jb.N % 256 == 0 && jb.K % 256 == 0 && jb.M % BK == 0 && (uintptr_t)jb.gY % 16 == 0 &&
+                        (uintptr_t)jb.X % 16 == 0 && (uintptr_t)jb.gW % 16 == 0;
+      best += staged_us(2.0 * jb.M * jb.K * (double)jb.N, false, false, even) - staged_us(0.0, false, false, even);
+    }
     for (const int cwm : {2, 4}) {
       double tiles = 0.0, chunks = 0.0, pieces = 0.0, outs = 0.0;
       int kmin = INT32_MAX;

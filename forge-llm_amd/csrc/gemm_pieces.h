@@ -72,16 +72,13 @@ __device__ __forceinline__ void split_unit(const SplitJob& j, int u, int e) {
   int r = rb * 32 + (lane & 31);
   const bool in = r < j.rows;
   if (j.swh > 0 && in) r = swiglu_row(r, j.swh);
-  const bool vec = j.kc && (j.ld & 3) == 0 && ((uintptr_t)j.src & 15) == 0;
   float f[kSplitNC][8];
 #pragma unroll
   for (int c = 0; c < kSplitNC; ++c) {
     const int k = (c0 + c) * 16 + (lane >> 5) * 8;
-    if (vec && in && k + 8 <= j.k) {
-      const float4 p = *reinterpret_cast<const float4*>(j.src + (size_t)r * j.ld + k);
-      const float4 q = *reinterpret_cast<const float4*>(j.src + (size_t)r * j.ld + k + 4);
-      f[c][0] = p.x; f[c][1] = p.y; f[c][2] = p.z; f[c][3] = p.w;
-      f[c][4] = q.x; f[c][5] = q.y; f[c][6] = q.z; f[c][7] = q.w;
+    if (j.kc && in && k + 8 <= j.k) {  // 16-byte loads at any element (rows of odd length)
+      __builtin_memcpy(f[c], j.src + (size_t)r * j.ld + k, 16);
+      __builtin_memcpy(f[c] + 4, j.src + (size_t)r * j.ld + k + 4, 16);
     } else if (j.kc) {
 #pragma unroll
       for (int q = 0; q < 8; ++q) f[c][q] = in && k + q < j.k ? j.src[(size_t)r * j.ld + k + q] : 0.f;

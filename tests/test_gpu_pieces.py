@@ -91,3 +91,22 @@ def test_swiglu_epilogue_on_pieces_is_the_separate_pass(fh, M, K, H):
     fh.call("swiglu_gu_fwd", o2, gu2, M, H)
     np.testing.assert_array_equal(gu.numpy(), gu2.numpy())
     np.testing.assert_array_equal(o.numpy(), o2.numpy())
+
+
+# shapes of a middle size take this form where their tiles or vectors are not
+# whole: odd rows of each operand, and K pieces in all three layouts
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(777, 1555, 666), (1501, 1499, 1502), (2048, 1026, 1537), (4095, 515, 771)])
+def test_uneven_shapes_vs_fp64(fh, M, K, N):
+    test_matmulT_on_pieces_vs_fp64(fh, M, K, N)
+
+
+# operands that start between 16-byte boundaries
+@pytest.mark.gpu
+def test_unaligned_operands_on_pieces(fh):
+    M, K, N = 1536, 1024, 1536
+    rs = np.random.default_rng(3)
+    X, W = rs.standard_normal(M * K + 1, dtype=np.float32), rs.standard_normal(N * K + 3, dtype=np.float32)
+    dX, dW, Y = up(fh, X), up(fh, W), fh.DeviceArray((M, N))
+    fh.call("matmulT_fwd", Y, dX.ptr + 4, dW.ptr + 12, M, K, N)
+    _check(Y.numpy(), X[1:].reshape(M, K).astype(np.float64) @ W[3:].reshape(N, K).astype(np.float64).T, K)
