@@ -500,7 +500,8 @@ int launch_qmatvec(OutT* y, const uint8_t* W, const float* x, int N, int K) {
     // x in LDS beside the kernel's own arrays (64 KB), whole units, aligned
     // blocks; Q8_0 rows of fewer units than lanes stay with the eight lanes per
     // block below (31586 x 256: 6.7 against 7.0 us)
-    if (K <= 16000 && K % unit_elems(QT) == 0 && (uintptr_t)W % 16 == 0 && (QT != kQ8_0 || K >= 1024)) {
+    if (K <= 16000 && K % unit_elems(QT) == 0 && (uintptr_t)W % 16 == 0 && (QT != kQ8_0 || K >= 1024) &&
+        units_pay(QT, K)) {
       const int P = unit_parts(K / unit_elems(QT)), slots = kUnitWaves / P;
       // four rows per wave group, or one where that would leave CUs idle
       const bool wide = (int64_t)((N + 3) / 4) * P >= 8LL * cus;
