@@ -1619,9 +1619,8 @@ int launch_fwd_mfma(float* O, float* lse, const float* Q, const float* K, const 
   const x3::Cut cut = plan_cut(nqb, (int64_t)B * nH, (int64_t)cus * (DH <= 32 ? 4 : DH <= 64 ? 3 : DH <= 96 ? 2 : 1),
                                CutCost{DH <= 32 ? 0.9 : 2.1, 1.0, 512.0 * (DH + 2), false},
                                [&](int r) { return nk32 < (nqb - r) * 4 ? nk32 : (nqb - r) * 4; });
-  if (cut.len) {
-    fg::Workspace wp;
-    if ((rc = wp.get(sizeof(float) * (size_t)cut.first[nqb] * x3::kFwdPart<DH>))) return rc;
+  fg::Workspace wp;  // whole chains where it cannot be had
+  if (cut.len && wp.get(sizeof(float) * (size_t)cut.first[nqb] * x3::kFwdPart<DH>) == FG_OK) {
     FG_LAUNCH((x3::attn_fwd<DH, true>), dim3(cut.first[nqb]), dim3(kMThreads), 0, O, lse, Q, K, V, T, nH, nKV, scale, L,
               X, cut, (float*)wp.ptr);
     const int64_t n = (int64_t)B * nH * T * (DH / 4);
@@ -1685,11 +1684,16 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
     cut = plan_cut(nkb, (int64_t)nbk * group, (int64_t)cus * (DH <= 32 ? 3 : DH <= 64 ? 2 : 1),
                    CutCost{DH <= 32 ? 3.5 : 5.2, 1.5, 1024.0 * DH, group > 1},
                    [&](int r) { return (int)nq32 - 4 * r; });
-  fg::Workspace wp;
+  fg::Workspace wp, wc;
   float* part = nullptr;
-  if (group > 1 || cut.len) {
-    const size_t items = cut.len ? (size_t)cut.first[nkb] : (size_t)nkb * nbk * group;
-    int rc = wp.get(sizeof(float) * items * 2 * 128 * DH);
+  if (cut.len) {
+    if (wc.get(sizeof(float) * (size_t)cut.first[nkb] * 2 * 128 * DH) == FG_OK)
+      part = (float*)wc.ptr;
+    else
+      cut.len = 0;  // whole chains where the pieces' sums cannot be had
+  }
+  if (group > 1 && !cut.len) {
+    int rc = wp.get(sizeof(float) * (size_t)nkb * nbk * group * 2 * 128 * DH);
     if (rc) return rc;
     part = (float*)wp.ptr;
   }
@@ -1699,10 +1703,8 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
   if (dS) {
     const x3::Cut qcut = plan_cut(nkb, (int64_t)B * nH, (int64_t)cus * 2, CutCost{0.95, 1.0, 512.0 * DH, false},
                                   [&](int r) { return nq32 < (nkb - r) * 4 ? (int)nq32 : (nkb - r) * 4; });
-    if (qcut.len) {
-      fg::Workspace wdq;
-      int rc = wdq.get(sizeof(float) * (size_t)qcut.first[nkb] * 128 * DH);
-      if (rc) return rc;
+    fg::Workspace wdq;
+    if (qcut.len && wdq.get(sizeof(float) * (size_t)qcut.first[nkb] * 128 * DH) == FG_OK) {
       FG_LAUNCH((x3::attn_dq_ds<DH, true>), dim3(qcut.first[nkb]), dim3(kMThreads), 0, dQ, bq, (const float*)dS, K, T, nH,
                 nKV, scale, L, npairs, X, qcut, (float*)wdq.ptr);
       const int64_t n = (int64_t)B * nH * T * (DH / 2);
