@@ -27,6 +27,9 @@
 //   * gemm_w_kernel: the ping-pong pipeline on 256x256 tiles, 64x128 wave
 //     tiles, k-step 16 (outputs of at least two full rounds of such tiles).
 // plan_gemm picks the shape and the K split per call.
+//   * gemm_pieces.h: operands split ahead and copied to LDS as pieces (large
+//     shapes, and uneven ones from 2^29 products on; plan_pieces);
+//   * gemm_small.h: small shapes on the fp32 MFMA, unsplit (plan_small).
 //
 // Launch shape: 1-D grid of tiles remapped so each of the 8 XCDs gets a
 // contiguous range, then grouped 8 tile-rows at a time for L2 reuse.  When the
