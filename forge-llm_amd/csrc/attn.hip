@@ -1821,11 +1821,23 @@ int pad_heads(const PadTable& t, int jobs, int64_t rows, int dH, int DP) {
   return DP == 64 ? pad_launch<64>(t, jobs, rows, dH) : DP == 96 ? pad_launch<96>(t, jobs, rows, dH)
                                                                : pad_launch<128>(t, jobs, rows, dH);
 }
+bool overlap(const float* a, int64_t na, const float* b, int64_t nb) { return a < b + nb && b < a + na; }
+// Outputs that share memory (the gradients of a tensor that is query, key and
+// value at once) are written in the order of the jobs, a launch for each.
 int unpad_heads(const PadTable& t, int jobs, int64_t rows, int dH, int DP) {
-  const dim3 grid((unsigned)(rows < 1024 ? rows : 1024), jobs), block(kPadThreads);
-  if (DP == 64) FG_LAUNCH(attn_unpad_kernel<64>, grid, block, 0, t, rows, dH);
-  else if (DP == 96) FG_LAUNCH(attn_unpad_kernel<96>, grid, block, 0, t, rows, dH);
-  else FG_LAUNCH(attn_unpad_kernel<128>, grid, block, 0, t, rows, dH);
+  bool shared = false;
+  for (int i = 0; i < jobs; ++i)
+    for (int j = 0; j < i; ++j)
+      shared |= overlap(t.job[i].X, rows * t.job[i].nh * dH, t.job[j].X, rows * t.job[j].nh * dH);
+  const int per = shared ? 1 : jobs;
+  for (int i = 0; i < jobs; i += per) {
+    PadTable u = t;
+    if (shared) u.job[0] = t.job[i];
+    const dim3 grid((unsigned)(rows < 1024 ? rows : 1024), per), block(kPadThreads);
+    if (DP == 64) FG_LAUNCH(attn_unpad_kernel<64>, grid, block, 0, u, rows, dH);
+    else if (DP == 96) FG_LAUNCH(attn_unpad_kernel<96>, grid, block, 0, u, rows, dH);
+    else FG_LAUNCH(attn_unpad_kernel<128>, grid, block, 0, u, rows, dH);
+  }
   return FG_OK;
 }
 
@@ -2040,6 +2052,22 @@ extern "C" int fg_attn_bwd(float* dQ, int beta_q, float* dK, int beta_k, float* 
   int rc = check_shape("fg_attn_bwd", B, T, nH, nKV, dH);
   if (rc) return rc;
   FG_ARG_CHECK(dQ && dK && dV && dO && Q && K && V && O && lse, "fg_attn_bwd: null pointer");
+  const bool padded = pad_mfma(dH) && nH >= nKV;
+  const int64_t nq = (int64_t)B * T * nH * dH, nk = (int64_t)B * T * nKV * dH;
+  if (dH <= 128 && !padded && (overlap(dQ, nq, dK, nk) || overlap(dQ, nq, dV, nk) || overlap(dK, nk, dV, nk))) {
+    // Gradients that share memory (the other paths add in order by
+    // themselves): the kernels below write them from one launch, or dQ after
+    // dK, so each goes to a buffer of its own and is added from there, in the
+    // order dQ, dK, dV.
+    fg::Workspace wg;
+    if ((rc = wg.get(sizeof(float) * (size_t)(nq + 2 * nk + 8)))) return rc;
+    float* gq = (float*)wg.ptr;
+    float* gk = gq + (nq + 3) / 4 * 4;
+    float* gv = gk + (nk + 3) / 4 * 4;
+    if ((rc = fg_attn_bwd(gq, 0, gk, 0, gv, 0, dO, Q, K, V, O, lse, B, T, nH, nKV, dH))) return rc;
+    if ((rc = fg_accum(dQ, gq, nq, beta_q)) || (rc = fg_accum(dK, gk, nk, beta_k))) return rc;
+    return fg_accum(dV, gv, nk, beta_v);
+  }
   const double pairs = (double)T * (T + 1) / 2.0;
   fg::KProfScope prof("attn_bwd", 8.0 * dH * pairs * B * nH,
                       4.0 * B * T * ((double)nH * dH * 4 + (double)nKV * dH * 4 + 2.0 * nH));
@@ -2059,15 +2087,15 @@ extern "C" int fg_attn_bwd(float* dQ, int beta_q, float* dK, int beta_k, float* 
     if (dH == 96) return launch_bwd_mfma<96>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, O, lse, Dq, B, T, nH, nKV, scale, L);
     return launch_bwd_mfma<128>(dQ, beta_q, dK, beta_k, dV, beta_v, dO, Q, K, V, O, lse, Dq, B, T, nH, nKV, scale, L);
   }
-  if (pad_mfma(dH) && nH >= nKV) {  // heads padded with zeros to the next MFMA size
+  if (padded) {  // heads padded with zeros to the next MFMA size
     const int DP = pad_dim(dH);
     const int64_t rows = (int64_t)B * T;
-    const size_t nq = (size_t)rows * nH * DP, nk = (size_t)rows * nKV * DP;
+    const size_t pq = (size_t)rows * nH * DP, pk = (size_t)rows * nKV * DP;
     fg::Workspace wq, wkv;
-    if ((rc = wq.get(sizeof(float) * nq * 4))) return rc;   // Q, O, dO, dQ
-    if ((rc = wkv.get(sizeof(float) * nk * 4))) return rc;  // K, V, dK, dV
-    float *Qp = (float*)wq.ptr, *Op = Qp + nq, *dOp = Op + nq, *dQp = dOp + nq;
-    float *Kp = (float*)wkv.ptr, *Vp = Kp + nk, *dKp = Vp + nk, *dVp = dKp + nk;
+    if ((rc = wq.get(sizeof(float) * pq * 4))) return rc;   // Q, O, dO, dQ
+    if ((rc = wkv.get(sizeof(float) * pk * 4))) return rc;  // K, V, dK, dV
+    float *Qp = (float*)wq.ptr, *Op = Qp + pq, *dOp = Op + pq, *dQp = dOp + pq;
+    float *Kp = (float*)wkv.ptr, *Vp = Kp + pk, *dKp = Vp + pk, *dVp = dKp + pk;
     fg::Workspace wx;
     if ((rc = wx.get(sizeof(float) * FG_XP_PARTS * 4))) return rc;
     float *xp = (float*)wx.ptr, *xg = xp + 3 * FG_XP_PARTS;

@@ -5,6 +5,9 @@ Bound: a score is a sum of dH products, an output of up to T weights, each
 rounding 2^-24 of terms of one size; exp turns a score's absolute error (|s|
 <= 20 here: 20 * 2^-24 = 1.2e-6) into a relative one of its weight.  4e-6 of
 the result's norm holds both.
+
+Gradients that share a buffer (attention of a tensor with itself) are added in
+the order dQ, dK, dV: one fp32 addition each after those of the separate run.
 """
 import numpy as np
 import pytest
@@ -71,3 +74,32 @@ def test_attention_below_32_vs_fp64(fh, B, T, nH, nKV, dH, beta):
 @pytest.mark.parametrize("beta", [0, 1])
 def test_attention_in_pieces_vs_fp64(fh, B, T, nH, nKV, dH, beta):
     check(fh, B, T, nH, nKV, dH, beta)
+
+
+# padded, scalar, MFMA (whole and in pieces) and GEMM heads
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,dH", [(130, 80), (700, 48), (70, 16), (65, 64), (600, 64), (40, 32), (33, 160)])
+@pytest.mark.parametrize("shared", ["kv", "qkv", "qk"])
+def test_gradients_that_share_a_buffer(fh, T, dH, shared):
+    B, nH = 2, 3
+    rs = np.random.default_rng(T + dH)
+    q, k, v, go = (fh.DeviceArray.from_numpy(rs.standard_normal((B, T, nH, dH)).astype(np.float32)) for _ in range(4))
+    shape = (B, T, nH, dH)
+    o, lse = fh.DeviceArray(shape), fh.DeviceArray((B, nH, T))
+    fh.call("attn_fwd", o, lse, q, k, v, B, T, nH, nH, dH)
+    own = [fh.DeviceArray(shape) for _ in range(3)]
+    fh.call("attn_bwd", own[0], 0, own[1], 0, own[2], 0, go, q, k, v, o, lse, B, T, nH, nH, dH)
+    for first in (0, 1):  # the shared gradient fresh, or there already
+        g = [fh.DeviceArray.from_numpy(np.ones(shape, np.float32)) for _ in range(3)]
+        want = [np.full(shape, float(first)) for _ in range(3)]
+        use = {"q": 0, "k": 1, "v": 2}
+        at, beta, seen = [0, 1, 2], [first] * 3, False
+        for c in shared:
+            at[use[c]] = use[shared[0]]
+            beta[use[c]] = 1 if seen else first
+            seen = True
+        fh.call("attn_bwd", g[at[0]], beta[0], g[at[1]], beta[1], g[at[2]], beta[2], go, q, k, v, o, lse, B, T, nH, nH, dH)
+        for i in range(3):
+            want[at[i]] += own[i].numpy().astype(np.float64)
+        for i in set(at):
+            assert rel_l2(g[i].numpy(), want[i]) < 3 * 2.0 ** -24
