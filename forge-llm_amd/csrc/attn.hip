@@ -1555,25 +1555,41 @@ int attn_maxima(fg::Workspace& ws, x3::AttnXp& X, const float* Q, const float* K
 }
 
 // When and how finely chains of chain(r) blocks, r = 0 .. nr - 1 row blocks of
-// `heads` chains each, are cut.  `slots` workgroups are resident at a time, a
-// block takes `us`, an item `start` blocks more (its fragments, its stores).
-// With fewer items than slots a launch lasts as long as its longest item, with
-// more as the mean load of a slot and some 0.6 of an item of unevenness.  A cut
-// (or what is joined anyway: GQA's group members) adds the partial results'
-// traffic (`bytes` per item, written and read, mostly in the last level cache:
-// 8 TB/s) and the launch that adds them.  Measured, forward / backward us, uncut -> cut:
+// `heads` chains each, are cut.
+//
+// How finely: `slots` workgroups are resident at a time, a block takes `us`, an
+// item `start` blocks more (its fragments, its stores).  With fewer items than
+// slots a launch lasts as long as its longest item, with more as the mean load
+// of a slot and some 0.6 of an item of unevenness; each item's partial results
+// (`bytes`, mostly in the last level cache) are written and read.
+//
+// Whether: an item alone on its CU takes `lone` us a block, CUs that are all
+// busy get through one block every `busy` us whatever the number of resident
+// items, an item costs `extra` blocks more.  A launch takes the longer of the longest item and the load (their
+// 4-norm: a smooth maximum); a cut (or what is joined anyway: GQA's group
+// members) adds `join` us for its launch and the partial results at `gbs`.  The
+// constants are least-squares fits per head size to the differences of whole and
+// cut calls over T = 200 .. 8192 and 1 .. 128 heads; of 2452 calls three take
+// longer than whole chains would, 6 - 7% (T512 nH64/nKV16 dH96 and 128, T200 nH64
+// dH32, backward).
+// Forward / backward us, whole -> cut:
 //   B1 T4096 nH4/nKV1 dH64    173 / 495 ->  59 / 152
 //   B1 T3000 nH2/nKV2 dH128   222 / 653 ->  51 / 124
 //   B1 T512  nH8/nKV2 dH64     30 /  78 ->  22 /  50
 //   B3 T777  nH12/nKV6 dH80    82 / 238 ->  60 / 181 (padded to 96, one launch for the copies)
-//   B1 T2048 nH16/nKV8 dH128  166 / 490 -> 155 / 412
-// B8 T1024 nH12 dH64 (768 items, longest first) stays whole.
+// and left whole, where pieces took longer:
+//   forward  T512 nH128 dH64 44 against 55, T2048 nH48 dH64 130 against 152
+//   backward T1400 nH48 dH64 244 against 283, T4096 nH32 dH32 707 against 770
+// Beyond kMaxCut row blocks (T > 8192) chains stay whole: the size of the
+// table, not a measurement.
 struct CutCost {
+  int64_t slots;
   double us, start, bytes;
+  double lone, busy, extra, join, gbs;
   bool joined;
 };
 template <class F>
-x3::Cut plan_cut(int nr, int64_t heads, int64_t slots, const CutCost& cost, F chain) {
+x3::Cut plan_cut(int nr, int64_t heads, int cus, const CutCost& cost, F chain) {
   x3::Cut c;
   c.len = 0;
   if (nr > x3::kMaxCut) return c;
@@ -1583,24 +1599,31 @@ x3::Cut plan_cut(int nr, int64_t heads, int64_t slots, const CutCost& cost, F ch
     longest = chain(r) > longest ? chain(r) : longest;
     total += heads * chain(r);
   }
-  auto lasts = [&](int64_t items, int len) {
-    const double item = len + cost.start;
-    const double mean = ((double)total + cost.start * (double)items) / (double)slots;
-    return cost.us * (items <= slots ? item : mean + 0.6 * item);
-  };
-  auto join = [&](int64_t items) { return 6.0 + (double)items * 2.0 * cost.bytes / 8e6; };
-  const double whole = (double)longest + cost.start, even = ((double)total + cost.start * (double)(heads * nr)) / (double)slots;
-  double best = 0.95 * (cost.us * (whole > even ? whole : even) + (cost.joined ? join(heads * nr) : 0.0));
-  for (int len = 4; len <= 32 && 2 * len <= longest + 8; ++len) {
+  auto items_of = [&](int len) {
     int64_t items = 0;
     for (int r = 0; r < nr; ++r) items += heads * ((chain(r) + len - 1) / len);
+    return items;
+  };
+  int len = 0;
+  double least = 0.0;
+  for (int l = 4; l <= 32 && 2 * l <= longest + 8; ++l) {
+    const int64_t items = items_of(l);
     if (items > (1 << 16)) continue;
-    const double us = lasts(items, len) + join(items);
-    if (us < best) {
-      best = us;
-      c.len = len;
+    const double item = l + cost.start, mean = ((double)total + cost.start * (double)items) / (double)cost.slots;
+    const double us = cost.us * (items <= cost.slots ? item : mean + 0.6 * item) + (double)items * 2.0 * cost.bytes / 8e6;
+    if (!len || us < least) {
+      least = us;
+      len = l;
     }
   }
+  if (!len) return c;
+  auto lasts = [&](int64_t items, int l, bool joined) {
+    const double item = cost.lone * (l + cost.extra);
+    const double load = cost.busy * ((double)total + cost.extra * (double)items) / cus;
+    return sqrt(sqrt(item * item * item * item + load * load * load * load)) +
+           (joined ? cost.join + (double)items * 2.0 * cost.bytes / (cost.gbs * 1e3) : 0.0);
+  };
+  if (lasts(items_of(len), len, true) < 0.98 * lasts(heads * nr, longest, cost.joined)) c.len = len;
   if (!c.len) return c;
   c.first[0] = 0;
   for (int r = 0; r < nr; ++r) c.first[r + 1] = c.first[r] + (int)heads * ((chain(r) + c.len - 1) / c.len);
@@ -1616,8 +1639,12 @@ int launch_fwd_mfma(float* O, float* lse, const float* Q, const float* K, const 
   if (rc) return rc;
   const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
   const int nqb = (T + 127) / 128, nk32 = (T + kBlk - 1) / kBlk;
-  const x3::Cut cut = plan_cut(nqb, (int64_t)B * nH, (int64_t)cus * (DH <= 32 ? 4 : DH <= 64 ? 3 : DH <= 96 ? 2 : 1),
-                               CutCost{DH <= 32 ? 0.9 : 2.1, 1.0, 512.0 * (DH + 2), false},
+  const double pb = 512.0 * (DH + 2);
+  const CutCost cost = DH <= 32   ? CutCost{4 * cus, 0.9, 1.0, pb, 0.87, 0.45, 0.4, 3.2, 3900.0, false}
+                       : DH <= 64 ? CutCost{3 * cus, 2.1, 1.0, pb, 1.14, 0.67, 0.0, 3.3, 4200.0, false}
+                       : DH <= 96 ? CutCost{2 * cus, 2.1, 1.0, pb, 1.55, 0.87, 8.0, 3.3, 5500.0, false}
+                                  : CutCost{cus, 2.1, 1.0, pb, 2.22, 2.11, 8.0, 5.0, 5300.0, false};
+  const x3::Cut cut = plan_cut(nqb, (int64_t)B * nH, cus, cost,
                                [&](int r) { return nk32 < (nqb - r) * 4 ? nk32 : (nqb - r) * 4; });
   fg::Workspace wp;  // whole chains where it cannot be had
   if (cut.len && wp.get(sizeof(float) * (size_t)cut.first[nqb] * x3::kFwdPart<DH>) == FG_OK) {
@@ -1680,10 +1707,15 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
   // few items and long chains: the query blocks of a key block in pieces
   x3::Cut cut;
   cut.len = 0;
-  if (dS)
-    cut = plan_cut(nkb, (int64_t)nbk * group, (int64_t)cus * (DH <= 32 ? 3 : DH <= 64 ? 2 : 1),
-                   CutCost{DH <= 32 ? 3.5 : 5.2, 1.5, 1024.0 * DH, group > 1},
-                   [&](int r) { return (int)nq32 - 4 * r; });
+  if (dS) {
+    const double pb = 1024.0 * DH;
+    const bool gqa = group > 1;
+    const CutCost cost = DH <= 32   ? CutCost{3 * cus, 3.5, 1.5, pb, 2.01, 0.81, 7.3, 1.1, 4400.0, gqa}
+                         : DH <= 64 ? CutCost{2 * cus, 5.2, 1.5, pb, 2.60, 1.71, 4.4, 1.8, 5100.0, gqa}
+                         : DH <= 96 ? CutCost{cus, 5.2, 1.5, pb, 4.52, 4.45, 8.0, 2.8, 5800.0, gqa}
+                                    : CutCost{cus, 5.2, 1.5, pb, 5.37, 5.51, 8.0, 2.5, 6300.0, gqa};
+    cut = plan_cut(nkb, (int64_t)nbk * group, cus, cost, [&](int r) { return (int)nq32 - 4 * r; });
+  }
   fg::Workspace wp, wc;
   float* part = nullptr;
   if (cut.len) {
@@ -1701,7 +1733,12 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
   FG_LAUNCH((x3::attn_bwd_merged<DH>), dim3(cut.len ? nkv_items : nkb * (nkv_items + nq_items)), dim3(kMThreads), 0, dQ, bq, dK, bk, dV,
             bv, Dq, dO, O, Q, K, V, lse, T, nH, nKV, scale, L, part, nbk, nkv_items, nq_items, dS, npairs, X, cut);
   if (dS) {
-    const x3::Cut qcut = plan_cut(nkb, (int64_t)B * nH, (int64_t)cus * 2, CutCost{0.95, 1.0, 512.0 * DH, false},
+    const double pb = 512.0 * DH;
+    const CutCost cost = DH <= 32   ? CutCost{2 * cus, 0.95, 1.0, pb, 0.79, 0.26, 4.0, 3.4, 3500.0, false}
+                         : DH <= 64 ? CutCost{2 * cus, 0.95, 1.0, pb, 0.94, 0.37, 4.0, 3.9, 4500.0, false}
+                         : DH <= 96 ? CutCost{2 * cus, 0.95, 1.0, pb, 1.07, 0.44, 4.0, 3.0, 4200.0, false}
+                                    : CutCost{2 * cus, 0.95, 1.0, pb, 1.27, 0.70, 4.0, 2.1, 3800.0, false};
+    const x3::Cut qcut = plan_cut(nkb, (int64_t)B * nH, cus, cost,
                                   [&](int r) { return nq32 < (nkb - r) * 4 ? (int)nq32 : (nkb - r) * 4; });
     fg::Workspace wdq;
     if (qcut.len && wdq.get(sizeof(float) * (size_t)qcut.first[nkb] * 128 * DH) == FG_OK) {
