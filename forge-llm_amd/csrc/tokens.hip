@@ -118,62 +118,109 @@ __global__ void __launch_bounds__(kThreads) embed_bwd_sorted_kernel(float* __res
   }
 }
 
-// The same sums for D % 4 == 0 and 16-byte aligned rows: one wave per sorted
-// position and run of 64 float4 columns, one float4 per lane (every element
-// still takes row + g[t1] + g[t2] + ... in increasing t, one fp32 add at a
-// time, as above).  A run's keys are read 64 at a time, one per lane, and its
-// gradient rows kRunLoads at a time before the first is added: text repeats
-// its commonest id hundreds of times in a step, and that run, walked one
-// dependent load after another by a wave that held the whole row, was the
-// launch's length (ids of frequency 1/rank, 8192 x 768: 323 us with one row
-// in flight, 50 us with 32).  beta 0 starts
-// each sum from +0 instead of reading the row (the same bits as reading a
-// zero row).
-constexpr int kRunLoads = 32;
+// The same sums for D % 4 == 0 and 16-byte aligned rows (every element still
+// takes row + g[t1] + g[t2] + ... in increasing t, one fp32 add at a time, as
+// above), by two kinds of workgroups.  Most ids of a step are alone or in a
+// short run: behind the first `scan` workgroups, one wave per sorted position
+// walks a run of up to kShortRun rows, J float4 per lane per pass (J·64 >= the
+// row width up to 1024 float4, so a row takes one pass): the row's loads and
+// those of its first gradient row are issued together.  Text repeats its
+// commonest id hundreds of times in a step, and such a run, walked like that,
+// was the launch's length.  A scan workgroup looks for longer runs at `span`
+// sorted positions and sums 256 of their columns, one float per lane, kRunLoads rows
+// in flight (as float4 their registers would leave three waves a SIMD, and a
+// launch with both kinds runs at the occupancy of the larger).  8192 x 768 onto
+// 32000 rows, ids of frequency 1/rank / uniform, us: every run by one wave 285 /
+// 12.4, every run with 32 rows of float4 in flight 47 / 21.2, this 42 / 12.7.
+// beta 0 starts each sum from +0 instead of reading the row (the same bits as
+// reading a zero row).
+constexpr int kShortRun = 8, kRunLoads = 32;
+template <int J>
 __global__ void __launch_bounds__(kThreads) embed_bwd_sorted4_kernel(float* __restrict__ gW,
                                                                      const float* __restrict__ g,
                                                                      const uint64_t* __restrict__ keys, int T,
-                                                                     int V, int D4, int beta) {
+                                                                     int V, int D, int beta, int scan,
+                                                                     int span) {
   const int lane = threadIdx.x & 63;
-  const int segs = (D4 + 63) / 64;
-  const int64_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6));
-  const int64_t nw = (int64_t)gridDim.x * (kThreads / 64);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if ((int)blockIdx.x < scan) {
+    const int segs = (D + 255) / 256;
+    const int s0 = (int)(blockIdx.x / segs) * span, s = s0 + lane;
+    const int col = (int)(blockIdx.x % segs) * 256 + wave * 64 + lane;
+    const int c = col < D ? col : D - 1;  // a valid column (not stored past D)
+    const uint32_t id = s < T ? (uint32_t)(keys[s] >> 32) : ~0u;  // kNoKey's id field is never a valid id
+    const uint32_t before = s > 0 && s < T ? (uint32_t)(keys[s - 1] >> 32) : ~0u;
+    const uint32_t after = s + kShortRun < T ? (uint32_t)(keys[s + kShortRun] >> 32) : ~0u;
+    for (uint64_t starts = __ballot(lane < span && id < (uint32_t)V && before != id && after == id); starts; starts &= starts - 1) {
+      const int at = __builtin_ctzll(starts);
+      const uint32_t own = __builtin_amdgcn_readlane(id, at);
+      float* row = gW + (int64_t)own * D;
+      float acc = beta ? row[c] : 0.f;
+      int64_t k = s0 + at;
+      for (bool more = true; more;) {
+        // the next keys of the run: lane l holds position k + l
+        const uint64_t kk = k + lane < T ? keys[k + lane] : kNoKey;
+        const uint64_t same = __ballot((uint32_t)(kk >> 32) == own);
+        const int n = ~same ? __builtin_ctzll(~same) : 64;
+        more = n == 64;
+        k += 64;
+        const int t = (int)(uint32_t)kk;
+        for (int i = 0; i < n; i += kRunLoads) {
+          float v[kRunLoads];
+#pragma unroll
+          for (int q = 0; q < kRunLoads; ++q)
+            if (i + q < n) v[q] = g[(int64_t)__builtin_amdgcn_readlane(t, i + q) * D + c];
+#pragma unroll
+          for (int q = 0; q < kRunLoads; ++q)
+            if (i + q < n) acc += v[q];
+        }
+      }
+      if (col < D) row[col] = acc;
+    }
+    return;
+  }
+  const int D4 = D / 4;
+  const int64_t nw = (int64_t)(gridDim.x - scan) * (kThreads / 64);
   const float4* g4 = reinterpret_cast<const float4*>(g);
-  for (int64_t w = wave; w < (int64_t)T * segs; w += nw) {
-    const int s = (int)(w / segs), seg = (int)(w - (int64_t)s * segs);
+  for (int64_t s = (int64_t)(blockIdx.x - scan) * (kThreads / 64) + wave; s < T; s += nw) {
     const uint64_t key = keys[s];
     const uint64_t prev = s > 0 ? keys[s - 1] : kNoKey;
+    const uint64_t far = s + kShortRun < T ? keys[s + kShortRun] : kNoKey;
     if (key == kNoKey) break;
     const uint32_t id = (uint32_t)(key >> 32);
     if (id >= (uint32_t)V) break;
-    if (s > 0 && (uint32_t)(prev >> 32) == id) continue;
-    const int col = seg * 64 + lane;
-    const bool in = col < D4;
-    const int c = in ? col : D4 - 1;  // a valid column (not stored past D4)
+    if ((s > 0 && (uint32_t)(prev >> 32) == id) || (uint32_t)(far >> 32) == id) continue;
     float4* row = reinterpret_cast<float4*>(gW) + (int64_t)id * D4;
-    float4 acc = beta ? row[c] : make_float4(0.f, 0.f, 0.f, 0.f);
-    int k = s;
-    for (bool more = true; more;) {
-      // the next keys of the run: lane l holds position k + l
-      const uint64_t kk = k + lane < T ? keys[k + lane] : kNoKey;
-      const uint64_t same = __ballot((uint32_t)(kk >> 32) == id);  // kNoKey's id field is never a valid id
-      const int n = ~same ? __builtin_ctzll(~same) : 64;
-      more = n == 64;
-      k += 64;
-      const int t = (int)(uint32_t)kk;
-      for (int i = 0; i < n; i += kRunLoads) {
-        float4 v[kRunLoads];
+    const float4* g0 = g4 + (int64_t)(uint32_t)key * D4;
+    for (int c0 = lane; c0 < D4; c0 += 64 * J) {
+      float4 acc[J], v[J];
 #pragma unroll
-        for (int q = 0; q < kRunLoads; ++q)
-          if (i + q < n) v[q] = g4[(int64_t)__builtin_amdgcn_readlane(t, i + q) * D4 + c];
+      for (int j = 0; j < J; ++j) {
+        const int c = c0 + 64 * j < D4 ? c0 + 64 * j : c0;  // a valid column (unused past D4)
+        acc[j] = beta ? row[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+        v[j] = g0[c];
+      }
 #pragma unroll
-        for (int q = 0; q < kRunLoads; ++q)
-          if (i + q < n) {
-            acc.x += v[q].x; acc.y += v[q].y; acc.z += v[q].z; acc.w += v[q].w;
-          }
+      for (int j = 0; j < J; ++j) {
+        acc[j].x += v[j].x; acc[j].y += v[j].y; acc[j].z += v[j].z; acc[j].w += v[j].w;
+      }
+      for (int64_t k = s + 1; k < T; ++k) {
+        const uint64_t kk = keys[k];
+        if ((uint32_t)(kk >> 32) != id) break;
+        const float4* gr = g4 + (int64_t)(uint32_t)kk * D4;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const int c = c0 + 64 * j < D4 ? c0 + 64 * j : c0;
+          const float4 u = gr[c];
+          acc[j].x += u.x; acc[j].y += u.y; acc[j].z += u.z; acc[j].w += u.w;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const int c = c0 + 64 * j;
+        if (c < D4) row[c] = acc[j];
       }
     }
-    if (in) row[col] = acc;
   }
 }
 
@@ -281,10 +328,15 @@ extern "C" int fg_embed_bwd_sorted(float* gW, const float* g, const uint64_t* ke
   fg::KProfScope prof("embed_bwd", 0.0, (beta ? 12.0 : 8.0) * (double)T * D);
   if (D % 4 == 0 && (uintptr_t)gW % 16 == 0 && (uintptr_t)g % 16 == 0) {
     const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
-    const int D4 = D / 4;
-    const int64_t waves = (int64_t)T * ((D4 + 63) / 64);
-    const int blocks = (int)max((int64_t)1, min((waves + 3) / 4, (int64_t)32 * cus));
-    FG_LAUNCH(embed_bwd_sorted4_kernel, dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D4, beta);
+    // one wave per sorted position, behind the scan; few positions are scanned in
+    // smaller shares, so that their long runs go side by side
+    const int span = T <= 1024 ? 16 : 64;
+    const int scan = T > kShortRun ? (T + span - 1) / span * ((D + 255) / 256) : 0;
+    const int blocks = scan + max(1, min((T + 3) / 4, 32 * cus)), D4 = D / 4;
+    if (D4 <= 64) FG_LAUNCH((embed_bwd_sorted4_kernel<1>), dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D, beta, scan, span);
+    else if (D4 <= 256) FG_LAUNCH((embed_bwd_sorted4_kernel<4>), dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D, beta, scan, span);
+    else if (D4 <= 512) FG_LAUNCH((embed_bwd_sorted4_kernel<8>), dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D, beta, scan, span);
+    else FG_LAUNCH((embed_bwd_sorted4_kernel<16>), dim3(blocks), dim3(kThreads), 0, gW, g, keys, T, V, D, beta, scan, span);
     return FG_OK;
   }
   const int grid = T < 2048 ? T : 2048;

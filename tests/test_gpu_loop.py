@@ -304,3 +304,29 @@ def test_embed_bwd_sorted_run_lengths(fh, run, D):
     fh.call("embed_bwd_sorted", gW, up(fh, g.ravel()), keys, T, V, D, 0)
     ref = oracle.embed_bwd(g.ravel(), ids, V, D, gW=np.zeros(V * D, np.float32))
     np.testing.assert_array_equal(gW.numpy(), ref)
+
+
+# runs on both sides of the rows that one wave walks (8), of the rows in flight
+# (32) and of the keys read at a time (64); several in the positions that one
+# workgroup scans (16 up to 1024 ids, then 64) and across its end
+@pytest.mark.gpu
+@pytest.mark.parametrize("run", [1, 7, 8, 9, 10, 31, 32, 33, 63, 64, 65, 127, 128, 200])
+@pytest.mark.parametrize("D,copies", [(4, 1), (256, 1), (260, 1), (260, 9), (1100, 3), (2052, 2), (4100, 1)])
+@pytest.mark.parametrize("beta", [0, 1])
+def test_embed_bwd_sorted_short_and_long_runs(fh, run, D, copies, beta):
+    """Runs of one id, columns of one lane, whole waves and a remainder, every
+    width of row: the sums in increasing position, bit for bit."""
+    ids = np.concatenate([np.full(run, 2 * i) for i in range(copies)] + [np.arange(1, 2 * copies, 2), [2 * copies] * 5, [-1, 99]])
+    T, V = len(ids), 2 * copies + 2
+    rng = np.random.default_rng(run + D)
+    ids = rng.permutation(ids).astype(np.int32)
+    g = rng.standard_normal((T, D)).astype(np.float32)
+    P = keys_len(fh, T)
+    keys = fh.DeviceArray((P,), np.uint64)
+    fh.call("embed_sort_keys", keys, P, up(fh, ids), T, V)
+    start = rng.standard_normal(V * D).astype(np.float32) if beta else np.zeros(V * D, np.float32)
+    gW = up(fh, start)
+    fh.call("embed_bwd_sorted", gW, up(fh, g.ravel()), keys, T, V, D, beta)
+    valid = (ids >= 0) & (ids < V)
+    ref = oracle.embed_bwd(g[valid].ravel(), ids[valid], V, D, gW=start.copy())
+    np.testing.assert_array_equal(gW.numpy(), ref)
