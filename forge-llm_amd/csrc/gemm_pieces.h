@@ -108,12 +108,37 @@ __global__ void __launch_bounds__(256) split_pieces_kernel(SplitTable t) {
   }
 }
 
-// 16 bytes per lane from base + voff straight into LDS at `lds` + 16 * lane
-// (lds wave-uniform).  The instruction has no register result; its arrival is
-// waited for explicitly (wait_lds_loads).
-__device__ __forceinline__ void load_to_lds(uint32_t lds, const char* base, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base)
-               : "memory");
+// 16 bytes per lane from each src[i] + voff straight into LDS at `lds` + 1024 i +
+// 16 * lane (lds wave-uniform).  The instructions have no register result; their
+// arrival is waited for explicitly (wait_lds_loads).  m0, which holds the LDS
+// address, cannot be named as clobbered (the compiler reserves it), so it is
+// given back; once per four or six loads that costs nothing (4096 x 28672 over K
+// = 4096 2362 us without, 2362 with, 2388 when every load gives it back).
+__device__ __forceinline__ void loads_to_lds(uint32_t lds, const char* const (&src)[4], uint32_t voff) {
+  uint32_t m0;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\t"
+      "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4\n\t"
+      "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %5\n\t"
+      "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %6\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(m0)
+      : "s"(lds), "v"(voff), "s"(src[0]), "s"(src[1]), "s"(src[2]), "s"(src[3])
+      : "memory", "scc");
+}
+__device__ __forceinline__ void loads_to_lds(uint32_t lds, const char* const (&src)[6], uint32_t voff) {
+  uint32_t m0;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\t"
+      "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4\n\t"
+      "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %5\n\t"
+      "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %6\n\t"
+      "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %7\n\t"
+      "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %8\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(m0)
+      : "s"(lds), "v"(voff), "s"(src[0]), "s"(src[1]), "s"(src[2]), "s"(src[3]), "s"(src[4]), "s"(src[5])
+      : "memory", "scc");
 }
 // All but this wave's N newest loads to LDS have arrived and its LDS reads are
 // done; then every wave's (barrier).
@@ -160,9 +185,7 @@ __device__ __forceinline__ void pieces_tile(char* lds, const char* __restrict__ 
   uint32_t vo = lane * 16;
   int ws = 0, rs = 0;  // stage of the next copy / read
   auto issue = [&]() {
-    const uint32_t s = l0 + ws * T::stage;
-#pragma unroll
-    for (int i = 0; i < L; ++i) load_to_lds(s + i * 1024, src[i], vo);
+    loads_to_lds(l0 + ws * T::stage, src, vo);
     vo += 2048;
     ws = ws == S - 1 ? 0 : ws + 1;
   };
