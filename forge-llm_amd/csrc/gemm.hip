@@ -2123,6 +2123,9 @@ namespace {
 // The list is cut into launches of at most kPieceJobs jobs, kGroupedBytes of
 // pieces and distinct outputs.
 constexpr int64_t kGroupedBytes = (int64_t)4 << 30;
+// A job's K pieces in the slab, up to where the next job's may start: the sum
+// reads them as float4.
+inline int64_t slab_floats(int splits, const fg_wgrad_job& jb) { return ((int64_t)splits * jb.N * jb.K + 3) / 4 * 4; }
 int grouped_pieces(const fg_wgrad_job* jobs, int count, int cus, bool& done) {
   done = false;
   double flop = 0.0;
@@ -2191,7 +2194,7 @@ int grouped_pieces(const fg_wgrad_job* jobs, int count, int cus, bool& done) {
     double lflop = 0.0, lbytes = 0.0;
     for (int j = b; j < e; ++j) {
       bytes += piece_bytes(jobs[j].N, jobs[j].M, TM) + piece_bytes(jobs[j].K, jobs[j].M, TN);
-      slab += (int64_t)splits * jobs[j].N * jobs[j].K;
+      slab += slab_floats(splits, jobs[j]);
       missing += !jobs[j].xp_gy + !jobs[j].xp_x;
     }
     fg::Workspace wsp, wss, wsx;
@@ -2236,7 +2239,7 @@ int grouped_pieces(const fg_wgrad_job* jobs, int count, int cus, bool& done) {
         next += kXpParts;
       }
       t.tiles += ((q.M + TM - 1) / TM) * ((q.N + TN - 1) / TN);
-      slab += (int64_t)splits * q.M * q.N;
+      slab += slab_floats(splits, jb);
       lflop += 2.0 * jb.M * jb.K * (double)jb.N;
       lbytes += 4.0 * ((double)q.M * jb.M + (double)q.N * jb.M + (1.0 + q.beta) * q.M * q.N);
     }

@@ -328,7 +328,7 @@ __global__ void __launch_bounds__(128 * WM, 2)
 
 // Several weight gradients in one launch (see GTable): job pieces per table
 // entry, one K split for all jobs (gridDim.y), its partial sums job after job
-// in `slab` ([job][split][M x N]).
+// in `slab` ([job][split][M x N], each job's from a 16-byte boundary on).
 struct PJob {
   float* C;
   const char* A;

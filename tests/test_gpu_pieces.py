@@ -110,3 +110,20 @@ def test_unaligned_operands_on_pieces(fh):
     dX, dW, Y = up(fh, X), up(fh, W), fh.DeviceArray((M, N))
     fh.call("matmulT_fwd", Y, dX.ptr + 4, dW.ptr + 12, M, K, N)
     _check(Y.numpy(), X[1:].reshape(M, K).astype(np.float64) @ W[3:].reshape(N, K).astype(np.float64).T, K)
+
+
+# jobs whose partial sums end between 16-byte boundaries, before others: odd
+# outputs over an odd number of K pieces
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes", [[(8192, 1535, 1535), (8192, 1536, 512)],
+                                    [(8192, 1103, 1101), (8192, 511, 1001), (8192, 512, 512)]])
+def test_grouped_partial_sums_of_odd_outputs(fh, shapes):
+    rs = np.random.default_rng(8)
+    host = [(rs.standard_normal((M, N), dtype=np.float32), rs.standard_normal((M, K), dtype=np.float32)) for M, K, N in shapes]
+    dev = [(up(fh, g), up(fh, x), fh.DeviceArray((N, K))) for (g, x), (M, K, N) in zip(host, shapes)]
+    jobs = (fh.WgradJob * len(shapes))(*[fh.WgradJob(w.ptr, g.ptr, x.ptr, M, K, N, 0, None, None)
+                                         for (g, x, w), (M, K, N) in zip(dev, shapes)])
+    fh.check(fh.lib.fg_matmulT_bwd_w_grouped(ctypes.cast(jobs, ctypes.c_void_p), len(shapes)), "grouped")
+    for (g, x), (_, _, w), (M, K, N) in zip(host, dev, shapes):
+        j = _sample(rs, N)
+        _check(w.numpy()[j], g[:, j].astype(np.float64).T @ x.astype(np.float64), M)
