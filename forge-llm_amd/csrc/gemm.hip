@@ -2117,158 +2117,360 @@ extern "C" int fg_matmulT_bwd_w(float* gW, const float* gY, const float* X, int 
 }
 
 namespace {
-// The grouped weight gradients on split operands, where the whole list gains
-// by it (the same times as plan_pieces, tiles and operands summed over the
-// jobs); `done` false: the caller takes the kernels that split while staging.
-// The list is cut into launches of at most kPieceJobs jobs, kGroupedBytes of
-// pieces and distinct outputs.
-constexpr int64_t kGroupedBytes = (int64_t)4 << 30;
+// ───────── grouped weight gradients: which kernels take which jobs ─────────
+// Jobs are planned in windows of at most kMaxJobs on distinct outputs (so that
+// their order does not matter): all on the kernels that split while staging,
+// all on split operands (gemm_pieces.h), or each job where it gains, by times
+// fitted to 332 lists (M 512 .. 8192, one job .. twelve layers with their head,
+// vocabularies of 1000 .. 50257; both within 10% of nearly all).  us, each side
+// measured, staging / pieces / taken:
+//   one job 50257 x 768, M 8192      2203 / 2518 / staging
+//   one job 50257 x 2048, M 8192     5692 / 4993 / pieces
+//   one job 1000 x 1024, M 4096       256 /   79 / pieces
+//   12 layers of 1024 with that head (V 50257, M 8192): the layers on pieces with
+//   the head 11800, all staging 12600, the head staging by itself and the layers
+//   together 10170
+// A staging launch: a 128 x 256 tile takes 0.88 us per 16 k (uneven: 0.93, 1.1
+// where they fill the chip), a 256 x 256 one 1.52 (1.74), the output goes out at
+// 6.5 TB/s (uneven 2.8).  Each XCD takes a contiguous range of the tiles, so the
+// slowest range counts.
+inline bool wgrad_even(const fg_wgrad_job& jb, int tm) {
+  return jb.N % tm == 0 && jb.K % 256 == 0 && jb.M % BK == 0 && (uintptr_t)jb.gY % 16 == 0 &&
+         (uintptr_t)jb.X % 16 == 0 && (uintptr_t)jb.gW % 16 == 0;
+}
+inline int64_t wgrad_tiles(const fg_wgrad_job& jb, int tm) {
+  return (int64_t)((jb.N + tm - 1) / tm) * ((jb.K + 255) / 256);
+}
+// us of one staged tile of `jb` in a list of `tiles`
+inline double staged_tile_us(const fg_wgrad_job& jb, bool wide, int64_t tiles, int cus) {
+  const bool even = wgrad_even(jb, wide ? 256 : 128);
+  const double busy = 2.0 * (double)tiles / cus - 1.0;
+  const double rate = wide ? (even ? 1.52 : 1.74)
+                           : (even ? 0.88 : 0.93 + 0.17 * (busy < 0.0 ? 0.0 : busy > 1.0 ? 1.0 : busy));
+  return rate * ((jb.M + 15) / 16);
+}
+inline double staged_out_us(const fg_wgrad_job& jb, bool wide) {
+  return 4.0 * jb.N * (double)jb.K / (wgrad_even(jb, wide ? 256 : 128) ? 6.5e6 : 2.8e6);
+}
+inline bool staged_wide(const fg_wgrad_job* const* jb, int count, int cus) {
+  int64_t n = 0;
+  for (int i = 0; i < count; ++i) n += wgrad_tiles(*jb[i], 256);
+  return n >= 2 * cus;
+}
+double staged_list_us(const fg_wgrad_job* const* jb, int count, int cus) {
+  if (!count) return 0.0;
+  const bool wide = staged_wide(jb, count, cus);
+  const int tm = wide ? 256 : 128;
+  int64_t tiles = 0;
+  int kmin = INT32_MAX;
+  for (int i = 0; i < count; ++i) {
+    tiles += wgrad_tiles(*jb[i], tm);
+    kmin = min(kmin, jb[i]->M);
+  }
+  constexpr int kXcds = 8;
+  double range[kXcds] = {}, longest = 0.0, out = 0.0;
+  int64_t at = 0;
+  for (int i = 0; i < count; ++i) {
+    const double us = staged_tile_us(*jb[i], wide, tiles, cus), end = (double)(at + wgrad_tiles(*jb[i], tm));
+    for (int x = 0; x < kXcds; ++x) {
+      const double lo = (double)tiles * x / kXcds, hi = (double)tiles * (x + 1) / kXcds;
+      const double n = (end < hi ? end : hi) - ((double)at > lo ? (double)at : lo);
+      if (n > 0.0) range[x] += n * us;
+    }
+    at = (int64_t)end;
+    longest = us > longest ? us : longest;
+    out += staged_out_us(*jb[i], wide);
+  }
+  if (tiles <= cus) return longest + out + 10.0;
+  double slowest = 0.0;
+  for (int x = 0; x < kXcds; ++x) slowest = range[x] > slowest ? range[x] : slowest;
+  const TailPlan tp = plan_tail(tiles, kmin, cus);
+  const double rounds = (double)(tiles / cus) + (tp.c > 1 ? (double)((tp.r * tp.c + cus - 1) / cus) / tp.c + 0.05
+                                                           : tiles % cus ? 1.0 : 0.0);
+  return rounds * slowest / ((double)tiles / kXcds) + out + 10.0;
+}
+
+// One launch on pieces: the times of plan_pieces, tiles and operands summed over
+// the jobs, and its outputs, which go out at 2.1 TB/s (the kernel's epilogue
+// reloads accumulators from scratch memory), once for every K piece.
+struct PieceList {
+  int wm, splits;
+  double us;
+};
+PieceList plan_piece_list(const fg_wgrad_job* const* jb, int count, int cus) {
+  PieceList best{2, 1, 1e30};
+  for (const int wm : {2, 4}) {
+    double tiles = 0.0, chunks = 0.0, pieces = 0.0, outs = 0.0;
+    int kmin = INT32_MAX;
+    for (int j = 0; j < count; ++j) {
+      const double t = (double)wgrad_tiles(*jb[j], 64 * wm);
+      const int nkc = (jb[j]->M + 15) / 16;
+      tiles += t;
+      chunks += t * nkc;
+      kmin = min(kmin, nkc);
+      pieces += (double)(piece_bytes(jb[j]->N, jb[j]->M, 64 * wm) + piece_bytes(jb[j]->K, jb[j]->M, 256)) / 4.0;
+      outs += (double)jb[j]->N * jb[j]->K;
+    }
+    for (int s = 1; s <= 8; ++s) {
+      if (s > 1 && kmin / s < 8) break;
+      double us = piece_waves_us((int64_t)tiles * s, (int)(chunks / tiles / s + 1.0), wm, cus) + pieces * 8.0 / 5.2e6 +
+                  s * outs * 4.0 / 2.1e6 + 10.0;
+      if (s > 1) us += (s + 1) * outs * 4.0 / 5e6 + 3.0;
+      if (us < best.us) best = PieceList{wm, s, us};
+    }
+  }
+  return best;
+}
+constexpr int64_t kGroupedBytes = (int64_t)4 << 30;  // pieces of one launch (of one job: whatever it needs up to this)
+inline int64_t wgrad_piece_bytes(const fg_wgrad_job& jb) {
+  return piece_bytes(jb.N, jb.M, 256) + piece_bytes(jb.K, jb.M, 256);
+}
+// How many jobs from the front one launch on pieces takes.
+int piece_launch_jobs(const fg_wgrad_job* const* jb, int count) {
+  int n = 0;
+  int64_t bytes = 0;
+  for (; n < count && n < kPieceJobs; ++n) {
+    bytes += wgrad_piece_bytes(*jb[n]);
+    if (n && bytes > kGroupedBytes) break;
+  }
+  return n;
+}
+double pieces_list_us(const fg_wgrad_job* const* jb, int count, int cus) {
+  double us = 0.0;
+  for (int b = 0; b < count;) {
+    const int n = piece_launch_jobs(jb + b, count - b);
+    us += plan_piece_list(jb + b, n, cus).us;
+    b += n;
+  }
+  return us;
+}
+
 // A job's K pieces in the slab, up to where the next job's may start: the sum
 // reads them as float4.
 inline int64_t slab_floats(int splits, const fg_wgrad_job& jb) { return ((int64_t)splits * jb.N * jb.K + 3) / 4 * 4; }
-int grouped_pieces(const fg_wgrad_job* jobs, int count, int cus, bool& done) {
-  done = false;
-  double flop = 0.0;
-  for (int i = 0; i < count; ++i) {
-    const fg_wgrad_job& jb = jobs[i];
-    if (!(jb.gW && jb.gY && jb.X && jb.M > 0 && jb.K > 0 && jb.N > 0)) return FG_OK;  // reported by the caller
-    if (4 * (piece_bytes(jb.N, jb.M, 256) + piece_bytes(jb.K, jb.M, 256)) > 2 * kPiecesMaxBytes) return FG_OK;
-    flop += 2.0 * jb.M * jb.K * (double)jb.N;
+
+// One launch on pieces; `got` is false when its workspace cannot be had, and
+// nothing is queued then.
+int launch_grouped_pieces(const fg_wgrad_job* const* jb, int count, int cus, bool& got) {
+  const PieceList pl = plan_piece_list(jb, count, cus);
+  const int TM = 64 * pl.wm, TN = 256;
+  int64_t bytes = 0, slab = 0;
+  int missing = 0;
+  for (int j = 0; j < count; ++j) {
+    bytes += piece_bytes(jb[j]->N, jb[j]->M, TM) + piece_bytes(jb[j]->K, jb[j]->M, TN);
+    slab += slab_floats(pl.splits, *jb[j]);
+    missing += !jb[j]->xp_gy + !jb[j]->xp_x;
   }
-  if (flop < 8e9) return FG_OK;
-  int b = 0;
-  while (b < count) {
-    // the next launch: jobs [b, e)
-    int e = b;
-    int64_t bytes = 0;
-    for (; e < count && e - b < kPieceJobs; ++e) {
-      const int64_t add = piece_bytes(jobs[e].N, jobs[e].M, 256) + piece_bytes(jobs[e].K, jobs[e].M, 256);
-      bool again = false;
-      for (int j = b; j < e; ++j) again |= jobs[j].gW == jobs[e].gW;
-      if (again || (e > b && bytes + add > kGroupedBytes)) break;
-      bytes += add;
+  fg::Workspace wsp, wss, wsx;
+  got = wsp.get((size_t)bytes) == FG_OK && (pl.splits == 1 || wss.get(sizeof(float) * (size_t)slab) == FG_OK) &&
+        (!missing || wsx.get((size_t)missing * kXpParts * sizeof(float)) == FG_OK);
+  if (!got) return FG_OK;
+  PTable t;
+  t.count = count;
+  t.tiles = 0;
+  t.splits = pl.splits;
+  t.slab = (float*)wss.ptr;
+  XpTable xt;
+  xt.count = 0;
+  float* next = static_cast<float*>(wsx.ptr);
+  char* pieces = (char*)wsp.ptr;
+  double lflop = 0.0, lbytes = 0.0;
+  slab = 0;
+  for (int j = 0; j < count; ++j) {
+    const fg_wgrad_job& w = *jb[j];
+    PJob& q = t.job[j];
+    q.C = w.gW;
+    q.M = w.N;  // gW[N,K] (+)= gY^T · X: M_gemm = N, N_gemm = K, K_gemm = M
+    q.N = w.K;
+    q.nkc = (w.M + 15) / 16;
+    q.beta = w.beta ? 1 : 0;
+    q.tile0 = t.tiles;
+    q.slab0 = slab;
+    q.A = pieces;
+    pieces += piece_bytes(w.N, w.M, TM);
+    q.B = pieces;
+    pieces += piece_bytes(w.K, w.M, TN);
+    q.xpa = w.xp_gy;
+    q.xpb = w.xp_x;
+    if (!q.xpa) {
+      xt.job[xt.count++] = xp_job(w.gY, false, w.N, w.M, w.N, next);
+      q.xpa = next;
+      next += kXpParts;
     }
-    int wm = 0, splits = 1;
-    double best = 10.0;  // the kernels that split while staging (see plan_pieces)
-    for (int j = b; j < e; ++j) {
-      const fg_wgrad_job& jb = jobs[j];
-      const bool even = jb.N % 256 == 0 && jb.K % 256 == 0 && jb.M % BK == 0 && (uintptr_t)jb.gY % 16 == 0 &&
-                        (uintptr_t)jb.X % 16 == 0 && (uintptr_t)jb.gW % 16 == 0;
-      best += staged_us(2.0 * jb.M * jb.K * (double)jb.N, false, false, even) - staged_us(0.0, false, false, even);
+    if (!q.xpb) {
+      xt.job[xt.count++] = xp_job(w.X, false, w.K, w.M, w.K, next);
+      q.xpb = next;
+      next += kXpParts;
     }
-    for (const int cwm : {2, 4}) {
-      double tiles = 0.0, chunks = 0.0, pieces = 0.0, outs = 0.0;
-      int kmin = INT32_MAX;
-      for (int j = b; j < e; ++j) {
-        const double t = (double)((jobs[j].N + 64 * cwm - 1) / (64 * cwm)) * ((jobs[j].K + 255) / 256);
-        const int nkc = (jobs[j].M + 15) / 16;
-        tiles += t;
-        chunks += t * nkc;
-        kmin = min(kmin, nkc);
-        pieces += (double)(piece_bytes(jobs[j].N, jobs[j].M, 64 * cwm) + piece_bytes(jobs[j].K, jobs[j].M, 256)) / 4.0;
-        outs += (double)jobs[j].N * jobs[j].K;
-      }
-      for (int s = 1; s <= 8; ++s) {
-        if (s > 1 && kmin / s < 8) break;
-        double us = piece_waves_us((int64_t)tiles * s, (int)(chunks / tiles / s + 1.0), cwm, cus) +
-                    pieces * 8.0 / 5.2e6 + 10.0;
-        if (s > 1) us += (s + 1) * outs * 4.0 / 5e6 + 3.0;
-        if (us < best) {
-          best = us;
-          wm = cwm;
-          splits = s;
-        }
-      }
-    }
-    if (!wm && b == 0) return FG_OK;
-    if (!wm) wm = 2;  // a remainder of a list that started on pieces
-    const int TM = 64 * wm, TN = 256;
-    PTable t;
-    t.count = e - b;
-    t.tiles = 0;
-    t.splits = splits;
-    t.slab = nullptr;
-    bytes = 0;
-    int64_t slab = 0;
-    int missing = 0;
-    double lflop = 0.0, lbytes = 0.0;
-    for (int j = b; j < e; ++j) {
-      bytes += piece_bytes(jobs[j].N, jobs[j].M, TM) + piece_bytes(jobs[j].K, jobs[j].M, TN);
-      slab += slab_floats(splits, jobs[j]);
-      missing += !jobs[j].xp_gy + !jobs[j].xp_x;
-    }
-    fg::Workspace wsp, wss, wsx;
-    if (wsp.get((size_t)bytes) != FG_OK || (splits > 1 && wss.get(sizeof(float) * (size_t)slab) != FG_OK)) {
-      if (b == 0) return FG_OK;
-      return FG_ERR_OOM;
-    }
-    if (missing) {
-      int rc = wsx.get((size_t)missing * kXpParts * sizeof(float));
+    t.tiles += ((q.M + TM - 1) / TM) * ((q.N + TN - 1) / TN);
+    slab += slab_floats(pl.splits, w);
+    lflop += 2.0 * w.M * w.K * (double)w.N;
+    lbytes += 4.0 * ((double)q.M * w.M + (double)q.N * w.M + (1.0 + q.beta) * q.M * q.N);
+  }
+  int rc = queue_absmax(xt, true);
+  if (rc) return rc;
+  SplitTable st;
+  st.count = 0;
+  for (int j = 0; j < count; ++j) {
+    const fg_wgrad_job& w = *jb[j];
+    const PJob& q = t.job[j];
+    st.job[st.count++] = SplitJob{w.gY, (char*)q.A, q.xpa, q.M, w.M, w.N, q.nkc, (q.M + TM - 1) / TM * 2 * pl.wm, 0, 0, 0};
+    st.job[st.count++] = SplitJob{w.X, (char*)q.B, q.xpb, q.N, w.M, w.K, q.nkc, (q.N + TN - 1) / TN * 8, 0, 0, 0};
+    if (st.count == kSplitJobs || j + 1 == count) {
+      rc = queue_split(st, true);
       if (rc) return rc;
+      st.count = 0;
     }
-    float* next = static_cast<float*>(wsx.ptr);
-    XpTable xt;
-    xt.count = 0;
-    char* pieces = (char*)wsp.ptr;
-    t.slab = (float*)wss.ptr;
-    slab = 0;
-    for (int j = b; j < e; ++j) {
-      const fg_wgrad_job& jb = jobs[j];
-      PJob& q = t.job[j - b];
-      q.C = jb.gW;
-      q.M = jb.N;  // gW[N,K] (+)= gY^T · X: M_gemm = N, N_gemm = K, K_gemm = M
-      q.N = jb.K;
-      q.nkc = (jb.M + 15) / 16;
-      q.beta = jb.beta ? 1 : 0;
-      q.tile0 = t.tiles;
-      q.slab0 = slab;
-      q.A = pieces;
-      pieces += piece_bytes(jb.N, jb.M, TM);
-      q.B = pieces;
-      pieces += piece_bytes(jb.K, jb.M, TN);
-      q.xpa = jb.xp_gy;
-      q.xpb = jb.xp_x;
-      if (!q.xpa) {
-        xt.job[xt.count++] = xp_job(jb.gY, false, jb.N, jb.M, jb.N, next);
-        q.xpa = next;
-        next += kXpParts;
-      }
-      if (!q.xpb) {
-        xt.job[xt.count++] = xp_job(jb.X, false, jb.K, jb.M, jb.K, next);
-        q.xpb = next;
-        next += kXpParts;
-      }
-      t.tiles += ((q.M + TM - 1) / TM) * ((q.N + TN - 1) / TN);
-      slab += slab_floats(splits, jb);
-      lflop += 2.0 * jb.M * jb.K * (double)jb.N;
-      lbytes += 4.0 * ((double)q.M * jb.M + (double)q.N * jb.M + (1.0 + q.beta) * q.M * q.N);
-    }
-    int rc = queue_absmax(xt, true);
+  }
+  fg::KProfScope prof("gemm_tn", lflop, lbytes);
+  const dim3 grid(t.tiles, pl.splits), block(128 * pl.wm);
+  if (pl.wm == 4)
+    FG_LAUNCH((gemm_pieces_grouped<4, 4, 4>), grid, block, 0, t);
+  else
+    FG_LAUNCH((gemm_pieces_grouped<2, 4, 3>), grid, block, 0, t);
+  if (pl.splits > 1) FG_LAUNCH(splitk_reduce_grouped, dim3(4 * cus, t.count), dim3(256), 0, t);
+  return FG_OK;
+}
+
+// One launch (and its tail's sum) on the kernels that split while staging:
+// 256x256 tiles (gemm_w_grouped) when they make at least two rounds of CUs,
+// else 128x256 ping-pong tiles (twice as many to spread).  At most kMaxJobs.
+int launch_grouped_staged(const fg_wgrad_job* const* jb, int count, int cus) {
+  const bool wide = staged_wide(jb, count, cus);
+  const int TM = wide ? 256 : 128, TN = 256;
+  GTable t;
+  double flop = 0.0, bytes = 0.0;
+  t.count = count;
+  t.prefix[0] = 0;
+  int missing = 0, kmin = INT32_MAX;
+  for (int j = 0; j < count; ++j) {
+    const fg_wgrad_job& w = *jb[j];
+    // gW[N,K] (+)= gY^T · X: the TN layout of fg_matmulT_bwd_w, M_gemm = N, N_gemm = K, K_gemm = M
+    const int64_t tiles = t.prefix[j] + wgrad_tiles(w, TM);
+    FG_ARG_CHECK(tiles < (1ll << 31), "fg_matmulT_bwd_w_grouped: too many tiles");
+    t.prefix[j + 1] = (int)tiles;
+    GJob& g = t.job[j];
+    g.C = w.gW;
+    g.A = w.gY;
+    g.B = w.X;
+    g.xpa = w.xp_gy;
+    g.xpb = w.xp_x;
+    g.M = w.N;
+    g.N = w.K;
+    g.K = w.M;
+    g.lda = w.N;
+    g.ldb = w.K;
+    g.beta = w.beta ? 1 : 0;
+    g.even = wgrad_even(w, TM);
+    missing += !g.xpa + !g.xpb;
+    kmin = min(kmin, w.M);
+    flop += 2.0 * w.M * w.K * (double)w.N;
+    bytes += 4.0 * ((double)w.N * w.M + (double)w.K * w.M + (1.0 + g.beta) * w.N * w.K);
+  }
+  // the maxima the jobs do not bring, into one workspace
+  fg::Workspace wsx;
+  XpTable xt;
+  xt.count = 0;
+  if (missing) {
+    int rc = wsx.get((size_t)missing * kXpParts * sizeof(float));
     if (rc) return rc;
-    SplitTable st;
-    st.count = 0;
-    for (int j = b; j < e; ++j) {
-      const fg_wgrad_job& jb = jobs[j];
-      const PJob& q = t.job[j - b];
-      st.job[st.count++] = SplitJob{jb.gY, (char*)q.A, q.xpa, q.M, jb.M, jb.N, q.nkc, (q.M + TM - 1) / TM * 2 * wm, 0, 0, 0};
-      st.job[st.count++] = SplitJob{jb.X, (char*)q.B, q.xpb, q.N, jb.M, jb.K, q.nkc, (q.N + TN - 1) / TN * 8, 0, 0, 0};
-      if (st.count == kSplitJobs || j + 1 == e) {
-        rc = queue_split(st, true);
-        if (rc) return rc;
-        st.count = 0;
+    float* next = static_cast<float*>(wsx.ptr);
+    for (int j = 0; j < count; ++j) {
+      GJob& g = t.job[j];
+      if (!g.xpa) {
+        xt.job[xt.count++] = xp_job(g.A, false, g.M, g.K, g.lda, next);
+        g.xpa = next;
+        next += kXpParts;
+      }
+      if (!g.xpb) {
+        xt.job[xt.count++] = xp_job(g.B, false, g.N, g.K, g.ldb, next);
+        g.xpb = next;
+        next += kXpParts;
       }
     }
-    fg::KProfScope prof("gemm_tn", lflop, lbytes);
-    const dim3 grid(t.tiles, splits), block(128 * wm);
-    if (wm == 4)
-      FG_LAUNCH((gemm_pieces_grouped<4, 4, 4>), grid, block, 0, t);
-    else
-      FG_LAUNCH((gemm_pieces_grouped<2, 4, 3>), grid, block, 0, t);
-    if (splits > 1) FG_LAUNCH(splitk_reduce_grouped, dim3(4 * cus, t.count), dim3(256), 0, t);
-    done = true;
-    b = e;
+  }
+  int rc = queue_absmax(xt, true);
+  if (rc) return rc;
+  fg::KProfScope prof("gemm_tn", flop, bytes);
+  // tail split over the whole launch, pieces sized by the smallest job K
+  const int tiles = t.prefix[count];
+  const TailPlan tp = plan_tail(tiles, kmin, cus);
+  fg::Workspace ws;
+  t.n_full = tiles - tp.r;
+  t.tail_c = tp.c;
+  t.slab = nullptr;
+  if (tp.c > 1) {
+    rc = ws.get(sizeof(float) * (size_t)tp.r * tp.c * TM * TN);
+    if (rc) return rc;
+    t.slab = (float*)ws.ptr;
+  }
+  if (wide) {
+    FG_LAUNCH((gemm_w_grouped<false, false>), dim3(t.n_full + tp.r * tp.c), dim3(kPPThreads), 0, t);
+    if (tp.c > 1) FG_LAUNCH((tail_reduce_grouped<256, 256>), dim3(32, tp.r), dim3(256), 0, t);
+  } else {
+    FG_LAUNCH((gemm_pp_grouped<128, 256, false, false>), dim3(t.n_full + tp.r * tp.c), dim3(kPPThreads), 0, t);
+    if (tp.c > 1) FG_LAUNCH((tail_reduce_grouped<128, 256>), dim3(32, tp.r), dim3(256), 0, t);
   }
   return FG_OK;
+}
+
+// A window: at most kMaxJobs jobs on distinct outputs.  Pieces have to be
+// faster by a margin of 8%, what the fitted times are good for.
+int grouped_window(const fg_wgrad_job* jobs, int count, int cus) {
+  const fg_wgrad_job *all[kMaxJobs], *pc[kMaxJobs], *st[kMaxJobs];
+  int np = 0, ns = 0;
+  bool fits = true;
+  double flop = 0.0, pflop = 0.0;
+  for (int i = 0; i < count; ++i) all[i] = jobs + i;
+  const bool wide = staged_wide(all, count, cus);
+  int64_t tiles = 0;
+  for (int i = 0; i < count; ++i) tiles += wgrad_tiles(jobs[i], wide ? 256 : 128);
+  for (int i = 0; i < count; ++i) {  // what the job takes of a full chip either way
+    const fg_wgrad_job& jb = jobs[i];
+    const double f = 2.0 * jb.M * jb.K * (double)jb.N, nk = (jb.M + 15) / 16;
+    const double staged =
+        wgrad_tiles(jb, wide ? 256 : 128) * staged_tile_us(jb, wide, tiles, cus) / cus + staged_out_us(jb, wide);
+    const double two = wgrad_tiles(jb, 128) * (1.18 * nk + 8.0) / 2.0, four = wgrad_tiles(jb, 256) * (1.13 * nk + 14.0);
+    const double piece = (two < four ? two : four) / cus + 2.0 * (double)wgrad_piece_bytes(jb) / 5.2e6 +
+                         4.0 * jb.N * (double)jb.K / 2.1e6;
+    const bool fit = wgrad_piece_bytes(jb) <= kGroupedBytes;
+    fits = fits && fit;
+    flop += f;
+    if (fit && piece < 0.92 * staged) {
+      pc[np++] = &jb;
+      pflop += f;
+    } else {
+      st[ns++] = &jb;
+    }
+  }
+  double best = 0.92 * staged_list_us(all, count, cus);
+  int form = 0;  // all staging
+  if (fits && flop >= 8e9) {
+    const double us = pieces_list_us(all, count, cus);
+    if (us < best) {
+      best = us;
+      form = 1;
+    }
+  }
+  if (np && ns && pflop >= 8e9) {
+    const double us = pieces_list_us(pc, np, cus) + 0.92 * staged_list_us(st, ns, cus);
+    if (us < best) form = 2;
+  }
+  if (form < 2) {
+    np = form ? count : 0;
+    ns = form ? 0 : count;
+    for (int i = 0; i < count; ++i) (form ? pc : st)[i] = all[i];
+  }
+  for (int b = 0; b < np;) {
+    const int n = piece_launch_jobs(pc + b, np - b);
+    bool got = false;
+    int rc = launch_grouped_pieces(pc + b, n, cus, got);
+    if (rc) return rc;
+    if (!got)  // no workspace for them: the kernels that need none
+      for (int i = 0; i < n; ++i) st[ns++] = pc[b + i];
+    b += n;
+  }
+  return ns ? launch_grouped_staged(st, ns, cus) : FG_OK;
 }
 }  // namespace
 
@@ -2280,7 +2482,6 @@ int grouped_small(const fg_wgrad_job* jobs, int count, bool& done) {
   int64_t work = 0;
   for (int i = 0; i < count; ++i) {
     const fg_wgrad_job& jb = jobs[i];
-    if (!(jb.gW && jb.gY && jb.X && jb.M > 0 && jb.K > 0 && jb.N > 0)) return FG_OK;  // reported by the caller
     if ((int64_t)jb.M * jb.K > kSmallMax || (int64_t)jb.M * jb.K * jb.N > kSmallMax - work) return FG_OK;
     work += (int64_t)jb.M * jb.K * jb.N;
   }
@@ -2318,123 +2519,28 @@ int grouped_small(const fg_wgrad_job* jobs, int count, bool& done) {
 extern "C" int fg_matmulT_bwd_w_grouped(const fg_wgrad_job* jobs, int count) {
   FG_REQUIRE_INIT();
   FG_ARG_CHECK(count >= 0 && (count == 0 || jobs), "fg_matmulT_bwd_w_grouped: bad job list");
-  const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
-  {
-    bool done = false;
-    int rc = grouped_small(jobs, count, done);
-    if (rc || done) return rc;
-    rc = grouped_pieces(jobs, count, cus, done);
-    if (rc || done) return rc;
-  }
-  // 256x256 tiles (gemm_w_grouped) when they make at least two rounds of
-  // CUs, else 128x256 ping-pong tiles (twice as many to spread)
-  int64_t w_tiles = 0;
   for (int i = 0; i < count; ++i)
-    w_tiles += (int64_t)((jobs[i].N + 255) / 256) * ((jobs[i].K + 255) / 256);
-  const bool wide = w_tiles >= 2 * cus;
-  const int TM = wide ? 256 : 128, TN = 256;
-  GTable t;
-  double flop = 0.0, bytes = 0.0;
-  auto flush = [&]() -> int {
-    if (t.count == 0) return FG_OK;
-    // the maxima the jobs do not bring, into one workspace
-    fg::Workspace wsx;
-    {
-      int missing = 0;
-      for (int j = 0; j < t.count; ++j) missing += (t.job[j].xpa == nullptr) + (t.job[j].xpb == nullptr);
-      XpTable xt;
-      xt.count = 0;
-      if (missing) {
-        int rc = wsx.get((size_t)missing * kXpParts * sizeof(float));
-        if (rc) return rc;
-        float* next = static_cast<float*>(wsx.ptr);
-        for (int j = 0; j < t.count; ++j) {
-          GJob& g = t.job[j];
-          if (!g.xpa) {
-            xt.job[xt.count++] = xp_job(g.A, false, g.M, g.K, g.lda, next);
-            g.xpa = next;
-            next += kXpParts;
-          }
-          if (!g.xpb) {
-            xt.job[xt.count++] = xp_job(g.B, false, g.N, g.K, g.ldb, next);
-            g.xpb = next;
-            next += kXpParts;
-          }
-        }
-      }
-      int rc = queue_absmax(xt, true);
-      if (rc) return rc;
+    FG_ARG_CHECK(jobs[i].gW && jobs[i].gY && jobs[i].X && jobs[i].M > 0 && jobs[i].K > 0 && jobs[i].N > 0,
+                 "fg_matmulT_bwd_w_grouped: job %d has a null pointer or a bad shape (M=%d K=%d N=%d)", i, jobs[i].M,
+                 jobs[i].K, jobs[i].N);
+  const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
+  bool done = false;
+  int rc = grouped_small(jobs, count, done);
+  if (rc || done) return rc;
+  for (int b = 0; b < count;) {
+    // a job on a gW that the window already writes starts the next one, so jobs
+    // on one output apply in list order
+    int e = b + 1;
+    for (; e < count && e - b < kMaxJobs; ++e) {
+      bool again = false;
+      for (int j = b; j < e; ++j) again |= jobs[j].gW == jobs[e].gW;
+      if (again) break;
     }
-    fg::KProfScope prof("gemm_tn", flop, bytes);
-    // tail split over the whole launch, pieces sized by the smallest job K
-    const int tiles = t.prefix[t.count];
-    int kmin = t.job[0].K;
-    for (int j = 1; j < t.count; ++j) kmin = min(kmin, t.job[j].K);
-    const TailPlan tp = plan_tail(tiles, kmin, cus);
-    fg::Workspace ws;
-    t.n_full = tiles - tp.r;
-    t.tail_c = tp.c;
-    t.slab = nullptr;
-    if (tp.c > 1) {
-      int rc = ws.get(sizeof(float) * (size_t)tp.r * tp.c * TM * TN);
-      if (rc) return rc;
-      t.slab = (float*)ws.ptr;
-    }
-    if (wide) {
-      FG_LAUNCH((gemm_w_grouped<false, false>), dim3(t.n_full + tp.r * tp.c), dim3(kPPThreads), 0, t);
-      if (tp.c > 1) FG_LAUNCH((tail_reduce_grouped<256, 256>), dim3(32, tp.r), dim3(256), 0, t);
-    } else {
-      FG_LAUNCH((gemm_pp_grouped<128, 256, false, false>), dim3(t.n_full + tp.r * tp.c), dim3(kPPThreads), 0, t);
-      if (tp.c > 1) FG_LAUNCH((tail_reduce_grouped<128, 256>), dim3(32, tp.r), dim3(256), 0, t);
-    }
-    t.count = 0;
-    flop = bytes = 0.0;
-    return FG_OK;
-  };
-  t.count = 0;
-  t.prefix[0] = 0;
-  for (int i = 0; i < count; ++i) {
-    const fg_wgrad_job& jb = jobs[i];
-    FG_ARG_CHECK(jb.gW && jb.gY && jb.X && jb.M > 0 && jb.K > 0 && jb.N > 0,
-                 "fg_matmulT_bwd_w_grouped: job %d has a null pointer or a bad shape (M=%d K=%d N=%d)", i, jb.M,
-                 jb.K, jb.N);
-    // a job on a gW already written by this table's jobs starts the next
-    // launch, so jobs on one output apply in list order
-    for (int j = 0; j < t.count; ++j) {
-      if (t.job[j].C == jb.gW) {
-        int rc = flush();
-        if (rc) return rc;
-        break;
-      }
-    }
-    // gW[N,K] (+)= gY^T · X: the TN layout of fg_matmulT_bwd_w, M_gemm = N, N_gemm = K, K_gemm = M
-    const int Mg = jb.N, Ng = jb.K, Kg = jb.M;
-    const int tiles = ((Mg + TM - 1) / TM) * ((Ng + TN - 1) / TN);
-    FG_ARG_CHECK((int64_t)t.prefix[t.count] + tiles < (1ll << 31), "fg_matmulT_bwd_w_grouped: too many tiles");
-    GJob& g = t.job[t.count];
-    g.C = jb.gW;
-    g.A = jb.gY;
-    g.B = jb.X;
-    g.xpa = jb.xp_gy;
-    g.xpb = jb.xp_x;
-    g.M = Mg;
-    g.N = Ng;
-    g.K = Kg;
-    g.lda = jb.N;
-    g.ldb = jb.K;
-    g.beta = jb.beta ? 1 : 0;
-    g.even = (Mg % TM == 0) && (Ng % TN == 0) && (Kg % BK == 0) && (g.lda % 4 == 0) && (g.ldb % 4 == 0) &&
-             ((uintptr_t)g.A % 16 == 0) && ((uintptr_t)g.B % 16 == 0) && ((uintptr_t)g.C % 16 == 0);
-    t.prefix[t.count + 1] = t.prefix[t.count] + tiles;
-    t.count += 1;
-    flop += 2.0 * Mg * Ng * (double)Kg;
-    bytes += 4.0 * ((double)Mg * Kg + (double)Ng * Kg + (1.0 + g.beta) * Mg * Ng);
-    if (t.count == kMaxJobs) {
-      int rc = flush();
-      if (rc) return rc;
-    }
+    rc = grouped_window(jobs + b, e - b, cus);
+    if (rc) return rc;
+    b = e;
   }
-  return flush();
+  return FG_OK;
 }
 
 extern "C" int fg_matmulT_bwd_p(float* gX, int beta_x, float* gW, int beta_w, const float* gY, const float* X,

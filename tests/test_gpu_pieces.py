@@ -127,3 +127,32 @@ def test_grouped_partial_sums_of_odd_outputs(fh, shapes):
     for (g, x), (_, _, w), (M, K, N) in zip(host, dev, shapes):
         j = _sample(rs, N)
         _check(w.numpy()[j], g[:, j].astype(np.float64).T @ x.astype(np.float64), M)
+
+
+# lists whose jobs are told apart: uneven ones go to pieces, even ones stay with
+# the kernels that split while staging; a list on pieces as a whole; more jobs
+# than a window; a job on an earlier job's output after it
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes", [
+    [(4096, 2048, 4001), (4096, 1024, 8192), (4096, 1024, 8192), (4096, 1024, 8192), (4096, 1024, 8192)],
+    [(8192, 1024, 4096), (8192, 1025, 1001), (8192, 1024, 4096), (8192, 1025, 1001), (8192, 1025, 1001)],
+    [(4096, 4096, 4096), (4096, 768, 16385), (4096, 4096, 4096)],
+    [(1024, 512, 512)] * 50 + [(1024, 300, 1001)] * 6,
+])
+def test_grouped_lists_told_apart(fh, shapes):
+    rs = np.random.default_rng(len(shapes))
+    host, dev = {}, {}
+    for M, K, N in set(shapes):
+        host[M, K, N] = rs.standard_normal((M, N), dtype=np.float32), rs.standard_normal((M, K), dtype=np.float32)
+        dev[M, K, N] = [up(fh, a) for a in host[M, K, N]]
+    w = [up(fh, np.full((N, K), 0.5, np.float32)) for M, K, N in shapes]
+    order = list(range(len(shapes))) + [0, len(shapes) - 1]  # the last two accumulate onto written outputs
+    jobs = (fh.WgradJob * len(order))(*[
+        fh.WgradJob(w[i].ptr, dev[shapes[i]][0].ptr, dev[shapes[i]][1].ptr, *shapes[i], int(p >= len(shapes) or p % 2), None, None)
+        for p, i in enumerate(order)])
+    fh.check(fh.lib.fg_matmulT_bwd_w_grouped(ctypes.cast(jobs, ctypes.c_void_p), len(order)), "grouped")
+    for i, (M, K, N) in enumerate(shapes):
+        g, x = host[M, K, N]
+        j = _sample(rs, N, 12)
+        ref = g[:, j].astype(np.float64).T @ x.astype(np.float64)
+        _check(w[i].numpy()[j], ref * order.count(i) + 0.5 * (i % 2), M)
