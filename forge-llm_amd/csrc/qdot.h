@@ -288,6 +288,11 @@ inline int unit_parts(int U) {
   while (P < kUnitWaves && 64 * P < U) P <<= 1;
   return P;
 }
+// The share of its lanes that P waves use over the steps of a row of U units.
+inline double unit_fill(int U) {
+  const int step = 64 * unit_parts(U);
+  return (double)U / ((U + step - 1) / step * step);
+}
 template <int CTRL>
 __device__ __forceinline__ double dpp_mov_d(double v) {
   const uint64_t b = __builtin_bit_cast(uint64_t, v);

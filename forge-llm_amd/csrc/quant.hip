@@ -491,23 +491,54 @@ unsigned grid_for(int64_t items, int per_block) {
   return (unsigned)(g < 1 ? 1 : g);
 }
 
+// Rows per wave in units, or 0 where the element order is the faster form: for
+// each type, 15 row lengths K = 256 .. 14336 and 12 counts N = 300 .. 128000, from
+// memory and from the caches; the lines below lose to the element order by more
+// than 3% in 2 of 1700 points (units as far as each type went before: 123, up to
+// 35%).  us from the caches, element order / one row / four rows a wave:
+//   few rows: one each, their loads all in flight (Q4_K 1000 x 4096 6.4 / 4.1 / 4.9)
+//   many rows, one wave to a row's units: four share x and its sums, except Q6_K,
+//     whose longer dot has no registers for four (12000 x 2048 10.9 / 10.0 / 9.6 from
+//     the caches, 16000: 13.6 / 12.5 / 13.1)
+//   more waves to a row: their barriers cost what the loads gain unless the units
+//     fill the lanes (Q6_K 16000 x 2304, 72 units on 128 lanes: 13.3 / 15.7 / 16.3;
+//     Q8_0 60000 x 2304 28.6 / - / 38.5; Q8_0 4000 x 4096 7.7 / 7.9 / 7.2) or the rows are
+//     long (Q8_0 2000 x 8192 8.9 / 6.9 / 5.4)
+template <int QT>
+int unit_rows(int N, int K) {
+  const int U = K / unit_elems(QT), P = unit_parts(U);
+  const double fill = unit_fill(U);
+  if ((QT == kQ6_K && K < 1280) || (QT == kQ8_0 && K < 512)) return 0;
+  if (P == 1) {
+    if (N <= (K >= 1024 ? 6000 : 4000)) return 1;
+    if (QT == kQ6_K) return N >= 12000 ? 1 : 0;
+    if (QT == kF16) return 4;
+    if (QT == kQ8_0) return N >= 8000 && fill >= 0.7 ? 4 : 0;
+    return N >= (K < 512 ? 32000 : QT == kQ5_K ? 12000 : 8000) ? 4 : 0;
+  }
+  if (P == 2) {
+    if (N <= (QT == kF16 ? 2000 : 3000)) return 1;
+    if (QT == kQ6_K) return N >= 12000 && fill > 0.99 ? 1 : 0;
+    return QT == kQ4_K || (QT == kQ5_K && (N <= 6000 || N >= 12000)) || (QT == kQ8_0 && fill >= 0.8) ? 4 : 0;
+  }
+  if (N <= 1000) return 1;
+  if (QT == kF16) return K >= 3072 || (K >= 1792 && (N <= 3000 || (N >= 12000 && fill >= 0.7))) ? 4 : 0;
+  return N <= 3000 || fill >= 0.7 || (QT == kQ8_0 && K >= 4096) ? 4 : 0;
+}
+
 template <int QT, typename OutT>
 int launch_qmatvec(OutT* y, const uint8_t* W, const float* x, int N, int K) {
   const int64_t rb = row_bytes(QT, K);
   fg::KProfScope prof("qmatvec", 2.0 * N * K, (double)rb * N + 4.0 * K + 4.0 * N);
   const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
   if constexpr (has_units(QT)) {
-    // x in LDS beside the kernel's own arrays (64 KB), whole units, aligned
-    // blocks; Q8_0 rows of fewer units than lanes stay with the eight lanes per
-    // block below (31586 x 256: 6.7 against 7.0 us)
-    if (K <= 16000 && K % unit_elems(QT) == 0 && (uintptr_t)W % 16 == 0 && (QT != kQ8_0 || K >= 1024) &&
-        units_pay(QT, K)) {
+    // x in LDS beside the kernel's own arrays (64 KB), whole units, aligned blocks
+    const int R = K <= 16000 && K % unit_elems(QT) == 0 && (uintptr_t)W % 16 == 0 ? unit_rows<QT>(N, K) : 0;
+    if (R) {
       const int P = unit_parts(K / unit_elems(QT)), slots = kUnitWaves / P;
-      // four rows per wave group, or one where that would leave CUs idle
-      const bool wide = (int64_t)((N + 3) / 4) * P >= 8LL * cus;
-      const int groups = wide ? (N + 3) / 4 : N;
+      const int groups = (N + R - 1) / R;
       const dim3 grid((unsigned)min((groups + slots - 1) / slots, 8 * cus)), block(kUnitThreads);
-      if (wide)
+      if (R == 4)
         FG_LAUNCH((qmatvec_unit_kernel<QT, 4, OutT>), grid, block, (size_t)K * sizeof(float), y, W, x, N, K, rb, P);
       else
         FG_LAUNCH((qmatvec_unit_kernel<QT, 1, OutT>), grid, block, (size_t)K * sizeof(float), y, W, x, N, K, rb, P);

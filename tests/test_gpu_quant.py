@@ -154,6 +154,30 @@ def test_qmatvec_vs_oracle(fh, name):
         assert ident >= 0.98 * total
 
 
+# Many rows of the types with a unit form: one row or four per wave (unit_rows in
+# csrc/quant.hip), one, two or four waves to a row's units, more groups than the
+# launch has room for, one to three rows in the last group.
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["F16", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
+@pytest.mark.parametrize("N,K", [(4099, 4096), (2051, 8192), (8195, 1024), (16390, 512), (33001, 2048), (16385, 1792)])
+def test_qmatvec_of_many_rows(fh, name, N, K):
+    t = TYPES[name]
+    W = _random_bytes(t, N * K // oracle.BLOCK[t][0], N + K)
+    x = np.random.default_rng(K).standard_normal(K).astype(np.float32)
+    ref = oracle.qmatvec(t, W, x, N, K)
+    y = fh.DeviceArray.from_numpy(np.full(N + 4, -7.0, np.float32))
+    Wd, xd = fh.DeviceArray.from_numpy(W), fh.DeviceArray.from_numpy(x)
+    fh.check(fh.lib.fg_qmatvec(t, ctypes.c_void_p(y.ptr), ctypes.c_void_p(Wd.ptr), ctypes.c_void_p(xd.ptr), N, K),
+             "fg_qmatvec")
+    got = y.numpy()
+    assert rel_l2(got[:N], ref) <= TOL_FWD
+    # row by row: fp32 runs of at most 16 products, whose integers (q + 128 for a Q8_0 q) are on
+    # average at most four times the weights'
+    mag = np.abs(oracle.dequantize(t, W, N * K).reshape(N, K)) @ np.abs(x)
+    assert np.max(np.abs(got[:N] - ref) / mag) <= 64 * 2.0 ** -24
+    assert np.all(got[N:] == -7.0)
+
+
 DECODE_TYPES = {
     "k_quants": {"wqkv": 12, "wo": 14, "gate": 13, "down": 12, "cls": 14},
     "q8_f16_emb": {"emb": 8, "cls": 8, "wqkv": 8, "wo": 1, "gate": 8, "down": 1},
