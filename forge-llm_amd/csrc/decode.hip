@@ -919,26 +919,40 @@ __global__ void __launch_bounds__(fgq::kUnitThreads, 3) dec_unit_kernel(Op op, i
 
 inline bool aligned16(const void* p) { return (uintptr_t)p % 16 == 0; }
 // Whether matrix rows of K run in the unit form: a type that has it, whole
-// units, aligned blocks, and x with the kernel's own arrays in 64 KB of LDS.
-// Few or short rows stay with the element-order kernels: a wave takes four rows
-// and a workgroup 16, so that a small matrix's launch is a few workgroups' chain
-// with most lanes idle.  A token of a two-layer model (hidden 2 dim, 3000 ids),
-// element order against units everywhere, us:
-//            dim 256       768         1024        1536         2048
-//   Q4_K   70.4 / 91.4  75.3 / 79.6  80.2 / 83.1  103.5 / 97.3  118.5 / 109.6
-//   Q5_K   70.9 / 99.8  75.7 / 83.9  82.5 / 87.5  105.1 / 104.1 124.2 / 114.4
-//   Q8_0   59.5 / 67.6  79.1 / 76.1  95.9 / 82.4  124.4 / 100.2 146.1 / 112.4
-//   F16    59.2 / 62.6  81.5 / 81.0  90.5 / 90.1  107.8 / 109.6 126.8 / 118.9
-inline bool units_pay_here(int type, int K, int rows) {
-  if (rows >= 16384) return fgq::units_pay(type, K);  // a head fills the chip at any K
-  if (type == fgq::kQ8_0) return K >= 768;
-  return rows >= 1536 && K >= (type == fgq::kF16 ? 2048 : 1536);
-}
-inline bool use_units(int type, const void* W, int K, int rows) {
-  const int e = type == fgq::kF16    ? fgq::unit_elems(fgq::kF16)
-                : type == fgq::kQ8_0 ? fgq::unit_elems(fgq::kQ8_0)
-                : type == fgq::kQ4_K || type == fgq::kQ5_K || type == fgq::kQ6_K ? fgq::unit_elems(fgq::kQ4_K) : 0;
-  return e > 0 && K % e == 0 && K <= 16000 && aligned16(W) && units_pay_here(type, K, rows);
+// units, aligned blocks, x with the kernel's own arrays in 64 KB of LDS, and rows
+// long enough for what precedes the product: the number of rows hardly matters,
+// as a launch of few rows is a chain over one group's K either way.  us a layer
+// saved by units (negative: lost), one matrix of K x rows at a time:
+//                        F16     Q8_0    Q4_K    Q5_K    Q6_K
+//   gate and up  768x512   +1.3    +2.0    +0.4    -0.3    -1.2
+//               1536x512   +3.1    +5.6    +1.5    +0.7    +0.3
+//              4096x8192   +8.1   +26.6    +8.2   +11.3    +9.6
+//   down        1024x768   +0.4    +0.5    -0.3    -0.6    -1.1
+//              2304x1024   +2.0    +2.9    +0.9    +0.7    +0.9
+//   wo         1536x1536   -0.4    +0.5    -1.0    -1.2    -1.4   (own combine)
+//              4096x4096   +0.2    +3.7    +1.0    +0.8    -0.3
+//              1024x1024   +3.8    +3.7    +3.2    +2.8    +2.2   (combined by a launch, 2000 positions)
+// A head of 16384 rows fills the chip at any K (256 x 32000 +4.0, +2.0, +4.3, +3.2,
+// +0.1; Q6_K below 1280 -0.1 at 16384 and -10 at 128000); from 65536 rows on, rows
+// that leave a fifth of the lanes idle lose where two or four waves share them
+// (Q8_0 1280 x 128000 -10).
+enum UnitAt { kAfterNorm, kWoCombines, kWoCombined, kDown };
+inline bool use_units(UnitAt at, int type, const void* W, int K, int rows) {
+  static constexpr int least[4][5] = {{768, 768, 1024, 1280, 1536},
+                                      {4096, 1280, 4096, 4096, 5120},
+                                      {768, 768, 768, 1024, 1024},
+                                      {1024, 768, 2048, 2304, 2304}};
+  const int i = type == fgq::kF16    ? 0
+                : type == fgq::kQ8_0 ? 1
+                : type == fgq::kQ4_K ? 2
+                : type == fgq::kQ5_K ? 3
+                : type == fgq::kQ6_K ? 4
+                                     : -1;
+  if (i < 0) return false;
+  const int e = i == 0 ? fgq::unit_elems(fgq::kF16) : fgq::unit_elems(i == 1 ? fgq::kQ8_0 : fgq::kQ4_K);
+  if (K % e != 0 || K > 16000 || !aligned16(W)) return false;
+  if (rows >= 65536 && (i < 2 || i == 4) && fgq::unit_parts(K / e) > 1 && fgq::unit_fill(K / e) < 0.8) return false;
+  return K >= least[at][i] || (rows >= 16384 && (i != 4 || K >= 1280));
 }
 template <int QT, typename Op>
 int launch_unit(const Op& op, int rows, int K, size_t more_lds = 0) {
@@ -1075,7 +1089,7 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
     {
       const uint8_t* W = static_cast<const uint8_t*>(ly.wqkv);
       const int64_t rb = fgq::row_bytes(ly.wqkv_type, D);
-      if (vec && aligned16(ly.ln1) && use_units(ly.wqkv_type, W, D, qD + 2 * kvD)) {
+      if (vec && aligned16(ly.ln1) && use_units(kAfterNorm, ly.wqkv_type, W, D, qD + 2 * kvD)) {
         const QkvOp op{m->q, kcache, vcache, m->x, emb0, V, ly.ln1, eps, W, rb, m->rope_cos, m->rope_sin, state,
                        D, qD, kvD, dH, m->maxSeq, layer_off};
         FGQ_DISPATCH(ly.wqkv_type, {
@@ -1122,13 +1136,14 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
       // (98 KB at 768 x 16 chunks); beyond that one more launch combines them
       // once, into q's place
       const size_t comb = ((size_t)nH * S + 2 * nH) * sizeof(double);
-      if (vec && use_units(ly.wo_type, W, D, D) && (int64_t)D * S <= 16384 && lds_wo <= 60 * 1024) {
+      const bool own = (int64_t)D * S <= 16384 && lds_wo <= 60 * 1024;
+      if (vec && own && use_units(kWoCombines, ly.wo_type, W, D, D)) {
         const WoOp op{m->x, (const double*)m->attn_part, state, W, rb, D, nH, dH, m->maxSeq, S};
         FGQ_DISPATCH(ly.wo_type, {
           const int rc = launch_unit<QT>(op, D, D, comb);
           if (rc) return rc;
         });
-      } else if (vec && use_units(ly.wo_type, W, D, D)) {
+      } else if (vec && !own && use_units(kWoCombined, ly.wo_type, W, D, D)) {
         FG_LAUNCH(dec_combine_kernel, dim3(nH, (dH + 63) / 64), dim3(kThreads), 0, m->q, (const double*)m->attn_part,
                   state, dH, m->maxSeq, S);
         const ResidOp op{m->x, m->q, W, rb, D, D};
@@ -1145,7 +1160,7 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
       const uint8_t* Wg = static_cast<const uint8_t*>(ly.gate);
       const uint8_t* Wu = static_cast<const uint8_t*>(ly.up);
       const int64_t rb = fgq::row_bytes(ly.gate_type, D);
-      if (vec && aligned16(ly.ln2) && use_units(ly.gate_type, Wg, D, 2 * H) && use_units(ly.gate_type, Wu, D, 2 * H)) {
+      if (vec && aligned16(ly.ln2) && use_units(kAfterNorm, ly.gate_type, Wg, D, 2 * H) && aligned16(Wu)) {
         const GateUpOp op{m->h, m->x, ly.ln2, eps, Wg, Wu, rb, H, D};
         FGQ_DISPATCH(ly.gate_type, {
           const int rc = launch_unit<QT>(op, 2 * H, D);
@@ -1159,7 +1174,7 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
     {
       const uint8_t* W = static_cast<const uint8_t*>(ly.down);
       const int64_t rb = fgq::row_bytes(ly.down_type, H);
-      if (vec && use_units(ly.down_type, W, H, D)) {
+      if (vec && use_units(kDown, ly.down_type, W, H, D)) {
         const ResidOp op{m->x, m->h, W, rb, D, H};
         FGQ_DISPATCH(ly.down_type, {
           const int rc = launch_unit<QT>(op, D, H);
@@ -1174,7 +1189,7 @@ extern "C" int fg_decode_step(const fg_decode_model* m, float* kcache, float* vc
   {
     const uint8_t* W = static_cast<const uint8_t*>(m->wcls);
     const int64_t rb = fgq::row_bytes(m->cls_type, D);
-    if (vec && use_units(m->cls_type, W, D, V)) {
+    if (vec && use_units(kAfterNorm, m->cls_type, W, D, V)) {
       const HeadOp op{logits, m->x, m->ln_f, eps, W, rb, V, D};
       FGQ_DISPATCH(m->cls_type, {
         const int rc = launch_unit<QT>(op, V, D);

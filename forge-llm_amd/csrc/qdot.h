@@ -31,16 +31,6 @@ __host__ __device__ constexpr int unit_elems(int t) {
   return t == kQ4_K || t == kQ5_K || t == kQ6_K ? 32 : t == kQ8_0 ? 16 : t == kF16 ? 8 : 0;
 }
 __host__ __device__ constexpr bool has_units(int t) { return unit_elems(t) > 0; }
-// Rows for which units are the faster form.  Rows of few units leave lanes
-// idle, which Q6_K's longer dot does not make up for (60000 rows, us, element
-// order against units: K 256 16.0 / 19.5, 1024 18.6 / 21.9, 1536 27.4 / 23.4);
-// half rows just past a wave's 64 units pay for two waves' sums (4000 rows:
-// K 512 3.2 / 3.3, 768 3.5 / 4.4, 1536 4.0 / 4.4, 2048 4.4 / 4.5 and at 500 rows
-// 4.2 / 3.3).
-__host__ __device__ constexpr bool units_pay(int t, int K) {
-  return t == kQ6_K ? K >= 1536 : t == kF16 ? K <= 512 || K >= 2048 : true;
-}
-
 // Place of x[i] (i a multiple of 4: a granule) in the LDS copy of x for rows
 // of U units.
 template <int QT>

@@ -206,6 +206,47 @@ def test_decode_step_quantized_vs_oracle(fh, name):
     assert err <= TOL_FWD
 
 
+# Models whose matrices take the unit kernels (use_units in csrc/decode.hip): the
+# five products in the five types; rows that are no whole groups of four; one, two
+# and four waves to a row; more groups than resident workgroups; the attention
+# combined by the output projection (dim x chunks up to 16384) and by a launch of
+# its own; positions over several chunks of 64; f32 and quantized embeddings.
+# dim, heads, kv heads, hidden, vocab, maxSeq, positions, types.
+UNIT_MODELS = {
+    "q8_0": (1280, 20, 4, 1056, 1537, 200, 140, dict(emb=8, cls=8, wqkv=8, wo=8, gate=8, down=8)),
+    "q8_0_long_cache": (1024, 16, 4, 1031, 1539, 1400, 140, dict(cls=8, wqkv=8, wo=8, gate=8)),
+    "q4_K": (1536, 12, 6, 2048, 1601, 800, 70, dict(emb=12, cls=12, wqkv=12, wo=12, gate=12, down=12)),
+    "q5_K": (1536, 24, 24, 2304, 1602, 800, 3, dict(cls=13, wqkv=13, wo=13, gate=13, down=13)),
+    "q6_K": (1536, 24, 8, 2304, 1603, 800, 3, dict(cls=14, wqkv=14, wo=14, gate=14, down=14)),
+    "f16": (2048, 16, 16, 2056, 1603, 800, 3, dict(cls=1, wqkv=1, wo=1, gate=1, down=1)),
+    "head_f16": (256, 4, 4, 512, 16387, 8, 2, dict(emb=1, cls=1)),
+    "head_q8_0": (256, 4, 4, 512, 16386, 8, 2, dict(emb=8, cls=8)),
+    "head_q4_K": (256, 4, 4, 512, 16385, 8, 2, dict(emb=12, cls=12)),
+    "head_q5_K": (256, 4, 4, 512, 16387, 8, 2, dict(emb=13, cls=13)),
+    "wo_f16": (4096, 32, 2, 32, 64, 200, 3, dict(wo=1)),
+    "wo_q4_K": (4096, 32, 2, 32, 64, 200, 3, dict(wo=12)),
+    "wo_q5_K": (4096, 32, 2, 32, 64, 200, 3, dict(wo=13)),
+    "wo_q6_K": (5120, 40, 2, 32, 64, 128, 3, dict(wo=14)),
+}
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(UNIT_MODELS))
+def test_decode_step_in_units_vs_oracle(fh, name):
+    dim, nH, nKV, hidden, vocab, maxSeq, T, types = UNIT_MODELS[name]
+    cfg = oracle.Cfg(dim=dim, hidden=hidden, nLayers=1, nHeads=nH, nKvHeads=nKV, vocab=vocab, tied=0)
+    rs = np.random.default_rng(dim + vocab)
+    params = oracle.init_weights(cfg, 5)
+    P = oracle.split_params(cfg, params)
+    P["wcls"][:] = rs.standard_normal(P["wcls"].size).astype(np.float32) * 0.02
+    ids = rs.integers(0, vocab, T).astype(np.int32)
+    dec = Decoder(fh, cfg, params, maxSeq=maxSeq, types=types)
+    ref = dec.oracle_logits(ids)
+    got = np.stack([dec.step(int(ids[t]), t) for t in range(T)])
+    errs = [rel_l2(got[t], ref[t]) for t in range(T)]
+    print("%s: rel-L2 %.2e at worst over %d positions" % (name, max(errs), T))
+    assert max(errs) <= TOL_FWD
+
+
 @pytest.mark.gpu
 def test_decode_rejects_mismatched_gate_up_and_ragged_blocks(fh):
     cfg = oracle.Cfg(dim=64, hidden=128, nLayers=1, nHeads=4, nKvHeads=2, vocab=40, tied=1)
