@@ -55,7 +55,11 @@ constexpr float kLn2 = 0.6931471805599453f;
 // MFMA kernels' alignment) keep one wave: their sums would not fit.
 // B8 T32 nH4/nKV2 dH16, forward / dQ / dK and dV, in the step: one wave 17 /
 // 13 / 27 us and D's launch 6, eight 7 / 10 / 10; B4 T1024 nH16 dH16, whole:
-// eight 166 us forward and 333 backward.
+// eight 170 us forward and 340 backward (branches over dH and one wave: 3518 and
+// 8044).  The classes above 32 gain from the branch-free loops alone, though they
+// hold more registers (64: 438 and 493 in dQ and dK/dV, one wave a SIMD; 128: 1.1 KB
+// of scratch): forward / backward, unaligned B4 T1024 nH16 dH64 6.6 / 16.3 -> 1.7 /
+// 3.1 ms, nH8 dH128 13.8 / 37.6 -> 3.4 / 19.4, backward with nH2 nKV4 dH80 7.1 -> 4.4.
 constexpr int kSRows = 64;
 template <int kSMax>
 constexpr int kSWaves = kSMax <= 32 ? 8 : 1;
@@ -1585,7 +1589,7 @@ int attn_maxima(fg::Workspace& ws, x3::AttnXp& X, const float* Q, const float* K
 struct CutCost {
   int64_t slots;
   double us, start, bytes;
-  double lone, busy, extra, join, gbs;
+  double lone, busy, extra, join, gbs, margin;
   bool joined;
 };
 template <class F>
@@ -1623,7 +1627,7 @@ x3::Cut plan_cut(int nr, int64_t heads, int cus, const CutCost& cost, F chain) {
     return sqrt(sqrt(item * item * item * item + load * load * load * load)) +
            (joined ? cost.join + (double)items * 2.0 * cost.bytes / (cost.gbs * 1e3) : 0.0);
   };
-  if (lasts(items_of(len), len, true) < 0.98 * lasts(heads * nr, longest, cost.joined)) c.len = len;
+  if (lasts(items_of(len), len, true) < cost.margin * lasts(heads * nr, longest, cost.joined)) c.len = len;
   if (!c.len) return c;
   c.first[0] = 0;
   for (int r = 0; r < nr; ++r) c.first[r + 1] = c.first[r] + (int)heads * ((chain(r) + c.len - 1) / c.len);
@@ -1640,10 +1644,10 @@ int launch_fwd_mfma(float* O, float* lse, const float* Q, const float* K, const 
   const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
   const int nqb = (T + 127) / 128, nk32 = (T + kBlk - 1) / kBlk;
   const double pb = 512.0 * (DH + 2);
-  const CutCost cost = DH <= 32   ? CutCost{4 * cus, 0.9, 1.0, pb, 0.87, 0.45, 0.4, 3.2, 3900.0, false}
-                       : DH <= 64 ? CutCost{3 * cus, 2.1, 1.0, pb, 1.14, 0.67, 0.0, 3.3, 4200.0, false}
-                       : DH <= 96 ? CutCost{2 * cus, 2.1, 1.0, pb, 1.55, 0.87, 8.0, 3.3, 5500.0, false}
-                                  : CutCost{cus, 2.1, 1.0, pb, 2.22, 2.11, 8.0, 5.0, 5300.0, false};
+  const CutCost cost = DH <= 32   ? CutCost{4 * cus, 0.9, 1.0, pb, 0.87, 0.45, 0.4, 3.2, 3900.0, 0.98, false}
+                       : DH <= 64 ? CutCost{3 * cus, 2.1, 1.0, pb, 1.14, 0.67, 0.0, 3.3, 4200.0, 0.98, false}
+                       : DH <= 96 ? CutCost{2 * cus, 2.1, 1.0, pb, 1.55, 0.87, 8.0, 3.3, 5500.0, 0.98, false}
+                                  : CutCost{cus, 2.1, 1.0, pb, 2.22, 2.11, 8.0, 5.0, 5300.0, 0.98, false};
   const x3::Cut cut = plan_cut(nqb, (int64_t)B * nH, cus, cost,
                                [&](int r) { return nk32 < (nqb - r) * 4 ? nk32 : (nqb - r) * 4; });
   fg::Workspace wp;  // whole chains where it cannot be had
@@ -1710,10 +1714,10 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
   if (dS) {
     const double pb = 1024.0 * DH;
     const bool gqa = group > 1;
-    const CutCost cost = DH <= 32   ? CutCost{3 * cus, 3.5, 1.5, pb, 2.01, 0.81, 7.3, 1.1, 4400.0, gqa}
-                         : DH <= 64 ? CutCost{2 * cus, 5.2, 1.5, pb, 2.60, 1.71, 4.4, 1.8, 5100.0, gqa}
-                         : DH <= 96 ? CutCost{cus, 5.2, 1.5, pb, 4.52, 4.45, 8.0, 2.8, 5800.0, gqa}
-                                    : CutCost{cus, 5.2, 1.5, pb, 5.37, 5.51, 8.0, 2.5, 6300.0, gqa};
+    const CutCost cost = DH <= 32   ? CutCost{3 * cus, 3.5, 1.5, pb, 2.01, 0.81, 7.3, 1.1, 4400.0, 0.98, gqa}
+                         : DH <= 64 ? CutCost{2 * cus, 5.2, 1.5, pb, 2.60, 1.71, 4.4, 1.8, 5100.0, 0.98, gqa}
+                         : DH <= 96 ? CutCost{cus, 5.2, 1.5, pb, 4.52, 4.45, 8.0, 2.8, 5800.0, 0.98, gqa}
+                                    : CutCost{cus, 5.2, 1.5, pb, 5.37, 5.51, 8.0, 2.5, 6300.0, 0.98, gqa};
     cut = plan_cut(nkb, (int64_t)nbk * group, cus, cost, [&](int r) { return (int)nq32 - 4 * r; });
   }
   fg::Workspace wp, wc;
@@ -1734,10 +1738,10 @@ int launch_bwd_mfma(float* dQ, int bq, float* dK, int bk, float* dV, int bv, con
             bv, Dq, dO, O, Q, K, V, lse, T, nH, nKV, scale, L, part, nbk, nkv_items, nq_items, dS, npairs, X, cut);
   if (dS) {
     const double pb = 512.0 * DH;
-    const CutCost cost = DH <= 32   ? CutCost{2 * cus, 0.95, 1.0, pb, 0.79, 0.26, 4.0, 3.4, 3500.0, false}
-                         : DH <= 64 ? CutCost{2 * cus, 0.95, 1.0, pb, 0.94, 0.37, 4.0, 3.9, 4500.0, false}
-                         : DH <= 96 ? CutCost{2 * cus, 0.95, 1.0, pb, 1.07, 0.44, 4.0, 3.0, 4200.0, false}
-                                    : CutCost{2 * cus, 0.95, 1.0, pb, 1.27, 0.70, 4.0, 2.1, 3800.0, false};
+    const CutCost cost = DH <= 32   ? CutCost{2 * cus, 0.95, 1.0, pb, 0.79, 0.26, 4.0, 3.4, 3500.0, 1.0, false}
+                         : DH <= 64 ? CutCost{2 * cus, 0.95, 1.0, pb, 0.94, 0.37, 4.0, 3.9, 4500.0, 1.0, false}
+                         : DH <= 96 ? CutCost{2 * cus, 0.95, 1.0, pb, 1.07, 0.44, 4.0, 3.0, 4200.0, 1.0, false}
+                                    : CutCost{2 * cus, 0.95, 1.0, pb, 1.27, 0.70, 4.0, 2.1, 3800.0, 1.0, false};
     const x3::Cut qcut = plan_cut(nkb, (int64_t)B * nH, cus, cost,
                                   [&](int r) { return nq32 < (nkb - r) * 4 ? (int)nq32 : (nkb - r) * 4; });
     fg::Workspace wdq;
