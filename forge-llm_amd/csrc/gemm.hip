@@ -2414,8 +2414,11 @@ int launch_grouped_staged(const fg_wgrad_job* const* jb, int count, int cus) {
   return FG_OK;
 }
 
-// A window: at most kMaxJobs jobs on distinct outputs.  Pieces have to be
-// faster by a margin of 8%, what the fitted times are good for.
+// What `us` on the staging kernels has to be beaten by: the fitted times are good
+// for 8% of a short launch and 3% of a long one.
+inline double beaten(double us) { return 0.97 * us - (0.05 * us < 20.0 ? 0.05 * us : 20.0); }
+
+// A window: at most kMaxJobs jobs on distinct outputs.
 int grouped_window(const fg_wgrad_job* jobs, int count, int cus) {
   const fg_wgrad_job *all[kMaxJobs], *pc[kMaxJobs], *st[kMaxJobs];
   int np = 0, ns = 0;
@@ -2436,14 +2439,14 @@ int grouped_window(const fg_wgrad_job* jobs, int count, int cus) {
     const bool fit = wgrad_piece_bytes(jb) <= kGroupedBytes;
     fits = fits && fit;
     flop += f;
-    if (fit && piece < 0.92 * staged) {
+    if (fit && piece < beaten(staged)) {
       pc[np++] = &jb;
       pflop += f;
     } else {
       st[ns++] = &jb;
     }
   }
-  double best = 0.92 * staged_list_us(all, count, cus);
+  double best = beaten(staged_list_us(all, count, cus));
   int form = 0;  // all staging
   if (fits && flop >= 8e9) {
     const double us = pieces_list_us(all, count, cus);
@@ -2453,7 +2456,7 @@ int grouped_window(const fg_wgrad_job* jobs, int count, int cus) {
     }
   }
   if (np && ns && pflop >= 8e9) {
-    const double us = pieces_list_us(pc, np, cus) + 0.92 * staged_list_us(st, ns, cus);
+    const double us = pieces_list_us(pc, np, cus) + staged_list_us(st, ns, cus);
     if (us < best) form = 2;
   }
   if (form < 2) {
