@@ -2029,10 +2029,15 @@ extern "C" int fg_matmulT_fwd_swiglu_p(float* O, float* GU, const float* X, cons
   FG_ARG_CHECK(M > 0 && K > 0 && H > 0, "fg_matmulT_fwd_swiglu: bad shape M=%d K=%d H=%d", M, K, H);
   FG_ARG_CHECK(O && GU && X && Wgu, "fg_matmulT_fwd_swiglu: null pointer");
   const int cus = fg::device_cu_count() > 0 ? fg::device_cu_count() : 256;
-  // small: a workgroup takes a gate tile and its up tile (the plain
-  // forward's sums: the same plan)
+  // small: a workgroup takes a gate tile and its up tile (the plain forward's
+  // sums: the same plan).  That saves a launch and a pass, and halves the tiles to
+  // spread: worth it for a short K, or where the pairs fit one round of CUs and
+  // their tiles do not.  Of 258 small shapes, fused against the GEMM and the SwiGLU
+  // pass: 0.93 - 0.97 up to K = 128 (one round of pairs 0.79), 0.75 - 1.0 for one
+  // round of pairs at a longer K, elsewhere 1.0 - 1.4 (416 x 1440 over H = 32
+  // 22.3 -> 29.9 us); this line is within 5% of the better form at all of them.
   const SmallPlan sp = plan_small(M, 2 * H, K, 0);
-  if (sp.waves && sp.splits == 1) {
+  if (sp.waves && sp.splits == 1 && (K <= 128 || (small_tiles(M, H) <= cus && small_tiles(M, 2 * H) > cus))) {
     STable t = small_table(GU, X, Wgu, M, H, K, K, K, 0, nullptr, XpArgs{xp_x, xp_w, have});
     t.job[0].O = O;
     fg::KProfScope prof("gemm_nt", 2.0 * M * 2.0 * H * K, 4.0 * ((double)M * K + 2.0 * H * K + 3.0 * (double)M * H));
