@@ -118,3 +118,11 @@ def test_small_fused_epilogues_are_the_separate_passes(fh, M, K, H):
     want = y.copy()
     want[:, 0:(nH + nKV) * dH:2], want[:, 1:(nH + nKV) * dH:2] = a * c - b * s, a * s + b * c
     np.testing.assert_array_equal(Y.numpy(), want)
+
+
+# the fused SwiGLU form at a longer K (pairs of tiles that fit a round of CUs), and
+# few tiles over a long K, which run as the GEMM and the pass
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,H", [(512, 200, 400), (1030, 477, 60), (416, 1440, 32), (17, 1396, 887)])
+def test_small_swiglu_projection_at_longer_k(fh, M, K, H):
+    test_small_fused_epilogues_are_the_separate_passes(fh, M, K, H)
