@@ -1571,7 +1571,8 @@ int attn_maxima(fg::Workspace& ws, x3::AttnXp& X, const float* Q, const float* K
 // busy get through one block every `busy` us whatever the number of resident
 // items, an item costs `extra` blocks more.  A launch takes the longer of the longest item and the load (their
 // 4-norm: a smooth maximum); a cut (or what is joined anyway: GQA's group
-// members) adds `join` us for its launch and the partial results at `gbs`.  The
+// members) adds `join` us for its launch and the partial results at `gbs`, and has
+// to take less than `margin` of the whole.  The
 // constants are least-squares fits per head size to the differences of whole and
 // cut calls over T = 200 .. 8192 and 1 .. 128 heads; of 2452 calls three take
 // longer than whole chains would, 6 - 7% (T512 nH64/nKV16 dH96 and 128, T200 nH64

@@ -1,5 +1,6 @@
 // Single-token inference forward (Transformer.forward, transformer.js:134-184)
-// for gfx950.  One decode step is four launches per layer plus one:
+// for gfx950.  One decode step is five launches per layer plus one (six where a
+// long cache's partials are combined by a launch of their own):
 //
 //   per layer:
 //     qkv        xn = rmsnorm(x, ln1); [q|k|v] = Wqkv·xn; RoPE on q, k with the
@@ -8,8 +9,8 @@
 //                120-129) and also stores it.
 //     attn       per (q head, 64-position chunk): scores q·K/√dH, the chunk's
 //                softmax partials and p·V (attentionDecode, attention.js:31-61)
-//     wo         the per-head combine of the partials, then x += Wo·att
-//                (transformer.js:176-177)
+//     wo         the per-head combine of the partials (dec_combine_kernel before
+//                it for long caches), then x += Wo·att (transformer.js:176-177)
 //     gateup     xn = rmsnorm(x, ln2); h = silu(Wg·xn) * (Wu·xn)     (nn.js:56-66)
 //     down       x += Wd·h                                           (:179-180)
 //   head         logits = Wcls·rmsnorm(x, ln_f)                      (:182-183)
@@ -419,8 +420,8 @@ __global__ void __launch_bounds__(kThreads) dec_attn_part_kernel(double* __restr
 // those of q and V at the start), so a score takes two shuffles instead of
 // log2(LP) per pass; every wave then takes the maximum and the exponentials of
 // all 64 scores itself (lane = position), which saves a barrier and leaves p
-// where its V rows need it.  32 heads of 128 over 2048 positions 28.8 -> 11 us,
-// 12 heads of 64 over 500 9.0 -> 6.5 us.
+// where its V rows need it.  32 heads of 128 over 2048 positions 27.5 -> 17.0 us,
+// 12 heads of 64 over 500 8.8 -> 6.8 us.
 template <int LP>
 __global__ void __launch_bounds__(kThreads) dec_attn_chunk_kernel(double* __restrict__ part,
                                                                   const float* __restrict__ q,

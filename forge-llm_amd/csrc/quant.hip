@@ -5,8 +5,10 @@
 //   fg_quantize    q = quantizeRow(x)              quant.js:322-590, bit-exact
 //
 // The matvec is HBM-bound (a weight is read once per call): units of qdot.h
-// for F16, Q8_0 and the K-quants; otherwise one wave per two rows, x staged
-// once per workgroup in LDS, per-format lane mappings from qformat.h.  Decoding is exact integer/fp16 work; sums are fp64.
+// for F16, Q8_0 and the K-quants where they are the faster form (unit_rows);
+// otherwise one wave per two rows, x staged once per workgroup in LDS, per-format
+// lane mappings from qformat.h.  Decoding is exact integer/fp16 work; sums are
+// fp64.
 //
 // The quantizers restate the reference's scalar algorithms (closed-form
 // Q8_0 and Q4_K, the make_qx_quants / make_qkx2_quants searches of Q6_K and
@@ -498,8 +500,8 @@ unsigned grid_for(int64_t items, int per_block) {
 // 35%).  us from the caches, element order / one row / four rows a wave:
 //   few rows: one each, their loads all in flight (Q4_K 1000 x 4096 6.4 / 4.1 / 4.9)
 //   many rows, one wave to a row's units: four share x and its sums, except Q6_K,
-//     whose longer dot has no registers for four (12000 x 2048 10.9 / 10.0 / 9.6 from
-//     the caches, 16000: 13.6 / 12.5 / 13.1)
+//     whose longer dot leaves three waves a SIMD with four rows, six with
+//     one (12000 x 2048 10.9 / 10.0 / 9.6, 16000: 13.6 / 12.5 / 13.1)
 //   more waves to a row: their barriers cost what the loads gain unless the units
 //     fill the lanes (Q6_K 16000 x 2304, 72 units on 128 lanes: 13.3 / 15.7 / 16.3;
 //     Q8_0 60000 x 2304 28.6 / - / 38.5; Q8_0 4000 x 4096 7.7 / 7.9 / 7.2) or the rows are

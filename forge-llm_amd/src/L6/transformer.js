@@ -92,7 +92,7 @@ const GRAPHS_KEPT = 4;
  * uploads the weights once; `forward(token, pos, cache)` runs one decode step
  * (fg_decode_step: embed, per layer RMSNorm → QKV → RoPE → KV write →
  * attention → Wo + residual → RMSNorm → SwiGLU FFN + residual, final norm,
- * LM head: 4 launches per layer + 1) and returns the logits as a host Float32Array (the same array
+ * LM head: 5 launches per layer + 1) and returns the logits as a host Float32Array (the same array
  * every call, like the reference's `this.logits`).  The first step with a
  * cache runs op by op; the second is recorded as a HIP graph that later
  * steps with that cache replay (token and position are read from device

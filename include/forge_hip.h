@@ -131,14 +131,17 @@ int fg_matmulT_bwd_w(float* gW, const float* gY, const float* X, int M, int K, i
 /* fg_matmulT_bwd_w; have bit 0: xp_gy, bit 1: xp_x. */
 int fg_matmulT_bwd_w_p(float* gW, const float* gY, const float* X, int M, int K, int N, int beta, float* xp_gy,
                        float* xp_x, int have);
-/* Several matmulT weight gradients in one launch — tensor.js:49-51 per job:
- * gW[N,K] (+)= gY[M,N]^T · X[M,K] (beta per job), each over its full M (no
- * K split).  The training step defers the weight gradients of its layer
- * matmuls to the end of backward() and issues them here: thousands of output
- * tiles in one grid fill the GPU without the split-K partial slabs that a
- * single small-output gradient needs.  Jobs on one gW (a weight used twice
- * in one pass) apply in list order, a later job's beta accumulating onto the
- * earlier result; gW must not partially overlap another job's gW.  xp_gy /
+/* Several matmulT weight gradients in few launches — tensor.js:49-51 per job:
+ * gW[N,K] (+)= gY[M,N]^T · X[M,K] (beta per job).  The training step defers the
+ * weight gradients of its layer matmuls to the end of backward() and issues
+ * them here: thousands of output tiles in one grid fill the GPU.  Jobs are
+ * planned together (small lists, operands split while staging or ahead of time,
+ * whichever is faster for a job); where the outputs leave the chip idle a
+ * launch is cut along M, and the pieces are summed in a fixed order from a
+ * workspace.  Jobs on one gW (a weight used twice in one pass) apply in list
+ * order, a later job's beta accumulating onto the earlier result; gW must not
+ * partially overlap another job's gW.  A bad job is reported before anything
+ * is queued.  xp_gy /
  * xp_x: the operands' maxima (FG_XP_PARTS floats each, as filled by a *_p
  * entry point over the same data) or NULL (computed here). */
 typedef struct fg_wgrad_job {
@@ -222,7 +225,8 @@ int fg_attn_bwd_qkv_p(float* gqkv, const float* dO, const float* qkv, const floa
 int fg_attn_fwd(float* O, float* lse, const float* Q, const float* K, const float* V,
                 int B, int T, int nH, int nKV, int dH);
 /* causalAttn* backward — tensor.js:231-267, 339-375.  Recomputes P from lse.
- * dQ (+)= ..., dK (+)= ..., dV (+)= ... (per-tensor beta).  dK/dV of a kv head
+ * dQ (+)= ..., dK (+)= ..., dV (+)= ... (per-tensor beta), in this order where
+ * they share memory (a tensor that is query, key and value at once).  dK/dV of a kv head
  * sum over the nH/nKV query heads of its group.  The head sizes with MFMA
  * kernels keep dS = P∘(dP − D) of every causal 32×32 block in a workspace
  * (4 bytes per causal pair and head) and form dQ from it in a second launch;
